@@ -157,6 +157,59 @@ def run(state):
     return [eng.dense_proj(w, t, x) for w, x in state["layers"]]
 
 
+def _decoded(gen, rows: int, cols: int) -> torch.Tensor:
+    """f64 values of the container tensor that ``_tensor`` / ``_slabs`` would draw next: 36-byte blocks of four scale bytes
+    (E4M3, 0x7F read as 448) and 32 bytes of two E2M1 codes each, the even value in the low nibble; times the global scale."""
+    blocks, gs = quantize_nvfp4(_normal(gen, rows, cols, std=WEIGHT_STD))
+    b = blocks.view(-1, BLOCK_BYTES)
+    scales = (b[:, :4] & 0x7F).clamp(max=0x7E).contiguous().view(torch.float8_e4m3fn).to(torch.float64)
+    codes = torch.stack((b[:, 4:] & 15, b[:, 4:] >> 4), dim=-1).view(-1, 4, 16)
+    e2m1 = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, 0, -0.5, -1, -1.5, -2, -3, -4, -6], dtype=torch.float64, device="cuda")
+    return (e2m1[codes.long()] * scales.unsqueeze(-1) * gs.to(torch.float64)).view(rows, cols)
+
+
+def _swiglu(gate_up: torch.Tensor, down: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    gate, up = (x @ gate_up.T).chunk(2, dim=-1)
+    return (gate / (1.0 + torch.exp(-gate)) * up) @ down.T
+
+
+def exact(case, seed):
+    """The same inputs through plain torch in f64, from the container bytes on.  Expert ids, the greedy token and the
+    encoder's bytes are whole numbers, its global scale is exact by definition: they have no such value."""
+    gen = _generator(seed)
+    kind = case["kind"]
+    if kind == "encode":
+        return None, None, _decoded(gen, case["rows"], case["cols"])
+    out = []
+    if kind == "moe":
+        e, k, h, i, t = case["experts"], case["topk"], case["hidden"], case["inter"], case["t"]
+        for _ in range(case["layers"]):
+            gate_up, down = _decoded(gen, e * 2 * i, h).view(e, 2 * i, h), _decoded(gen, e * h, i).view(e, h, i)
+            router = _normal(gen, e, h, std=h ** -0.5).to(torch.float64)
+            x = _normal(gen, t, h).to(torch.float64)
+            top, ids = (x @ router.T).topk(k, dim=-1)
+            weights = torch.softmax(top, dim=-1)
+            y = torch.zeros_like(x)
+            for expert in ids.unique().tolist():
+                rows, picks = (ids == expert).nonzero(as_tuple=True)
+                y[rows] += weights[rows, picks].unsqueeze(-1) * _swiglu(gate_up[expert], down[expert], x[rows])
+            out.append((None, weights, y))
+        return out
+    if kind == "ffn":
+        h, i = case["hidden"], case["inter"]
+        for _ in range(case["layers"]):
+            gate, up, down = _decoded(gen, i, h), _decoded(gen, i, h), _decoded(gen, h, i)
+            out.append(_swiglu(torch.cat((gate, up)), down, _activations(gen, case["t"], h, case["x"]).to(torch.float64)))
+        return out
+    x = {"proj": case.get("x"), "head": "f32", "gemm": "bf16"}[kind]
+    t = case.get("t", case.get("m", 1))
+    for _ in range(case.get("layers", 1)):
+        w = _decoded(gen, case["rows"], case["cols"])
+        y = _activations(gen, t, case["cols"], x).to(torch.float64) @ w.T
+        out.append((y.view(-1), None) if kind == "head" else y)
+    return out
+
+
 def work(case):
     kind = case["kind"]
     layers = case.get("layers", 1)
