@@ -80,6 +80,9 @@ const FnEntry g_table[] = {
     {"gemm_nvfp4_bf16_w64", (const void*)&gemm_nvfp4_bf16_w64, checked_nargs<7, 0>(&gemm_nvfp4_bf16_w64), 2u * 64u * 528u, 0, 8, 0, 1, false},
     {"gemm_nvfp4_bf16_w80", (const void*)&gemm_nvfp4_bf16_w80, checked_nargs<7, 0>(&gemm_nvfp4_bf16_w80), 2u * 80u * 528u, 0, 8, 0, 1, false},
     {"gemm_nvfp4_bf16_w96", (const void*)&gemm_nvfp4_bf16_w96, checked_nargs<7, 0>(&gemm_nvfp4_bf16_w96), 2u * 96u * 528u, 0, 8, 0, 1, false},
+    {"gemm_nvfp4_bf16_t64", (const void*)&gemm_nvfp4_bf16_t64, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t64), 2u * 64u * 528u, 0, 4, 0, 1, false},
+    {"gemm_nvfp4_bf16_t96", (const void*)&gemm_nvfp4_bf16_t96, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t96), 2u * 96u * 528u, 0, 4, 0, 1, false},
+    {"gemm_nvfp4_bf16_t128", (const void*)&gemm_nvfp4_bf16_t128, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t128), 2u * 128u * 528u, 0, 4, 0, 1, false},
     CROW_FN(gemm_nvfp4_bf16_m32, 7), CROW_FN(gemm_nvfp4_bf16_m16, 7), CROW_FN(gemv_bf16_w, 5),
     CROW_FN(gemv_bf16, 5), CROW_FN(gemv_bf16_b, 5), CROW_FN(gemv_b, 5), CROW_FN(gemv_bf16_ws, 5), CROW_FN(gemv_bf16_bs, 6),
     CROW_FN(gemv_nvfp4_w_valu1, 6), CROW_FN(gemv_nvfp4_w_valu2, 6), CROW_FN(gemv_nvfp4_w_valu4, 6),  // measurement only
@@ -368,29 +371,28 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
     return launch_entry(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream, g.ws_static);
 }
 
-// Which GEMM entry point for m token rows on a [rows, *] tensor.  Up to 16 rows: the K-split body over blocks; up to 96:
-// the K-split body with 32-token blocks.  Beyond that the shared-X body, whose blocks are 4 row tiles x MT tokens: the
-// dispatcher deals ceil(rows / 256) * ceil(m / MT) blocks over the CUs, so the launch lasts as long as the fullest CU.
-// Measured per-block times at K = 5120 (us; they scale with K alike, so only their ratios matter): alone on a CU / sharing it.
+// Which GEMM entry point for m token rows on a [rows, *] tensor.  Up to 16 rows: the K-split body over blocks.  Beyond that
+// the launch lasts as long as the fullest compute unit, and the choice is between blocks that deal one 64-row tile's K over
+// four waves (m32: two of them share a compute unit, short, but a decoded weight serves 32 tokens only) and blocks of 320 rows
+// whose waves each walk all of K (t64 / t96 / t128: one per compute unit, long, a decoded weight serves 64 to 128 tokens).
+// Measured on MI355X at K = 5120 over rows 1024..17408 and 17..2048 tokens: n blocks of m32 on one compute unit take
+// 5.8 + 10.7 n microseconds (within 10 %), a round of t64 / t96 / t128 60 / 72 / 86; at K = 1024 and 17408 all scale
+// alike.  So few row tiles stay with m32 far beyond 96 tokens ([1024, 5120] x 512: 19.7 us against 57 for t64 and 52 for the
+// best of the other tilings), and [17408, 5120] leaves it at about 128 ([.., 5120] x 512: t128 86 us, w80 104).  The remaining
+// entry points (m48 .. w96) are not the fastest anywhere in that range by more than 1 us; they stay callable by name.
 const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) {
     if (m <= 16) return "gemm_nvfp4_bf16_m16";
-    if (m <= 96) return "gemm_nvfp4_bf16_m32";
-    // Measured on MI355X at K = 5120 (microseconds): a block of the four-wave kernels alone on a compute unit / each of several
-    // sharing one; a block of the eight-wave kernels (one per compute unit: two waves per SIMD) per round of the launch.  The
-    // launch lasts as long as the fullest compute unit.
-    static const struct { const char* name; uint32_t mt, tiles_per_block; double alone, shared; } cand[] = {
-        {"gemm_nvfp4_bf16_m48", 48, 4, 58.0, 45.0},  {"gemm_nvfp4_bf16_m64", 64, 4, 63.0, 48.5},  {"gemm_nvfp4_bf16_m96", 96, 4, 78.0, 78.0},
-        {"gemm_nvfp4_bf16_w48", 48, 8, 82.0, 82.0},  {"gemm_nvfp4_bf16_w64", 64, 8, 93.0, 93.0},  {"gemm_nvfp4_bf16_w80", 80, 8, 110.0, 110.0},
-        {"gemm_nvfp4_bf16_w96", 96, 8, 118.0, 118.0}};
-    const unsigned long long row_tiles = (rows + CROW_TILE_ROWS - 1) / CROW_TILE_ROWS;
+    static const struct { const char* name; uint32_t mt, strips; double start, each; } cand[] = {
+        {"gemm_nvfp4_bf16_m32", 32, 4, 5.8, 10.7},  {"gemm_nvfp4_bf16_t64", 64, 20, 0.0, 60.0},
+        {"gemm_nvfp4_bf16_t96", 96, 20, 0.0, 72.0}, {"gemm_nvfp4_bf16_t128", 128, 20, 0.0, 86.0}};
+    const unsigned long long strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
     const unsigned long long cus = g.cus > 0 ? (unsigned long long)g.cus : 256ull;
-    const char* best = cand[1].name;
+    const char* best = nullptr;
     double best_t = 0.0;
     for (const auto& c : cand) {
-        const unsigned long long blocks = ((row_tiles + c.tiles_per_block - 1) / c.tiles_per_block) * ((m + c.mt - 1) / c.mt);
-        const unsigned long long per_cu = (blocks + cus - 1) / cus;
-        const double t = per_cu <= 1 ? c.alone : (double)per_cu * c.shared;
-        if (best_t == 0.0 || t < best_t) {
+        const unsigned long long blocks = ((strips + c.strips - 1) / c.strips) * ((m + c.mt - 1) / c.mt);
+        const double t = c.start + c.each * (double)((blocks + cus - 1) / cus);
+        if (best == nullptr || t < best_t) {
             best_t = t;
             best = c.name;
         }
@@ -513,6 +515,13 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         if (name[15] == '_' && name[16] == 'w') {  // gemm_nvfp4_bf16_w<tokens per block>: eight row tiles per block
             const uint32_t mtw = (uint32_t)atoi(name + 17);
             *out = crow_dims{(rt + 7) / 8, (z + mtw - 1) / mtw, 1, 512};
+            return CROW_OK;
+        }
+        if (name[15] == '_' && name[16] == 't') {  // gemm_nvfp4_bf16_t<tokens per block>: four waves of five strips
+            const uint32_t mtt = (uint32_t)atoi(name + 17);
+            const unsigned long long tiles = (unsigned long long)((strips + 19) / 20) * ((z + mtt - 1) / mtt);
+            if (tiles > 0x7FFFFFFFull) return CROW_ERR_SHAPE;
+            *out = crow_dims{(uint32_t)tiles, 1, 1, 256};
             return CROW_OK;
         }
         const uint32_t mt = name[15] == '_' ? (uint32_t)atoi(name + 17) : 128;  // gemm_nvfp4_bf16_m<tokens per block>

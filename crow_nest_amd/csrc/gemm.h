@@ -387,6 +387,205 @@ __device__ __forceinline__ void gemm_wide_body(const unsigned char* __restrict__
     gemm_store<TBK>(acc, gs_ptr[0], y, rt, m0, rows, m_total, lane);
 }
 
+// Tall-tile body: a block is FOUR waves, one per SIMD, wave w owning NJ adjacent strips (16 NJ weight rows) and all of the
+// block's MT = 16 TBK token rows, so that one decoded operand feeds TBK matrix instructions and the decode (17 vector
+// instructions a unit) fits under them.  With one wave per SIMD nothing else hides a latency, so the wave's own stream does.
+// It runs unit by unit - unit u = NJ S + J is segment S of strip J - and is written out in the order in which it is to be
+// issued (sched_barrier keeps it so): a matrix instruction occupies the matrix pipe for as long as two to three vector
+// instructions take to issue, and a wave that issues its matrix instructions back to back waits for each of them in turn.
+//   * behind each matrix instruction of unit u stand two vector instructions of the decode of unit u + 1;
+//   * the activation operands of segment S + 1 are read from LDS during segment S, across panels too;
+//   * the codes of a half panel (segments 0..3 / 4..7) are requested again, for the next panel, as soon as that half has been
+//     decoded: half a panel of matrix work covers the round trip with a single register set;
+//   * the next X tile travels through registers, one 16-byte chunk requested per unit and one written per unit to the other LDS
+//     buffer, and the panel's only barrier stands before segment 7, whose operands are in registers by then.
+// Measured ([17408, 5120] x 512 tokens / [5120, 17408] x 1999, TBK = 8): 82 us / 289 us against 107 / 342 for the eight-wave
+// body at 80 tokens, 1.11 / 1.23 PFLOP/s; a library bf16 product of the first shape takes 100 us, and 8192^3 runs at 1.07 to
+// 1.39.  A panel takes 8250 cycles at 1.9 to 2.0 GHz where its matrix instructions alone take 5280; without the decode 7000, without
+// the matrix instructions 5000, with all activations zero the same cycles at 2.2 GHz: what remains is the two kinds of
+// instruction that only partly overlap, and the power of the matrix cores.
+// blockIdx.x counts tiles in an order that keeps the tiles of one compute die (blockIdx.x % 8) together: four row blocks by
+// as many token blocks as fall to the die, so that its L2 serves both operands.
+__device__ const unsigned gemm_zeros[4] = {0u, 0u, 0u, 0u};
+typedef float f32x4_dword __attribute__((ext_vector_type(4), aligned(4)));  // rows of Y start at any dword
+template <int TBK, int NJ>
+struct TallTile {
+    static constexpr int MT = 16 * TBK;
+    static constexpr int XCH = MT * 32 / 256;  // 16-byte chunks of an X tile per thread
+    static constexpr int XBUF = MT * CROW_GEMM_XS_STRIDE;
+    static constexpr int UNITS = 8 * NJ, STORE0 = 7 * NJ - XCH;  // the first unit that writes a chunk of the next X tile
+    static_assert(MT * 32 % 256 == 0 && STORE0 > XCH / 2, "whole chunks per thread, requested well before they are written");
+    unsigned sc[NJ], even[NJ], odd[NJ];
+    uint4 cd[2][NJ];
+    uint4 xv[XCH];
+    bf16x8 A[2][TBK];
+    u32x4 B[2];
+    f32x4 acc[TBK][NJ];
+    const unsigned char* wp[NJ];
+    unsigned xrow, xlast, kd;  // element offsets of this thread's first row of X and of the last row; the row stride
+    const unsigned short* x;
+    const __bf16 *cur, *nxt;  // this lane's view of the X tile that is being multiplied / of the next one
+    __bf16* put;              // this thread's first chunk of the next X tile
+    f32x2 pair;               // the decode under way: two values, their scale, the first product
+    float scale, low;
+    const unsigned short* from;  // this lane's X, its column in the next panel and a mask for its row offsets
+    unsigned at_k, inside;
+    int lane;
+
+    __device__ __forceinline__ void load_scale(int J, int p) { sc[J] = *((const unsigned*)(wp[J] + (size_t)p * CROW_GROUP_BYTES) + lane); }
+    __device__ __forceinline__ void load_codes(int H, int J, int p) {
+        cd[H][J] = *((const uint4*)(wp[J] + (size_t)p * CROW_GROUP_BYTES + CROW_GROUP_SCALE_BYTES + 1024 * H) + lane);
+    }
+    // both segments' scale words of every pair, as in TileScales
+    __device__ __forceinline__ void set_scales() {
+#pragma unroll
+        for (int J = 0; J < NJ; J++) {
+            const u32x2 sw = __builtin_amdgcn_permlane16_swap(sc[J], sc[J], false, false);
+            even[J] = sw.x;
+            odd[J] = sw.y;
+        }
+    }
+    // columns beyond K (the last, partial panel) meet zero weights, but must not be NaN: their lanes read a word of zeros
+    // (an address, not a branch: the panel stays one block of code, and the accumulators stay where they are)
+    __device__ __forceinline__ void load_x(int i) { 
+        const unsigned row = xrow + (unsigned)(8 * i) * kd;  // rows beyond M read row M - 1 (never stored)
+        const u32x4 v = *(const __attribute__((address_space(1))) u32x4*)(from + (size_t)(((row < xlast ? row : xlast) & inside) + at_k));
+        xv[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    __device__ __forceinline__ void store_x(int i) { *(uint4*)(put + i * 8 * CROW_GEMM_XS_STRIDE) = xv[i]; }
+    // one of the eight steps of unit U's decode: a pair's conversion and first product / its second product and packing
+    template <int U, int STEP>
+    __device__ __forceinline__ void decode() {
+        constexpr int S = U / NJ, J = U % NJ, Q = STEP / 2;
+        const unsigned codes = u4_get(cd[S >> 2][J], S & 3);
+        if constexpr (STEP == 0) scale = e4m3_to_f32<(S >> 1)>((S & 1) ? odd[J] : even[J]);
+        if constexpr (STEP % 2 == 0) {
+            pair = fp4x2_to_f32<Q>(codes);
+            low = pair.x * scale;
+        } else {
+            B[U & 1][Q] = __builtin_amdgcn_perm(__float_as_uint(pair.y * scale), __float_as_uint(low), 0x07060302u);
+        }
+    }
+    template <int U, int T>
+    __device__ __forceinline__ void unit_steps() {
+        if constexpr (T < TBK) {
+            constexpr int J = U % NJ, S = U / NJ;
+            acc[T][J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, B[U & 1]), A[S & 1][T], acc[T][J], 0, 0, 0);
+            constexpr int N = (U + 1) % UNITS;
+            constexpr int D0 = T * 8 / TBK, D1 = (T + 1) * 8 / TBK;  // decode steps behind this matrix instruction
+            if constexpr (D0 < D1) decode<N, D0>();
+            if constexpr (D0 + 1 < D1) decode<N, D0 + 1>();
+            static_assert(D1 - D0 <= 2, "at least four token blocks");
+            __builtin_amdgcn_sched_barrier(0);
+            unit_steps<U, T + 1>();
+        }
+    }
+    template <int U>
+    __device__ __forceinline__ void units(int pn) {
+        if constexpr (U < UNITS) {
+            constexpr int S = U / NJ, J = U % NJ;
+            if constexpr (U == 7 * NJ) __syncthreads();  // the next X tile is written by every wave, this one's last operands are in registers
+            // memory work of this unit: operands of segment S + 1, a chunk of the next X tile, the codes whose registers are free
+#pragma unroll
+            for (int tb = J * TBK / NJ; tb < (J + 1) * TBK / NJ; tb++)
+                A[(S + 1) & 1][tb] = *(const bf16x8*)((S == 7 ? nxt : cur) + tb * 16 * CROW_GEMM_XS_STRIDE + ((S + 1) & 7) * 32);
+            if constexpr (U < XCH) load_x(U);
+            if constexpr (U >= STORE0 && U < 7 * NJ) store_x(U - STORE0);
+            if constexpr (S == 4) load_scale(J, pn);
+            if constexpr (S == 4) load_codes(0, J, pn);
+            if constexpr (U == UNITS - 1) set_scales();
+            __builtin_amdgcn_sched_barrier(0);
+            unit_steps<U, 0>();
+            units<U + 1>(pn);
+        }
+    }
+
+    __device__ __forceinline__ void run(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x_, const float* __restrict__ gs_ptr,
+                                        float* __restrict__ y, int k_dim, int rows, int m_total, __bf16* xs2) {
+        lane = lane_id();
+        x = x_;
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        const int strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
+        const int panels = (k_dim + CROW_PANEL_COLS - 1) / CROW_PANEL_COLS;
+        const int row_blocks = (strips + 4 * NJ - 1) / (4 * NJ), token_blocks = (m_total + MT - 1) / MT;
+        // tile of this block: runs of consecutive tile numbers per compute die, numbers counting four row blocks first
+        const int blocks = (int)gridDim.x, die = (int)blockIdx.x & 7, at = (int)blockIdx.x >> 3;
+        const int t = die * (blocks >> 3) + (die < (blocks & 7) ? die : (blocks & 7)) + at;
+        if (t >= row_blocks * token_blocks) return;  // a grid larger than the problem: the whole block leaves
+        const int band = t / (4 * token_blocks), in_band = t - band * 4 * token_blocks;
+        const int band_rows = row_blocks - 4 * band < 4 ? row_blocks - 4 * band : 4;
+        const int rb = 4 * band + in_band % band_rows, m0 = in_band / band_rows * MT;
+        const int strip0 = (rb * 4 + wave) * NJ;  // strips beyond the tensor re-read the last one (their rows are never stored)
+#pragma unroll
+        for (int J = 0; J < NJ; J++) wp[J] = w + (size_t)(strip0 + J < strips ? strip0 + J : strips - 1) * panels * CROW_GROUP_BYTES;
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // chunk c = i * 256 + thread: token row c / 32, 8 columns from 8 (c % 32)
+        const int xq = ((int)threadIdx.x & 31) * 8;
+        kd = (unsigned)k_dim;
+        xlast = (unsigned)(m_total - 1) * kd;
+        xrow = (unsigned)(m0 + ((int)threadIdx.x >> 5)) * kd;
+        auto next_panel = [&](int p, int buf) {  // the X tile that load_x and store_x move
+            const int k = p * CROW_PANEL_COLS + xq;
+            from = k < k_dim ? x : (const unsigned short*)gemm_zeros;
+            inside = k < k_dim ? ~0u : 0u;
+            at_k = k < k_dim ? (unsigned)k : 0u;
+            put = xs2 + buf * XBUF + ((int)threadIdx.x >> 5) * CROW_GEMM_XS_STRIDE + xq;
+        };
+        const int lane_off = (lane & 15) * CROW_GEMM_XS_STRIDE + (lane >> 4) * 8;
+        next_panel(0, 0);
+#pragma unroll
+        for (int i = 0; i < XCH; i++) load_x(i);
+#pragma unroll
+        for (int J = 0; J < NJ; J++) {
+            load_scale(J, 0);
+            load_codes(0, J, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < XCH; i++) store_x(i);
+        __syncthreads();
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++) A[0][tb] = *(const bf16x8*)(xs2 + lane_off + tb * 16 * CROW_GEMM_XS_STRIDE);
+        set_scales();
+        decode<0, 0>(), decode<0, 1>(), decode<0, 2>(), decode<0, 3>(), decode<0, 4>(), decode<0, 5>(), decode<0, 6>(), decode<0, 7>();
+        int h = 0;
+        for (int p = 0; p < panels; p++) {
+            const int pn = p + 1 < panels ? p + 1 : p;  // behind the last panel: requested once more, never used
+            cur = xs2 + h * XBUF + lane_off;
+            h ^= 1;
+            nxt = xs2 + h * XBUF + lane_off;
+            next_panel(pn, h);
+#pragma unroll
+            for (int J = 0; J < NJ; J++) load_codes(1, J, p);
+            units<0>(pn);
+        }
+        // acc[tb][j][r] of lane (g, n): weight row 16 (strip0 + j) + 4 g + r, token m0 + 16 tb + n (the weights ride on the M side, so
+        // that a lane holds four neighbours of one row of Y: one store instruction instead of four)
+        const float gs = gs_ptr[0];
+        const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int col = (strip0 + j) * CROW_STRIP_ROWS + 4 * g;
+#pragma unroll
+            for (int tb = 0; tb < TBK; tb++) {
+                const int m = m0 + 16 * tb + n;
+                const f32x4 v = acc[tb][j] * gs;
+                if (m >= m_total) continue;
+                float* to = y + (size_t)m * rows + col;
+                if (col + 3 < rows) {
+                    *(f32x4_dword*)to = v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < rows) to[r] = v[r];
+                }
+            }
+        }
+    }
+};
+
 }  // namespace crow
 
 // Y[M][rows] f32 = X[M][k_dim] bf16 times the tiled NVFP4 tensor, times gs.  The argument list is
@@ -454,3 +653,20 @@ CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w48, 3)
 CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w64, 4)
 CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w80, 5)
 CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w96, 6)
+// the tall-tile body: grid (ceil(strips / (4 NJ)) * ceil(M / MT)), block 256, MT = 16 TBK tokens; dynamic LDS = two X tiles
+#define CROW_GEMM_TALL_ENTRY(NAME, TBK, NJ)                                                                                    \
+    extern "C" __global__ void __launch_bounds__(256, 1) NAME(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x, \
+                                                         const float* __restrict__ gs_ptr, float* __restrict__ y,              \
+                                                         const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,      \
+                                                         const int* __restrict__ m_p) {                                        \
+        /* 256 threads; X is addressed with 32-bit element offsets */                                                         \
+        if (block_threads() != 256 || *m_p < 1 || (unsigned long long)*m_p * (unsigned long long)*k_dim_p > 0xffffffffull) {   \
+            if (threadIdx.x == 0) atomicOr(crow::g_ws.status, crow::STATUS_BAD_SHAPE);                                         \
+            return;                                                                                                            \
+        }                                                                                                                      \
+        crow::TallTile<TBK, NJ> t;                                                                                             \
+        t.run(w, x, gs_ptr, y, *k_dim_p, *rows_p, *m_p, (__bf16*)crow_dyn_lds);                                                \
+    }
+CROW_GEMM_TALL_ENTRY(gemm_nvfp4_bf16_t64, 4, 5)
+CROW_GEMM_TALL_ENTRY(gemm_nvfp4_bf16_t96, 6, 5)
+CROW_GEMM_TALL_ENTRY(gemm_nvfp4_bf16_t128, 8, 5)

@@ -77,6 +77,21 @@ def test_gemm_kernel_choice_names_table_entries():
     assert all(v != "gemm_nvfp4_bf16_m16" for m, v in picks.items() if m > 16)  # that entry point refuses m > 16
 
 
+def test_gemm_kernel_choice_by_the_fullest_compute_unit():
+    """Few row tiles stay with the K-split blocks well beyond 96 tokens; large products go to the tall tiles, whose grid is
+    one block per (320 rows, tokens per block) tile."""
+    import ctypes as C
+    lib = L.lib()
+    pick = lambda rows, m: lib.crow_hip_gemm_kernel(rows, m).decode()[len("gemm_nvfp4_bf16_"):]
+    assert [pick(1024, m) for m in (17, 512, 1024)] == ["m32"] * 3
+    assert pick(5120, 1024) == "t64" and pick(2816, 2048) == "t96" and pick(17408, 512) == pick(5120, 1999) == "t128"
+    for name, mt in (("t64", 64), ("t96", 96), ("t128", 128)):
+        for rows, m in ((1, 1), (320, mt), (321, mt + 1), (17408, 2048)):
+            d = L.Dims()
+            assert lib.crow_hip_launch_dims(f"gemm_nvfp4_bf16_{name}".encode(), rows, 5120, m, C.byref(d)) == 0
+            assert (d.gx, d.gy, d.gz, d.bx) == (-(-rows // 320) * -(-m // mt), 1, 1, 256)
+
+
 def test_launch_dims_depend_on_the_matrix_only():
     import ctypes as C
     lib = L.lib()

@@ -877,6 +877,28 @@ def test_gemm_ragged_shapes_drawn_at_random(eng):
             assert gamma_ratio(y[:2], w, rows, cols, gs, xw.reshape(m, cols)[:2]) <= 1.0, (case, kernel)
 
 
+@pytest.mark.parametrize("kernel,m,rows,cols", [
+    ("gemm_nvfp4_bf16_t64", 1, 16, 64),         # one token, one strip, a quarter of one panel
+    ("gemm_nvfp4_bf16_t64", 65, 321, 320),      # one token, one row and 64 columns beyond a block / a panel
+    ("gemm_nvfp4_bf16_t96", 97, 330, 576),      # rows that are no multiple of four: every row of Y starts at another dword
+    ("gemm_nvfp4_bf16_t128", 129, 639, 512),    # a second row block one row short of full
+    ("gemm_nvfp4_bf16_t128", 300, 1601, 832),   # six row blocks (a full band of four and one of two) x three token blocks
+    ("gemm_nvfp4_bf16_t128", 128, 2880, 256),   # nine blocks of one panel: more than one per compute die
+])
+def test_gemm_tall_tiles_at_their_edges(eng, kernel, m, rows, cols):
+    _gemm_case(eng, m, rows, cols, kernel)
+    # ... and a Y whose rows start at odd dwords, with nothing written outside them
+    w = random_nvfp4(3, rows, cols)
+    f = _load(w, rows, cols, 6.0e-4)
+    xb, _ = _bf16_dev(normal_f32(7, m, m * cols))
+    y = torch.full((m * rows + 8,), float("nan"), device="cuda")
+    got = eng.gemm(f, m, xb.reshape(m, cols).contiguous(), y[1:1 + m * rows].view(m, rows), kernel=kernel)
+    ref = eng.gemm(f, m, xb.reshape(m, cols).contiguous(), kernel="gemm_nvfp4_bf16_w48")  # same order of sums: same bits
+    eng.check()
+    assert torch.equal(got, ref)
+    assert torch.isnan(y[0]) and torch.isnan(y[1 + m * rows:]).all()
+
+
 def test_gemm_m16_full_size_cross_block_split(eng):
     """[17408, 5120] at 16 tokens: the K-split kernel's five column slices meet through the workspace."""
     _gemm_case(eng, 16, 17408, 5120, "gemm_nvfp4_bf16_m16")
