@@ -532,7 +532,12 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         }
         return CROW_OK;
     }
-    if (strcmp(name, "repack_nvfp4") == 0 || strcmp(name, "unpack_nvfp4") == 0 || strcmp(name, "dequant_nvfp4_tiled") == 0) {
+    if (strcmp(name, "repack_nvfp4") == 0 || strcmp(name, "dequant_nvfp4_tiled") == 0) {  // adjacent groups, one per wave
+        const uint32_t waves = groups < CROW_LAYOUT_WAVES ? groups : CROW_LAYOUT_WAVES;
+        *out = crow_dims{(groups + waves - 1) / waves, strips, 1, 64 * waves};
+        return CROW_OK;
+    }
+    if (strcmp(name, "unpack_nvfp4") == 0) {
         *out = crow_dims{groups, strips, 1, 64};
         return CROW_OK;
     }

@@ -7,35 +7,47 @@ using namespace crow;
 #define CROW_STATUS_BAD_SCALE_BYTE 8u
 
 // ------------------------------------------------------------------ container <-> tiled
-// One 64-thread block per group (blockIdx.x = group, blockIdx.y = strip); thread l moves the 36-byte container block
-// (strip row l % 16, block l / 16 of the group's four).  Load-time work: neither the strided 36-byte reads nor the
-// scattered 4-byte writes are coalesced, and they need not be.
-extern "C" __global__ void __launch_bounds__(64) repack_nvfp4(const unsigned char* __restrict__ src, unsigned char* __restrict__ dst,
-                                                              const int* __restrict__ rows_p, const int* __restrict__ k_dim_p) {
+// One wave per group, up to four adjacent groups of a strip (blockIdx.y) in a block.  Bound by memory: both sides are read and
+// written in whole dwords, 256 contiguous bytes per instruction on the tiled side and runs of 144 bytes (a row's share of the
+// group) on the container side; the byte shuffle between the two runs through LDS, each wave in its own part.  Adjacent groups
+// share a block because a row's 144-byte runs share cache lines.  [17408, 5120]: 19 us for 100 MB; 25 us when every thread
+// moved one container block with 36-byte strides and scattered stores.
+#define CROW_LAYOUT_WAVES 4
+extern "C" __global__ void __launch_bounds__(64 * CROW_LAYOUT_WAVES) repack_nvfp4(const unsigned char* __restrict__ src, unsigned char* __restrict__ dst,
+                                                                                  const int* __restrict__ rows_p, const int* __restrict__ k_dim_p) {
+    __shared__ unsigned raw_all[CROW_LAYOUT_WAVES][CROW_STRIP_ROWS * 36];
     const int rows = *rows_p, k = *k_dim_p;
     const int groups = (k + CROW_GROUP_COLS - 1) / CROW_GROUP_COLS, bpr = k / CROW_BLOCK_VALUES;
-    const int gi = (int)blockIdx.x, strip = (int)blockIdx.y, lane = lane_id();
-    const int r = lane & 15, b = lane >> 4;
-    const int row = strip * CROW_STRIP_ROWS + r, blk = gi * 4 + b;
-    unsigned char* grp = dst + ((size_t)strip * groups + gi) * CROW_GROUP_BYTES;
-    unsigned q[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (row < rows && blk < bpr) {
-        const unsigned* sq = (const unsigned*)(src + ((size_t)row * bpr + blk) * CROW_BLOCK_BYTES);
+    const int wave = (int)(threadIdx.x >> 6), lane = lane_id();
+    const int gi = (int)blockIdx.x * (block_threads() >> 6) + wave, strip = (int)blockIdx.y;
+    if (gi >= groups) return;  // no block barrier below
+    unsigned* raw = raw_all[wave];
+    const unsigned* s32 = (const unsigned*)src;
+    unsigned q[9];
 #pragma unroll
-        for (int i = 0; i < 9; i++) q[i] = sq[i];
-    }
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        unsigned v = (q[0] >> (8 * i)) & 0xFFu;
-        if (v == 0xFFu) bad = true;
-        v &= 0x7Fu;
-        if (v == 0x7Fu) v = 0x7Eu;
-        grp[crow_group_scale_offset((unsigned)r, (unsigned)(4 * b + i))] = (unsigned char)v;
+    for (int t = 0; t < 9; t++) {  // dword j of the group's container bytes: strip row j / 36
+        const int j = 64 * t + lane, r = j / 36, dw = j - 36 * r, row = strip * CROW_STRIP_ROWS + r;
+        q[t] = 0;
+        if (row < rows && 36 * gi + dw < 9 * bpr) q[t] = s32[(size_t)row * bpr * 9 + (size_t)(36 * gi + dw)];
     }
 #pragma unroll
-    for (int wd = 0; wd < 8; wd++) *(unsigned*)(grp + crow_group_code_offset((unsigned)r, (unsigned)(8 * b + wd))) = q[1 + wd];
-    if (bad) atomicOr(g_ws.status, CROW_STATUS_BAD_SCALE_BYTE);
+    for (int t = 0; t < 9; t++) raw[64 * t + lane] = q[t];
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses execute in order)
+    unsigned* out = (unsigned*)(dst + ((size_t)strip * groups + gi) * CROW_GROUP_BYTES);
+    // dword l = 16 g + n: byte jj = sub-block 2 (g & 1) + (g >> 1) of container block jj, row n (layout.h)
+    const int n = lane & 15, g = lane >> 4, sub = 2 * (g & 1) + (g >> 1);
+    unsigned v = 0;
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) v |= ((raw[36 * n + 9 * jj] >> (8 * sub)) & 0xFFu) << (8 * jj);
+    // four bytes at once: 0xFF is refused, bit 7 is cleared, 0x7F becomes 0x7E
+    const unsigned top = ((v & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;
+    if ((v & top) != 0) atomicOr(g_ws.status, CROW_STATUS_BAD_SCALE_BYTE);
+    out[lane] = (v & 0x7F7F7F7Fu) - (top >> 7);
+#pragma unroll
+    for (int t = 0; t < 8; t++) {  // code dword 256 h + 4 l + d: row l % 16, container block 2 h + d / 2, word 4 (d % 2) + l / 16
+        const int o = 64 * t + lane, h = o >> 8, l = (o >> 2) & 63, d = o & 3;
+        out[64 + o] = raw[36 * (l & 15) + 9 * (2 * h + (d >> 1)) + 1 + 4 * (d & 1) + (l >> 4)];
+    }
 }
 
 // The inverse: tiled -> container bytes (scale bytes come back canonical: 0x7F has become 0x7E and
@@ -60,32 +72,45 @@ extern "C" __global__ void __launch_bounds__(64) unpack_nvfp4(const unsigned cha
 
 // Dequantise a tiled tensor to f32 [rows][k_dim]: w = e2m1(code) * f32(ue4m3(scale) * gs), the two
 // roundings of the reference decode in that order (engine/src/cnq.rs:1298-1308 with the scale rule of
-// cpu_nvfp4.rs:98-105 already applied by the repacker).  Same grid as repack_nvfp4: thread l decodes the 64 values of
-// strip row l % 16, container block l / 16 of the group.
-extern "C" __global__ void __launch_bounds__(64) dequant_nvfp4_tiled(const unsigned char* __restrict__ w, const float* __restrict__ gs_ptr,
-                                                                     float* __restrict__ out, const int* __restrict__ rows_p,
-                                                                     const int* __restrict__ k_dim_p) {
+// cpu_nvfp4.rs:98-105 already applied by the repacker).  Same grid as repack_nvfp4.  Bound by the f32 values it writes: the wave
+// reads its group with 256 contiguous bytes per instruction, keeps it in LDS and writes row by row, 1024 contiguous bytes per
+// instruction, taking four codes and a scale byte per lane and row from there.  The stores are non-temporal: plain ones leave the
+// memory-side cache full of lines that the next kernel's reads must first push out (the encoder's maximum pass behind it 77 to
+// 113 us instead of 60).  [17408, 5120]: 69 to 74 us for 406 MB (66 with plain stores); 139 us when every thread decoded 64 values
+// of one row with scattered stores.
+extern "C" __global__ void __launch_bounds__(64 * CROW_LAYOUT_WAVES) dequant_nvfp4_tiled(const unsigned char* __restrict__ w, const float* __restrict__ gs_ptr,
+                                                                                         float* __restrict__ out, const int* __restrict__ rows_p,
+                                                                                         const int* __restrict__ k_dim_p) {
+    __shared__ unsigned tile_all[CROW_LAYOUT_WAVES][CROW_GROUP_BYTES / 4];
     const int rows = *rows_p, k = *k_dim_p;
     const int groups = (k + CROW_GROUP_COLS - 1) / CROW_GROUP_COLS;
-    const int gi = (int)blockIdx.x, strip = (int)blockIdx.y, lane = lane_id();
-    const int r = lane & 15, b = lane >> 4;
-    const int row = strip * CROW_STRIP_ROWS + r, col_b = gi * CROW_GROUP_COLS + b * CROW_BLOCK_VALUES;
-    if (row >= rows || col_b >= k) return;
+    const int wave = (int)(threadIdx.x >> 6), lane = lane_id();
+    const int gi = (int)blockIdx.x * (block_threads() >> 6) + wave, strip = (int)blockIdx.y;
+    if (gi >= groups) return;  // no block barrier below
+    unsigned* tile = tile_all[wave];
+    const unsigned* grp = (const unsigned*)(w + ((size_t)strip * groups + gi) * CROW_GROUP_BYTES);
+    unsigned q[9];
+#pragma unroll
+    for (int t = 0; t < 9; t++) q[t] = stream_load_u32(grp + 64 * t + lane);
+#pragma unroll
+    for (int t = 0; t < 9; t++) tile[64 * t + lane] = q[t];
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses execute in order)
+    const int col = gi * CROW_GROUP_COLS + 4 * lane;
+    if (col >= k) return;
     const float gs = gs_ptr[0];
-    const unsigned char* grp = w + ((size_t)strip * groups + gi) * CROW_GROUP_BYTES;
-    for (int i = 0; i < 4; i++) {
-        const int sb = 4 * b + i;
-        const unsigned byte = grp[crow_group_scale_offset((unsigned)r, (unsigned)sb)];
-        const float sf = __builtin_amdgcn_cvt_f32_fp8((int)byte, 0) * gs;
-        float* o = out + (size_t)row * k + col_b + 16 * i;
-        for (int d = 0; d < 2; d++) {
-            const unsigned wd = *(const unsigned*)(grp + crow_group_code_offset((unsigned)r, (unsigned)(2 * sb + d)));
-            for (int j = 0; j < 8; j++) {
-                const unsigned nib = (wd >> (4 * j)) & 0xFu;
-                const f32x2 v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(nib, 1.0f, 0);
-                o[d * 8 + j] = v.x * sf;
-            }
-        }
+    // this lane's four codes and scale byte of strip row 0; row r's lie 16 r and 4 r bytes on
+    const unsigned char* codes = (const unsigned char*)tile + crow_group_code_offset(0, (unsigned)(lane >> 1)) + 2 * (lane & 1);
+    const unsigned char* scale = (const unsigned char*)tile + crow_group_scale_offset(0, (unsigned)(lane >> 2));
+    typedef unsigned short __attribute__((may_alias)) u16_of_dword;
+    typedef float f32x4_dword __attribute__((ext_vector_type(4), aligned(4)));  // the caller's buffer may start at any dword
+    float* o = out + (size_t)strip * CROW_STRIP_ROWS * k + col;
+    const int n = rows - strip * CROW_STRIP_ROWS < CROW_STRIP_ROWS ? rows - strip * CROW_STRIP_ROWS : CROW_STRIP_ROWS;
+#pragma unroll 4
+    for (int r = 0; r < n; r++) {
+        const unsigned c = *(const u16_of_dword*)(codes + 16 * r);
+        const float sf = __builtin_amdgcn_cvt_f32_fp8((int)scale[4 * r], 0) * gs;
+        const f32x2 a = fp4x2_to_f32<0>(c), b = fp4x2_to_f32<1>(c);
+        __builtin_nontemporal_store(f32x4_dword{a.x * sf, a.y * sf, b.x * sf, b.y * sf}, (f32x4_dword*)(o + (size_t)r * k));
     }
 }
 
@@ -220,17 +245,26 @@ __device__ __forceinline__ float subblock_amax(const float4 (&q)[4]) {
 __device__ __forceinline__ float subblock_raw(const float4 (&q)[4]) { return __fdiv_rn(subblock_amax(q), 6.0f); }
 // pass 1: the largest |value| of the tensor, as the bit pattern of a non-negative f32 (they order like unsigned integers).
 // The largest raw scale is that maximum over 6: a correctly rounded division is monotonic, so the maximum of the quotients is
-// the quotient of the maximum, bit for bit.  Grid-stride over the n / 16 sub-blocks, one atomic per block; *max_bits starts
+// the quotient of the maximum, bit for bit.  A maximum asks for no order, so the lanes read 16 contiguous bytes each (whole
+// sub-blocks per lane touch every cache line four times, and a block's four requests 8 MB apart fall on few channels: 74 to 113 us
+// for 356 MB against 60); one atomic per block; *max_bits starts
 // as 0 (quantize_nvfp4_clear: a kernel rather than a memset, so that the three launches can be captured into a graph).
 extern "C" __global__ void quantize_nvfp4_clear(unsigned* __restrict__ max_bits) { *max_bits = 0u; }
 extern "C" __global__ void __launch_bounds__(256) quantize_nvfp4_amax(const float* __restrict__ values, unsigned long long n_sub,
                                                                        unsigned* __restrict__ max_bits) {
     __shared__ float per_wave[4];
     float best = 0.0f;
-    for (unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; i < n_sub; i += (unsigned long long)gridDim.x * blockDim.x) {
-        const float4* p = (const float4*)(values + 16 * i);
-        const float4 q[4] = {p[0], p[1], p[2], p[3]};
-        best = fmaxf(best, subblock_amax(q));
+    // sixteen contiguous KB per block and trip, four requests of 1 KB per wave in flight
+    const unsigned long long n4 = 4 * n_sub, T = blockDim.x, step = 4 * T * gridDim.x;
+    const float4* p = (const float4*)values;
+    for (unsigned long long i = 4 * T * blockIdx.x + threadIdx.x; i < n4; i += step) {
+        if (i + 3 * T < n4) {
+            const float4 q[4] = {p[i], p[i + T], p[i + 2 * T], p[i + 3 * T]};
+            best = fmaxf(best, subblock_amax(q));
+        } else {
+            for (unsigned long long e = i; e < n4 && e < i + 4 * T; e += T)
+                best = fmaxf(fmaxf(fmaxf(fmaxf(best, fabsf(p[e].x)), fabsf(p[e].y)), fabsf(p[e].z)), fabsf(p[e].w));
+        }
     }
     for (int o = 32; o > 0; o >>= 1) best = fmaxf(best, __shfl_xor(best, o));
     if ((threadIdx.x & 63u) == 0) per_wave[threadIdx.x >> 6] = best;
@@ -240,13 +274,14 @@ extern "C" __global__ void __launch_bounds__(256) quantize_nvfp4_amax(const floa
         if (best > 0.0f) atomicMax(max_bits, __float_as_uint(best));
     }
 }
-// pass 2: one thread per sub-block: its scale byte and its sixteen codes; thread 0 also leaves the global scale
+// pass 2: one thread per sub-block: its scale byte and its sixteen codes; thread 0 also leaves the global scale.  The blocks run
+// from the end of the tensor to its start: what pass 1 read last is still in the memory-side cache.
 extern "C" __global__ void __launch_bounds__(256) quantize_nvfp4_encode(const float* __restrict__ values, unsigned long long n_sub,
                                                                          const unsigned* __restrict__ max_bits, unsigned char* __restrict__ blocks,
                                                                          float* __restrict__ global_out) {
     const float max_scale = __fdiv_rn(__uint_as_float(*max_bits), 6.0f);  // the largest raw scale (see pass 1)
     const float global = max_scale > 0.0f ? __fdiv_rn(max_scale, 448.0f) : 1.0f;
-    const unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned long long i = (unsigned long long)(gridDim.x - 1 - blockIdx.x) * blockDim.x + threadIdx.x;
     if (i == 0) global_out[0] = global;
     if (i >= n_sub) return;
     const float4* p = (const float4*)(values + 16 * i);
@@ -268,10 +303,13 @@ extern "C" __global__ void __launch_bounds__(256) quantize_nvfp4_encode(const fl
     }
     unsigned char* blk = blocks + (i >> 2) * CROW_BLOCK_BYTES;
     const unsigned sb = (unsigned)(i & 3);
-    blk[sb] = (unsigned char)byte;
-    unsigned* codes = (unsigned*)(blk + 4 + 8 * sb);  // (36-byte blocks: every code dword is four-byte aligned)
-    codes[0] = lo;
-    codes[1] = hi;
+    // the four scale bytes of a block meet in its first thread (n_sub is a multiple of four: whole quads are here)
+    unsigned scales = byte << (8 * sb);
+    scales |= (unsigned)__builtin_amdgcn_mov_dpp((int)scales, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+    scales |= (unsigned)__builtin_amdgcn_mov_dpp((int)scales, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+    if (sb == 0) *(unsigned*)blk = scales;
+    typedef unsigned u32x2_dword __attribute__((ext_vector_type(2), aligned(4)));  // (36-byte blocks: code dwords are four-byte aligned)
+    *(u32x2_dword*)(blk + 4 + 8 * sb) = u32x2_dword{lo, hi};
 }
 
 // ------------------------------------------------------------------ router

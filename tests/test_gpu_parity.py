@@ -58,6 +58,30 @@ def test_repack_round_trip_and_dequant_bits(eng, rows, cols):
     eng.check()
 
 
+# groups per strip around the four that share a block, a partial last group, a partial last strip
+@pytest.mark.parametrize("rows,cols", [(1, 64), (17, 256), (15, 960), (33, 1024), (16, 1088), (5, 2304)])
+def test_encode_repack_dequant_at_the_edges_of_their_blocks(eng, rows, cols):
+    from crow_nest_amd import lib
+    from crow_nest_amd.weights import dequant, load_fp4_quantized, quantize_nvfp4, unpack
+    v = normal_f32(11, rows + cols, rows * cols) * np.exp2(normal_f32(12, rows, rows * cols))
+    v[:64] = 0.0
+    v[-1] = np.float32(3.0e38)  # one value that dwarfs the rest; most scale bytes become the smallest ones
+    v[-2] = np.nan  # ignored by the maxima, code 0
+    for values in (v[:-16 * 4] if rows * cols > 64 else v[:64], v):
+        want, want_gs = orc.quantize_ceil(values)
+        blocks, gs = quantize_nvfp4(torch.from_numpy(values).cuda())
+        assert np.array_equal(blocks.cpu().numpy(), want) and float(gs.item()) == want_gs
+    f = load_fp4_quantized(blocks, gs, rows, cols)
+    ref = orc.dequant(want, want_gs)
+    assert np.array_equal(unpack(f), np.where((want.reshape(-1, 36) == 0x7F) & (np.arange(36) < 4), 0x7E, want.reshape(-1, 36)).reshape(-1))
+    assert np.array_equal(dequant(f).cpu().numpy().reshape(-1).view(np.uint32), ref.view(np.uint32))
+    # an output that starts at an odd dword, with nothing written outside it
+    out = torch.full((rows * cols + 8,), -1.0, device="cuda")
+    lib.check(lib.lib().crow_hip_dequant_tiled(f.w_ptr, f.gs_ptr, rows, cols, out[1:].data_ptr()), "crow_hip_dequant_tiled")
+    got = out.cpu().numpy()
+    assert np.array_equal(got[1:1 + rows * cols].view(np.uint32), ref.view(np.uint32)) and got[0] == -1.0 and (got[1 + rows * cols:] == -1.0).all()
+
+
 def test_dequant_every_scale_byte_and_the_refused_one(eng):
     from crow_nest_amd.lib import CrowHipError
     from crow_nest_amd.weights import dequant
