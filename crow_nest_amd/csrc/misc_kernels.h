@@ -754,6 +754,8 @@ extern "C" __global__ void __launch_bounds__(1024) argmax_finish(int* __restrict
 //                              the grid of the reference's block-per-row kernels, whose call sites keep their dims.
 // Order: a lane adds its products in column order with one FMA each, four steps of loads in flight at a time, then the
 // 64 lane sums are added by halving (lane l += lane l + 32, + 16, ... + 1), then (second shape) the wave sums in wave order.
+// Bound by latency (a row is 8 KB): weights and activations of four steps are requested together; [256, 2048] f32: one token 3.3 us
+// (3.6 with the activations requested behind the weights), 64 tokens 10.7 us (12.6).
 //   gemv_bf16_w   engine/src/kernels.rs:1130-1157 (warp per row; k_dim % 8 == 0)
 //   gemv_bf16     engine/src/kernels.rs:1061-1077 (block per row, one token; + rows_p: the reference's grid.x is the row count)
 //   gemv_bf16_b   engine/src/kernels.rs:1080-1098 (block per row, grid.y tokens; + rows_p)
@@ -774,37 +776,63 @@ __device__ __forceinline__ void keep_gemv_body(const void* __restrict__ w, const
     const float* xp = x + (size_t)t * k;
     const int run = parts * 64 * PER;  // columns between two loads of a lane
     float acc = 0.0f;
-    for (int i0 = (part * 64 + lane) * PER; i0 < k; i0 += 4 * run) {
+    auto add = [&](const uint4& v, const float4& a, const float4& b) {
+        if (WBF16) {
+            acc = __builtin_fmaf(__uint_as_float(v.x << 16), a.x, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.x & 0xffff0000u), a.y, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.y << 16), a.z, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.y & 0xffff0000u), a.w, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.z << 16), b.x, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.z & 0xffff0000u), b.y, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.w << 16), b.z, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.w & 0xffff0000u), b.w, acc);
+        } else {
+            acc = __builtin_fmaf(__uint_as_float(v.x), a.x, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.y), a.y, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.z), a.z, acc);
+            acc = __builtin_fmaf(__uint_as_float(v.w), a.w, acc);
+        }
+    };
+    int i0 = (part * 64 + lane) * PER;
+    // four steps at a time, weights and activations requested together: one round trip a trip, not two.  With several
+    // activation rows in the launch the weights are read again (from the die's L2): plain loads
+    const bool reread = gridDim.y > 1;  // uniform
+    for (; i0 + 3 * run < k; i0 += 4 * run) {
         uint4 v[4];
+        float4 a[4], b[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
+            const int i = i0 + j * run;
+            a[j] = *(const float4*)(xp + i);
+            b[j] = WBF16 ? *(const float4*)(xp + i + 4) : a[j];
+        }
+        if (reread) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = *(const uint4*)(wp + (size_t)(i0 + j * run) * (WBF16 ? 2 : 4));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = stream_load((const uint4*)(wp + (size_t)(i0 + j * run) * (WBF16 ? 2 : 4)));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) add(v[j], a[j], b[j]);
+    }
+    if (i0 < k) {  // up to three steps more, requested together as well
+        uint4 v[3];
+        float4 a[3], b[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
             const int i = i0 + j * run;
             v[j] = make_uint4(0, 0, 0, 0);
-            if (i < k) v[j] = stream_load((const uint4*)(wp + (size_t)i * (WBF16 ? 2 : 4)));
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = i0 + j * run;
+            a[j] = b[j] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (i < k) {
-                const float4 a = *(const float4*)(xp + i);
-                if (WBF16) {
-                    const float4 b = *(const float4*)(xp + i + 4);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].x << 16), a.x, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].x & 0xffff0000u), a.y, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].y << 16), a.z, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].y & 0xffff0000u), a.w, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].z << 16), b.x, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].z & 0xffff0000u), b.y, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].w << 16), b.z, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].w & 0xffff0000u), b.w, acc);
-                } else {
-                    acc = __builtin_fmaf(__uint_as_float(v[j].x), a.x, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].y), a.y, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].z), a.z, acc);
-                    acc = __builtin_fmaf(__uint_as_float(v[j].w), a.w, acc);
-                }
+                v[j] = stream_load((const uint4*)(wp + (size_t)i * (WBF16 ? 2 : 4)));
+                a[j] = *(const float4*)(xp + i);
+                if (WBF16) b[j] = *(const float4*)(xp + i + 4);
             }
         }
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            if (i0 + j * run < k) add(v[j], a[j], b[j]);
     }
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
     auto finish = [](float v) { return SIGMOID ? 1.0f / (1.0f + expf(-v)) : v; };
