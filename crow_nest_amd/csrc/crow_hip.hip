@@ -96,6 +96,7 @@ struct State {
     hipStream_t stream = nullptr;
     crow::Workspace ws{};
     crow::Workspace ws_static{};  // the same roles inside `scratch`, through the device address crow_hip_init asked for
+    unsigned* said = nullptr;  // pinned host words: the two status words as the layout calls last read them, eight pairs in turn
     int* scalars = nullptr;  // device words for the library's own launches: (rows, k_dim) of the layout calls, the encoder's maxima
     char name[256] = {0};
     crow::Geo model{0, 0, 0, 0};  // the routed geometry (crow_hip_set_geo): appended by value to the kernels that take it
@@ -225,12 +226,14 @@ int crow_hip_init(int device) {
     ws.partial_floats = PARTIAL_FLOATS;
     ws.counter_slots = COUNTER_SLOTS;
     int* scalars = nullptr;
+    unsigned* said = nullptr;
     // one failure path: everything allocated so far is released again
     auto fail = [&](hipError_t why) {
         (void)hipFree(ws.partials);
         (void)hipFree(ws.counters);
         (void)hipFree(ws.head);
         (void)hipFree(scalars);
+        (void)hipHostFree(said);
         return (int)why;
     };
     if ((e = hipMalloc((void**)&ws.partials, PARTIAL_FLOATS * sizeof(float))) != hipSuccess) return fail(e);
@@ -239,6 +242,7 @@ int crow_hip_init(int device) {
     if ((e = hipMemset(ws.head, 0, HEAD_WORDS * sizeof(unsigned long long))) != hipSuccess) return fail(e);
     ws.head_words = HEAD_WORDS;
     if ((e = hipMalloc((void**)&scalars, 32 * sizeof(int))) != hipSuccess) return fail(e);  // words 0..15: (rows, k_dim) of the layout calls, 16..23: the encoder's maxima, 24: the read probe's sink
+    if ((e = hipHostMalloc((void**)&said, 16 * sizeof(unsigned), hipHostMallocDefault)) != hipSuccess) return fail(e);
     if ((e = hipMemset(ws.counters, 0, COUNTER_WORDS * sizeof(unsigned))) != hipSuccess) return fail(e);
     ws.status = ws.counters + COUNTER_SLOTS;
     if ((e = hipMemcpyToSymbol(HIP_SYMBOL(crow::g_ws), &ws, sizeof ws)) != hipSuccess) return fail(e);
@@ -273,6 +277,7 @@ int crow_hip_init(int device) {
     if ((e = hipMemset(st.counters, 0, (NOALLOC_COUNTER_SLOTS + NOALLOC_TAIL_WORDS) * sizeof(unsigned))) != hipSuccess) return fail(e);
     if ((e = hipDeviceSynchronize()) != hipSuccess) return fail(e);
     g.scalars = scalars;
+    g.said = said;
     g.ws = ws;
     g.ws_static = st;
     g.device = device;
@@ -288,6 +293,7 @@ int crow_hip_shutdown(void) {
     (void)hipFree(g.ws.counters);
     (void)hipFree(g.ws.head);
     (void)hipFree(g.scalars);
+    (void)hipHostFree(g.said);
     g = State{};
     return CROW_OK;
 }
@@ -804,13 +810,15 @@ uint32_t crow_hip_tile_scale_offset(uint32_t row, uint32_t sb) { return row < 16
 static int layout_launch(const char* name, const void* a, const void* b, const void* c, uint32_t rows, uint32_t cols) {
     if (!g.ready) return CROW_ERR_NOT_INITIALIZED;
     if (!a || !b || rows == 0 || cols == 0 || cols % CROW_BLOCK_VALUES != 0) return a && b ? CROW_ERR_SHAPE : CROW_ERR_BAD_ARGUMENT;
-    // the two scalars ride in a small ring of device words so that back-to-back calls do not race
-    static int slot = 0;
-    int* sc = g.scalars + 2 * (slot++ & 7);
-    int host[2] = {(int)rows, (int)cols};
-    hipError_t e = hipMemcpyAsync(sc, host, sizeof host, hipMemcpyHostToDevice, g.stream);
+    // the two scalars ride in a small ring of device words so that back-to-back calls do not race; a kernel writes them (a copy
+    // from the stack would have to be waited for)
+    static std::atomic<unsigned> slot{0};
+    const unsigned turn = slot.fetch_add(1) & 7u;
+    int* sc = g.scalars + 2 * turn;
+    int r = (int)rows, c2 = (int)cols;
+    void* a0[3] = {(void*)&sc, (void*)&r, (void*)&c2};
+    hipError_t e = hipLaunchKernel((const void*)&layout_words, dim3(1), dim3(1), a0, 0, g.stream);
     if (e != hipSuccess) return (int)e;
-    if ((e = hipStreamSynchronize(g.stream)) != hipSuccess) return (int)e;  // `host` is a stack buffer
     crow_dims d;
     int rc = crow_hip_launch_dims(name, rows, cols, 1, &d);
     if (rc != CROW_OK) return rc;
@@ -823,7 +831,13 @@ static int layout_launch(const char* name, const void* a, const void* b, const v
     vals[n++] = (uint64_t)(sc + 1);
     rc = launch_entry(find(name), dim3(d.gx, d.gy, d.gz), dim3(d.bx), vals, n, g.stream, g.ws);
     if (rc != CROW_OK) return rc;
-    return crow_hip_status();
+    // both status words come back in pinned memory behind the kernel, so that one wait for the device is all the host does; what
+    // they say when one is raised is crow_hip_status's to report (a bit raised meanwhile on another stream stays for the next call)
+    unsigned* said = g.said + 2 * turn;
+    void* a1[3] = {(void*)&g.ws.status, (void*)&g.ws_static.status, (void*)&said};
+    if ((e = hipLaunchKernel((const void*)&status_words, dim3(1), dim3(1), a1, 0, g.stream)) != hipSuccess) return (int)e;
+    if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
+    return (said[0] | said[1]) == 0 ? CROW_OK : crow_hip_status();
 }
 
 int crow_hip_quantize_nvfp4(const float* values_dev, size_t n_values, void* blocks_dev, float* global_scale_dev) {

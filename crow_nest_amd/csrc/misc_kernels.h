@@ -7,6 +7,10 @@ using namespace crow;
 #define CROW_STATUS_BAD_SCALE_BYTE 8u
 
 // ------------------------------------------------------------------ container <-> tiled
+// around a layout call: its two scalars into device words, and the library's two status words into pinned host memory
+extern "C" __global__ void layout_words(int* __restrict__ words, int rows, int k_dim) { words[0] = rows, words[1] = k_dim; }
+extern "C" __global__ void status_words(const unsigned* a, const unsigned* b, unsigned* host) { host[0] = *a, host[1] = *b; }
+
 // One wave per group, up to four adjacent groups of a strip (blockIdx.y) in a block.  Bound by memory: both sides are read and
 // written in whole dwords, 256 contiguous bytes per instruction on the tiled side and runs of 144 bytes (a row's share of the
 // group) on the container side; the byte shuffle between the two runs through LDS, each wave in its own part.  Adjacent groups
@@ -502,7 +506,10 @@ extern "C" __global__ void __launch_bounds__(1024) moe_route_gate_up_silu(const 
     __shared__ unsigned long long s_slab;
     const int E = model.experts, K = model.topk;
     if (E < 64 || E > 1024 || (E & (E - 1)) != 0 || K < 1 || K > 16 || K > E || table == nullptr) {
-        if (threadIdx.x == 0) atomicOr(ws.status, STATUS_BAD_GEO);
+        if (threadIdx.x == 0) {
+            atomicOr(ws.status, STATUS_BAD_GEO);
+            if (blockIdx.x == 0) dn_ptrs[blockIdx.z] = 0;  // one entry per combo: the kernel behind this one follows no stale pointer
+        }
         return;
     }
     const int combo = (int)blockIdx.z, t = combo / K, j = combo % K;

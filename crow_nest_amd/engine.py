@@ -10,7 +10,8 @@ put the HIP library behind ``gen.rs``:
     lm_head_row   gen.rs:4766-4784   lm_head through dense_proj, then argmax_k (gen.rs:6197-6198)
     moe_run       gen.rs:4168-4534   router_top10 -> routed gate|up -> SwiGLU -> routed down -> acc_combo
 Buffers are torch tensors on the device (allocation only); every launch goes through
-``launch_v(k.f(name), ...)`` with device addresses, exactly like the reference call sites.
+``k.run(name, ...)`` - ``launch_v`` under the library's launch dimensions - with device addresses, like the reference call
+sites.
 """
 from __future__ import annotations
 
@@ -18,7 +19,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .kernels import KernelGeo, Kernels, compile, launch_dims, launch_v, set_geo, status
+from .kernels import KernelGeo, Kernels, compile, launch_dims, set_geo, status
 from .weights import ExpertSlabs, Fp4, Params
 
 NVFP4_MMAX = 4  # kernels_p2.rs:397
@@ -68,16 +69,13 @@ class Engine:
             y = torch.empty((t, rows), dtype=torch.float32, device=self.dev)
         p = self.p
         if t == 1 and x.dtype == torch.float32:
-            gx, gy, gz, bx = launch_dims("gemv_nvfp4_w", rows, k)
-            launch_v(self.k.f("gemv_nvfp4_w"), gx, gy, gz, bx, [w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows)])
+            self.k.run("gemv_nvfp4_w", rows, k, 1, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows))
         elif t <= NVFP4_MMAX:
             self.proj_m(w, t, x, y)
         elif x.dtype == torch.bfloat16:
             self.gemm(w, t, x, y)
         else:
-            gx, gy, gz, bx = launch_dims("gemv_fp4_b", rows, k, t)
-            launch_v(self.k.f("gemv_fp4_b"), gx, gy, gz, bx,
-                     [w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(t)])
+            self.k.run("gemv_fp4_b", rows, k, t, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(t))
         return y
 
     def proj_m(self, w: Fp4, m: int, x: torch.Tensor, y: torch.Tensor | None = None) -> torch.Tensor:
@@ -88,9 +86,8 @@ class Engine:
         if y is None:
             y = torch.empty((m, rows), dtype=torch.float32, device=self.dev)
         name = "gemv_nvfp4_wm" if x.dtype == torch.float32 else "gemv_nvfp4_wm_bf16"
-        gx, gy, gz, bx = launch_dims(name, rows, k, m)
         p = self.p
-        launch_v(self.k.f(name), gx, gy, gz, bx, [w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m)])
+        self.k.run(name, rows, k, m, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m))
         return y
 
     def gate_up(self, mlp: MlpW, t: int, x: torch.Tensor, h: torch.Tensor | None = None) -> torch.Tensor:
@@ -102,14 +99,10 @@ class Engine:
         p = self.p
         if t == 1:
             name = "gemv_nvfp4_gu" if x.dtype == torch.float32 else "gemv_nvfp4_gu_bf16"
-            gx, gy, gz, bx = launch_dims(name, inter, k)
-            launch_v(self.k.f(name), gx, gy, gz, bx,
-                     [mlp.gate.w_ptr, mlp.up.w_ptr, x.data_ptr(), mlp.gate.gs_ptr, mlp.up.gs_ptr, h.data_ptr(), p.i32(k), p.i32(inter)])
+            self.k.run(name, inter, k, 1, mlp.gate.w_ptr, mlp.up.w_ptr, x.data_ptr(), mlp.gate.gs_ptr, mlp.up.gs_ptr, h.data_ptr(), p.i32(k), p.i32(inter))
         else:
             name = "gemv_nvfp4_gum" if x.dtype == torch.float32 else "gemv_nvfp4_gum_bf16"
-            gx, gy, gz, bx = launch_dims(name, inter, k, t)
-            launch_v(self.k.f(name), gx, gy, gz, bx,
-                     [mlp.gate.w_ptr, mlp.up.w_ptr, x.data_ptr(), mlp.gate.gs_ptr, mlp.up.gs_ptr, h.data_ptr(), p.i32(k), p.i32(inter), p.i32(t)])
+            self.k.run(name, inter, k, t, mlp.gate.w_ptr, mlp.up.w_ptr, x.data_ptr(), mlp.gate.gs_ptr, mlp.up.gs_ptr, h.data_ptr(), p.i32(k), p.i32(inter), p.i32(t))
         return h
 
     def dense_ffn_w(self, mlp: MlpW, x: torch.Tensor, t: int) -> torch.Tensor:
@@ -123,12 +116,10 @@ class Engine:
         else gemv_nvfp4_w + argmax_k over all logits, as the reference."""
         rows, k = w.rows, w.cols
         logits = torch.empty(rows, dtype=torch.float32, device=self.dev)
-        idx = torch.zeros(1, dtype=torch.int32, device=self.dev)
+        idx = torch.empty(1, dtype=torch.int32, device=self.dev)  # written by every launch
         p = self.p
         if fused:
-            gx, gy, gz, bx = launch_dims("gemv_nvfp4_w_argmax", rows, k)
-            launch_v(self.k.f("gemv_nvfp4_w_argmax"), gx, gy, gz, bx,
-                     [w.w_ptr, x.data_ptr(), w.gs_ptr, logits.data_ptr(), p.i32(k), p.i32(rows), idx.data_ptr()])
+            self.k.run("gemv_nvfp4_w_argmax", rows, k, 1, w.w_ptr, x.data_ptr(), w.gs_ptr, logits.data_ptr(), p.i32(k), p.i32(rows), idx.data_ptr())
         else:
             self.dense_proj(w, 1, x, logits.view(1, rows))
             self.argmax(logits, idx)
@@ -137,7 +128,7 @@ class Engine:
     def argmax(self, logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         if out is None:
             out = torch.zeros(1, dtype=torch.int32, device=self.dev)
-        launch_v(self.k.f("argmax_k"), 1, 1, 1, 1024, [logits.data_ptr(), out.data_ptr(), self.p.i32(logits.numel())])
+        self.k.run_at("argmax_k", 1, 1, 1, 1024, logits.data_ptr(), out.data_ptr(), self.p.i32(logits.numel()))
         return out
 
     # ------------------------------------------------------------------ routed experts
@@ -159,8 +150,7 @@ class Engine:
         gu = torch.zeros((t, k), dtype=torch.int64, device=self.dev)
         dn = torch.zeros((t, k), dtype=torch.int64, device=self.dev)
         table = moe.table.data_ptr() if moe is not None else 0
-        launch_v(self.k.f("router_top10"), t, 1, 1, 64,
-                 [logits.data_ptr(), 0, ids.data_ptr(), wts.data_ptr(), gu.data_ptr(), dn.data_ptr(), table, 0, 0, 0])
+        self.k.run_at("router_top10", t, 1, 1, 64, logits.data_ptr(), 0, ids.data_ptr(), wts.data_ptr(), gu.data_ptr(), dn.data_ptr(), table, 0, 0, 0)
         return ids, wts, gu, dn
 
     def moe_layer(self, moe: MoeW, x: torch.Tensor, logits: torch.Tensor, y: torch.Tensor | None = None):
@@ -182,25 +172,26 @@ class Engine:
         self._check_moe(moe)
         assert hdim == self.geo.hidden and moe.gate_up.rows == 2 * inter and moe.down.rows == hdim
         p = self.p
-        ids, wts, _, _ = self.router(logits, moe)
+        assert logits.shape[1] == experts and logits.dtype == torch.float32 and logits.is_contiguous()
+        routed = logits.shape[0]
+        ids = torch.empty((routed, topk), dtype=torch.int32, device=self.dev)
+        wts = torch.empty((routed, topk), dtype=torch.float32, device=self.dev)
+        # the grouped kernels look slabs up in the table themselves: no pointers per combo
+        self.k.run_at("router_top10", routed, 1, 1, 64, logits.data_ptr(), 0, ids.data_ptr(), wts.data_ptr(), 0, 0, 0, 0, 0, 0)
         combos = t * topk
         max_tiles = min(combos, experts) + combos // 4
         if y is None:
             y = torch.zeros((t, hdim), dtype=torch.float32, device=self.dev)
         perm = torch.empty((combos,), dtype=torch.int32, device=self.dev)
         tiles = torch.empty((max_tiles, 4), dtype=torch.int32, device=self.dev)
-        n_tiles = torch.zeros((1,), dtype=torch.int32, device=self.dev)
+        n_tiles = torch.empty((1,), dtype=torch.int32, device=self.dev)  # written by every moe_group, 0 where it refuses
         h2 = torch.empty((combos, inter), dtype=torch.float32, device=self.dev)
         eo = torch.empty((combos, hdim), dtype=torch.float32, device=self.dev)
         table, gs_gu, gs_dn = moe.table.data_ptr(), moe.gate_up.gs.data_ptr(), moe.down.gs.data_ptr()
-        launch_v(self.k.f("moe_group"), *launch_dims("moe_group", 1, 64, combos),
-                 [ids.data_ptr(), p.i32(combos), perm.data_ptr(), tiles.data_ptr(), n_tiles.data_ptr(), p.i32(max_tiles)])
-        launch_v(self.k.f("moe_gate_up_silu_grouped"), *launch_dims("moe_gate_up_silu_grouped", inter, hdim, max_tiles),
-                 [tiles.data_ptr(), n_tiles.data_ptr(), perm.data_ptr(), table, x.data_ptr(), gs_gu, h2.data_ptr(),
-                  p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter)])
-        launch_v(self.k.f("moe_down_grouped"), *launch_dims("moe_down_grouped", hdim, inter, max_tiles),
-                 [tiles.data_ptr(), n_tiles.data_ptr(), perm.data_ptr(), table, h2.data_ptr(), gs_dn, eo.data_ptr(), p.i32(inter), p.i32(hdim)])
-        launch_v(self.k.f("acc_combo"), (hdim + 255) // 256, t, 1, 256, [eo.data_ptr(), wts.data_ptr(), y.data_ptr()])
+        self.k.run("moe_group", 1, 64, combos, ids.data_ptr(), p.i32(combos), perm.data_ptr(), tiles.data_ptr(), n_tiles.data_ptr(), p.i32(max_tiles))
+        self.k.run("moe_gate_up_silu_grouped", inter, hdim, max_tiles, tiles.data_ptr(), n_tiles.data_ptr(), perm.data_ptr(), table, x.data_ptr(), gs_gu, h2.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter))
+        self.k.run("moe_down_grouped", hdim, inter, max_tiles, tiles.data_ptr(), n_tiles.data_ptr(), perm.data_ptr(), table, h2.data_ptr(), gs_dn, eo.data_ptr(), p.i32(inter), p.i32(hdim))
+        self.k.run_at("acc_combo", (hdim + 255) // 256, t, 1, 256, eo.data_ptr(), wts.data_ptr(), y.data_ptr())
         return ids, wts, y, (perm, tiles, n_tiles)
 
     def moe_run(self, moe: MoeW, x: torch.Tensor, logits: torch.Tensor, fused: bool = True, y: torch.Tensor | None = None):
@@ -222,32 +213,22 @@ class Engine:
             assert logits.shape == (t, self.geo.experts) and logits.dtype == torch.float32 and logits.is_contiguous()
             ids = torch.empty((t, topk), dtype=torch.int32, device=self.dev)
             wts = torch.empty((t, topk), dtype=torch.float32, device=self.dev)
-            dn = torch.zeros((t, topk), dtype=torch.int64, device=self.dev)
-            launch_v(self.k.f("moe_route_gate_up_silu"), *launch_dims("moe_route_gate_up_silu", inter, hdim, combos),
-                     [logits.data_ptr(), moe.table.data_ptr(), x.data_ptr(), gs_gu, h2.data_ptr(), ids.data_ptr(), wts.data_ptr(), dn.data_ptr(),
-                      p.i32(hdim), p.i32(hdim), p.i32(inter)])
-            launch_v(self.k.f("moe_down_combine"), *launch_dims("moe_down_combine", hdim, inter, t),
-                     [dn.data_ptr(), h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim)])
+            dn = torch.empty((t, topk), dtype=torch.int64, device=self.dev)  # written by every launch, zeros where it refuses
+            self.k.run("moe_route_gate_up_silu", inter, hdim, combos, logits.data_ptr(), moe.table.data_ptr(), x.data_ptr(), gs_gu, h2.data_ptr(), ids.data_ptr(), wts.data_ptr(), dn.data_ptr(), p.i32(hdim), p.i32(hdim), p.i32(inter))
+            self.k.run("moe_down_combine", hdim, inter, t, dn.data_ptr(), h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim))
             return ids, wts, y
         ids, wts, gu, dn = self.router(logits, moe)
         if fused:
-            gx, gy, gz, bx = launch_dims("moe_gate_up_silu", inter, hdim, combos)
-            launch_v(self.k.f("moe_gate_up_silu"), gx, gy, gz, bx,
-                     [gu.data_ptr(), x.data_ptr(), gs_gu, h2.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter)])
-            launch_v(self.k.f("moe_down_combine"), *launch_dims("moe_down_combine", hdim, inter, t),
-                     [dn.data_ptr(), h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim)])
+            self.k.run("moe_gate_up_silu", inter, hdim, combos, gu.data_ptr(), x.data_ptr(), gs_gu, h2.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter))
+            self.k.run("moe_down_combine", hdim, inter, t, dn.data_ptr(), h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim))
         else:
             h1 = torch.empty((combos, 2 * inter), dtype=torch.float32, device=self.dev)
             eo = torch.empty((combos, hdim), dtype=torch.float32, device=self.dev)
-            gx, gy, gz, bx = launch_dims("gemv_fp4_ptrb", 2 * inter, hdim, combos)
-            launch_v(self.k.f("gemv_fp4_ptrb"), gx, gy, gz, bx,
-                     [gu.data_ptr(), x.data_ptr(), gs_gu, h1.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(2 * inter)])
+            self.k.run("gemv_fp4_ptrb", 2 * inter, hdim, combos, gu.data_ptr(), x.data_ptr(), gs_gu, h1.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(2 * inter))
             n = combos * inter
-            launch_v(self.k.f("silu_mul_combo"), (n + 255) // 256, 1, 1, 256, [h1.data_ptr(), h2.data_ptr(), p.i32(n)])
-            gx, gy, gz, bx = launch_dims("gemv_fp4_ptrb", hdim, inter, combos)
-            launch_v(self.k.f("gemv_fp4_ptrb"), gx, gy, gz, bx,
-                     [dn.data_ptr(), h2.data_ptr(), gs_dn, eo.data_ptr(), p.i32(inter), p.i32(1), p.i32(inter), p.i32(hdim)])
-            launch_v(self.k.f("acc_combo"), (hdim + 255) // 256, t, 1, 256, [eo.data_ptr(), wts.data_ptr(), y.data_ptr()])
+            self.k.run_at("silu_mul_combo", (n + 255) // 256, 1, 1, 256, h1.data_ptr(), h2.data_ptr(), p.i32(n))
+            self.k.run("gemv_fp4_ptrb", hdim, inter, combos, dn.data_ptr(), h2.data_ptr(), gs_dn, eo.data_ptr(), p.i32(inter), p.i32(1), p.i32(inter), p.i32(hdim))
+            self.k.run_at("acc_combo", (hdim + 255) // 256, t, 1, 256, eo.data_ptr(), wts.data_ptr(), y.data_ptr())
         return ids, wts, y
 
     # ------------------------------------------------------------------ BF16 keeps (router, q/k, MTP head)
@@ -265,8 +246,7 @@ class Engine:
         rows, k = w.shape
         assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.numel() == t * k and y.is_cuda and y.dtype == torch.float32
         p = self.p
-        launch_v(self.k.f("gemv_bf16_bs"), *launch_dims("gemv_bf16_bs", rows, k, t),
-                 [w.data_ptr(), x.data_ptr(), y.data_ptr(), p.i32(k), p.i32(y_stride), p.i32(rows)])
+        self.k.run("gemv_bf16_bs", rows, k, t, w.data_ptr(), x.data_ptr(), y.data_ptr(), p.i32(k), p.i32(y_stride), p.i32(rows))
         return y
 
     def f32_proj(self, w: torch.Tensor, t: int, x: torch.Tensor, y: torch.Tensor | None = None) -> torch.Tensor:
@@ -282,7 +262,11 @@ class Engine:
         if y is None:
             y = torch.empty((t, rows), dtype=torch.float32, device=self.dev)
         p = self.p
-        launch_v(self.k.f(name), *launch_dims(name, rows, k, t, split=(0, waves_per_row)), [w.data_ptr(), x.data_ptr(), y.data_ptr(), p.i32(k), p.i32(rows)])
+        vals = (w.data_ptr(), x.data_ptr(), y.data_ptr(), p.i32(k), p.i32(rows))
+        if waves_per_row == 0:
+            self.k.run(name, rows, k, t, *vals)
+        else:
+            self.k.run_at(name, *launch_dims(name, rows, k, t, split=(0, waves_per_row)), *vals)
         return y
 
     # ------------------------------------------------------------------ prefill GEMM (M >= 16)
@@ -294,9 +278,8 @@ class Engine:
         if y is None:
             y = torch.empty((m, rows), dtype=torch.float32, device=self.dev)
         name = kernel or gemm_kernel_for(m, rows)
-        gx, gy, gz, bx = launch_dims(name, rows, k, m)
         p = self.p
-        launch_v(self.k.f(name), gx, gy, gz, bx, [w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m)])
+        self.k.run(name, rows, k, m, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m))
         return y
 
 

@@ -82,6 +82,27 @@ class Kernels:
         for i in range(L.crow_hip_function_count()):
             name = L.crow_hip_function_name(i).decode()
             self.map[name] = module.get(name)
+        from . import _launch  # built beside the library; missing = not built, like the library itself
+        _launch.bind(C.cast(L.crow_hip_launch_dims_split, C.c_void_p).value, C.cast(L.crow_hip_launch, C.c_void_p).value)
+        self._launch, self._launch_at = _launch.launch, _launch.launch_at
+        self._native = {name: (name.encode(), f) for name, f in self.map.items()}
+
+    def run(self, name: str, rows: int, k_dim: int, z: int, *vals: int) -> None:
+        """``launch_v(f(name), *launch_dims(name, rows, k_dim, z), vals)`` in one native call: same dimensions, same errors."""
+        try:
+            native, f = self._native[name]
+        except KeyError:
+            raise KernelMissing(f"kernel missing: {name}") from None
+        rc = self._launch(native, f, rows, k_dim, z, *vals)
+        if rc:
+            launch_dims(name, rows, k_dim, z)  # raises if the dimensions were refused
+            _l.check(rc, "launch_v")
+
+    def run_at(self, name: str, gx: int, gy: int, gz: int, bx: int, *vals: int) -> None:
+        """``launch_v(f(name), gx, gy, gz, bx, vals)`` in one native call."""
+        rc = self._launch_at(self.f(name), gx, gy, gz, bx, *vals)
+        if rc:
+            _l.check(rc, "launch_v")
 
     def f(self, name: str) -> int:
         try:

@@ -244,10 +244,12 @@ class Params:
     def __init__(self):
         self._dev = _device()
         self._cache: dict[int, torch.Tensor] = {}
+        self._ptr: dict[int, int] = {}
 
     def i32(self, v: int) -> int:
-        t = self._cache.get(v)
-        if t is None:
+        ptr = self._ptr.get(v)
+        if ptr is None:
             t = torch.tensor([v], dtype=torch.int32, device=self._dev)
-            self._cache[v] = t
-        return t.data_ptr()
+            self._cache[v] = t  # kept: the words live as long as this object
+            ptr = self._ptr[v] = t.data_ptr()
+        return ptr

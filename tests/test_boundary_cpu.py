@@ -92,6 +92,31 @@ def test_gemm_kernel_choice_by_the_fullest_compute_unit():
             assert (d.gx, d.gy, d.gz, d.bx) == (-(-rows // 320) * -(-m // mt), 1, 1, 256)
 
 
+def test_native_launch_call_arguments():
+    """The package's native launch call hands its integers to the library and returns the library's codes; what is not an
+    integer, or too much, raises.  (Nothing is launched: the library is not initialised here.)"""
+    import ctypes as C
+    import torch
+    from crow_nest_amd import _launch
+    lib = L.lib()
+    _launch.bind(C.cast(lib.crow_hip_launch_dims_split, C.c_void_p).value, C.cast(lib.crow_hip_launch, C.c_void_p).value)
+    f = C.c_void_p()
+    assert lib.crow_hip_get_function(b"gemv_nvfp4_w", C.byref(f)) == 0
+    vals = [16] * 6
+    assert _launch.launch(b"no_such_kernel", f.value, 16, 256, 1, *vals) == -2
+    assert _launch.launch(b"gemv_nvfp4_w", f.value, 16, 100, 1, *vals) == -7  # K is no whole block
+    assert _launch.launch(b"gemv_nvfp4_w", 0, 16, 256, 1, *vals) == -2 and _launch.launch_at(0, 1, 1, 1, 64, *vals) == -2
+    if not torch.cuda.is_available():
+        assert _launch.launch(b"gemv_nvfp4_w", f.value, np.int64(16), 256, 1, *vals) == -1  # not initialised
+        assert _launch.launch_at(f.value, 1, 4, 1, 64, *vals) == -1
+    for bad in ((b"gemv_nvfp4_w", f.value, 16, 256, 1, 1.5), ("gemv_nvfp4_w", f.value, 16, 256, 1), (b"gemv_nvfp4_w", f.value, 16), (b"x",) + (1,) * 40):
+        with pytest.raises(TypeError):
+            _launch.launch(*bad)
+    for bad in (-1, 1 << 32):
+        with pytest.raises(OverflowError):
+            _launch.launch(b"gemv_nvfp4_w", f.value, bad, 256, 1, *vals)
+
+
 def test_launch_dims_depend_on_the_matrix_only():
     import ctypes as C
     lib = L.lib()

@@ -1088,6 +1088,26 @@ def test_launches_with_a_wrong_block_shape_are_refused(eng):
     eng.check()
 
 
+def test_a_refused_routing_launch_leaves_no_pointers(eng):
+    """The fused routing launch under a geometry it does not take (none set) writes zeros over whatever its pointer buffer held:
+    the engine hands it uninitialised memory, and the down kernel behind it must not follow that."""
+    from crow_nest_amd.kernels import KernelGeo, launch_dims, launch_v, set_geo
+    from crow_nest_amd.lib import CrowHipError
+    E, H, I, K, p = eng.geo.experts, eng.geo.hidden, eng.geo.inter, eng.geo.topk, eng.p
+    z = torch.zeros((3, max(E, H, I)), device="cuda")
+    dn = torch.full((3, K), 0x7777, dtype=torch.int64, device="cuda")
+    dims = launch_dims("moe_route_gate_up_silu", I, H, 3 * K)
+    try:
+        set_geo(KernelGeo())
+        launch_v(eng.k.f("moe_route_gate_up_silu"), *dims, [z.data_ptr(), z.data_ptr(), z.data_ptr(), z.data_ptr(), z.data_ptr(), z.data_ptr(), z.data_ptr(),
+                                                            dn.data_ptr(), p.i32(H), p.i32(H), p.i32(I)])
+        with pytest.raises(CrowHipError) as ei:
+            eng.check()
+        assert ei.value.code == -8 and not dn.any()
+    finally:
+        set_geo(eng.geo)
+
+
 def test_an_unsupported_geometry_is_refused_and_an_empty_pointer_table_is_not_followed(eng):
     """crow_hip_set_geo refuses an expert count the routing kernels do not take (on the host, nothing launched); and the
     routed kernels, handed a pointer table a refused routing launch would have left as zeros, report through the status
