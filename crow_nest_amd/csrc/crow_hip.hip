@@ -30,7 +30,11 @@ struct FnEntry {
     // dimensions say so; its dynamic LDS is the zero area and one staging area of twelve rows per GROUP (per block, not per wave)
     const void* tile_stub;
     bool takes_geo;  // the launcher appends the model geometry (crow_hip_set_geo) by value, last
+    const void* one_stub = nullptr;  // a twin of `stub` with one strip per block, started in its place when S = CROW_ONE_STRIP
 };
+// value of S in a launch's `gy` word (GEMV family, K up to 16384): one slice, and one strip per block where the kernel otherwise
+// takes `ns` of them.  A strip of at most 64 groups never has that many slices.
+#define CROW_ONE_STRIP 0x81u
 
 // The launcher builds a kernel's argument array from the fields of its table entry: the caller's `nargs` values, then the
 // geometry word (GEMV family), the scratch descriptor (takes_ws), the model geometry (takes_geo).  A kernel that gains a
@@ -55,12 +59,15 @@ constexpr int checked_nargs(F) {
 // (the bodies for several rows need more registers than a block of sixteen waves leaves each: they run in blocks of eight)
 #define CROW_GEMV(name, nargs, NR, MMAX, XBF16) \
     {#name, (const void*)&name, checked_nargs<nargs, 2>(&name), 0u, NR, MMAX > 1 ? 8 : 16, crow::crow_gemv_lds_per_wave(MMAX, XBF16), MMAX > 1 ? (XBF16 ? CROW_MULTI_STRIPS_BF16 : CROW_MULTI_STRIPS) : 1, true, nullptr, false}
+// ... with a twin for one strip per block
+#define CROW_GEMV_ONE(name, nargs, NR, MMAX) \
+    {#name, (const void*)&name, checked_nargs<nargs, 2>(&name) + 0 * checked_nargs<nargs, 2>(&name##_one), 0u, NR, 8, crow::crow_gemv_lds_per_wave(MMAX, false), CROW_MULTI_STRIPS, true, nullptr, false, (const void*)&name##_one}
 #define CROW_GEMV_GEO(name, nargs, NR, MMAX, XBF16) \
     {#name, (const void*)&name, checked_nargs<nargs, 3>(&name), 0u, NR, 16, crow::crow_gemv_lds_per_wave(MMAX, XBF16), 1, true, nullptr, true}
 const FnEntry g_table[] = {
     CROW_GEMV(gemv_nvfp4_w, 6, 1, 1, false),       CROW_GEMV(gemv_nvfp4_w_bf16, 6, 1, 1, true),  CROW_GEMV(gemv_nvfp4_w_argmax, 7, 1, 1, false),
     CROW_GEMV(gemv_nvfp4_gu, 8, 2, 1, false),      CROW_GEMV(gemv_nvfp4_gu_bf16, 8, 2, 1, true),
-    CROW_GEMV(gemv_nvfp4_wm, 7, 1, 4, false),      CROW_GEMV(gemv_nvfp4_gum, 9, 2, 4, false),
+    CROW_GEMV_ONE(gemv_nvfp4_wm, 7, 1, 4),         CROW_GEMV_ONE(gemv_nvfp4_gum, 9, 2, 4),
     CROW_GEMV(gemv_nvfp4_wm_bf16, 7, 1, 4, true),  CROW_GEMV(gemv_nvfp4_gum_bf16, 9, 2, 4, true), CROW_GEMV(gemv_fp4, 6, 1, 1, false),
     CROW_GEMV(gemv_fp4_b, 7, 1, 4, false),         CROW_GEMV(gemv_fp4_b1k, 7, 1, 4, false),      CROW_GEMV(gemv_fp4_bs, 8, 1, 4, false),
     CROW_GEMV(gemv_fp4_ptrb, 8, 1, 1, false),      CROW_GEMV(moe_gate_up_silu, 8, 2, 1, false),  CROW_GEMV_GEO(moe_down_combine, 7, 1, 1, false),
@@ -177,10 +184,12 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
             grid.y = 1;
             lds = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)tile_groups(e->nr, (unsigned)pairs) * (size_t)(e->lds_per_wave / 2);
         } else {
-            const int slices = (int)(word >> 24) == 0 ? 1 : (int)(word >> 24);
+            const bool one = e->one_stub != nullptr && (word >> 24) == CROW_ONE_STRIP && pairs <= 64 * CROW_GROUP_PAIRS;
+            const int slices = one || (word >> 24) == 0 ? 1 : (int)(word >> 24);
+            if (one) stub = e->one_stub;
             lds = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)waves * (size_t)e->lds_per_wave;
             // a split launch must fit the scratch memory it is given (the kernels check again and report through the status word)
-            if (slices > 1 && ((unsigned long long)grid.x * grid.z * (unsigned)slices * (unsigned)(e->nr * e->ns) * 64ull > ws.partial_floats ||
+            if (slices > 1 && ((unsigned long long)grid.x * grid.z * (unsigned)slices * (unsigned)(e->nr * (one ? 1 : e->ns)) * 64ull > ws.partial_floats ||
                                (unsigned long long)grid.x * grid.z > ws.counter_slots))
                 return CROW_ERR_WORKSPACE;
             geo = (int)(word & 0xFFFFFFu);
@@ -255,6 +264,9 @@ int crow_hip_init(int device) {
         }
         if (most > 48 * 1024 &&
             (e = hipFuncSetAttribute(g_table[i].stub, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most)) != hipSuccess)
+            return fail(e);
+        if (g_table[i].one_stub != nullptr && most > 48 * 1024 &&
+            (e = hipFuncSetAttribute(g_table[i].one_stub, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most)) != hipSuccess)
             return fail(e);
         // the twin for short strips stages up to eight groups of twelve rows per block
         const size_t tile_most = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)CROW_TILE_MAX_GROUPS * (size_t)(g_table[i].lds_per_wave / 2);
@@ -480,9 +492,16 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
             const uint32_t per_wave = e->nr == 2 ? 10 : 7;
             w = (groups + per_wave - 1) / per_wave;
             s = 1;
+            // One tensor of up to 512 strips leaves the chip idle between such long walks: four waves there.  Measured with w = 1..8 at
+            // 512 to 17408 rows, K = 1024..5120 and 1 to 64 rows of activations (us, one row unless said): [512, 2048] 3.7 -> 3.3,
+            // [6151, 3008] 5.9 -> 4.8 (three rows 8.9 -> 7.0), [1024, 5120] 5.4 -> 5.0 (three rows 10.1 -> 8.6), 64 rows 52.5 -> 47.2 at
+            // [4096, 5120].  Eight would win again up to four rows (4.3) and lose from sixteen on (60 against 47); at 1088 strips and 8
+            // groups four waves lose (one row 8.1 against 7.1, five 13.6 against 12.3).  Up to seven groups a wave walks the strip
+            // alone, here and in the grouped expert kernels.
             // (The split depends on the tensor's shape only, never on the number of tokens or experts in the launch: a token's
             // bits are the same in every batch, and the grouped expert kernels reproduce them.  Four waves per tensor at
             // batch 1 would take routed gate|up [1024, 2048] x 8 experts from 8.0 to 7.2 us and give that up.)
+            if (e->nr == 1 && strips <= 512 && groups > 7 && w < 4) w = 4;
         } else {
             w = 4;
             s = (groups + 13) / 14;
@@ -497,9 +516,14 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         }
         const uint32_t gz = routed ? z : (tokens ? (z + 3) / 4 : 1);
         const uint32_t hint = from_memory ? 0 : (verify ? z : (tokens ? (z - 1) % 4 + 1 : 0));
-        const uint32_t gx = (strips + (uint32_t)e->ns - 1) / (uint32_t)e->ns;
-        *out = crow_dims{gx, pairs | (hint << 20) | (s << 24), gz, 64u * w * (uint32_t)e->nr};
-        if (s > 1 && ((unsigned long long)gx * gz * s * (unsigned)(e->nr * e->ns) * 64 > PARTIAL_FLOATS || (unsigned long long)gx * gz > COUNTER_SLOTS)) return CROW_ERR_WORKSPACE;
+        // Two strips per block share the operand reads of several f32 rows; where that leaves compute units without a block, and
+        // up to two blocks a unit where a strip is short, one strip per block is faster (three rows, us, two / one strips per block:
+        // [2048, 5120] 8.6 / 7.4, [4096, 5120] 8.7 / 8.3, [8192, 2048] 6.0 / 5.5, [6151, 3008] 7.0 / 6.7; [5120, 5120] 8.8 / 10.1,
+        // [12288, 3072] 9.2 / 9.6; gate|up [4096, 5120] 13.3 / 11.3, [5120, 2048] 10.8 / 11.1).  Same bits.
+        const bool one = e->one_stub != nullptr && s == 1 && (strips <= 256 || (e->nr == 1 && strips <= 512 && groups <= 12));
+        const uint32_t ns = one ? 1u : (uint32_t)e->ns, gx = (strips + ns - 1) / ns;
+        *out = crow_dims{gx, pairs | (hint << 20) | ((one ? CROW_ONE_STRIP : s) << 24), gz, 64u * w * (uint32_t)e->nr};
+        if (s > 1 && ((unsigned long long)gx * gz * s * (unsigned)(e->nr * ns) * 64 > PARTIAL_FLOATS || (unsigned long long)gx * gz > COUNTER_SLOTS)) return CROW_ERR_WORKSPACE;
         return CROW_OK;
     }
     if (strncmp(name, "gemv_nvfp4_w_valu", 17) == 0) {  // a 16-lane group per RG rows, four groups per wave, four waves per block

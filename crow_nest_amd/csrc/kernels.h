@@ -161,6 +161,27 @@ extern "C" __global__ void __launch_bounds__(512) gemv_nvfp4_gum(const unsigned 
     GemvArgs a = gemv_args(wg, wu, gs_g, gs_u, x, (size_t)pairs * CROW_PAIR_COLS, y, 0, pairs, k_dim_p, rows_p);
     gemv_m_dispatch<2, false, EPI_SILU_GU>(a, rows_of(a, geo, m_p), 0, LDS, ws);
 }
+// The two kernels above with ONE strip per block, which the launcher starts in their place when the launch dimensions say
+// so (crow_hip_launch_dims: tensors of few strips).  Same bits: a strip's waves and their runs of columns are the same.
+extern "C" __global__ void __launch_bounds__(512) gemv_nvfp4_wm_one(const unsigned char* __restrict__ w, const float* __restrict__ x,
+                                                                     const float* __restrict__ gs_ptr, float* __restrict__ y,
+                                                                     const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
+                                                                     const int* __restrict__ m_p, int geo, const Workspace ws) {
+    ENTER(w, x, gs_ptr, y, k_dim_p, rows_p, m_p, geo);
+    const int pairs = geo & 0xFFFFF;
+    GemvArgs a = gemv_args(w, nullptr, gs_ptr, nullptr, x, (size_t)pairs * CROW_PAIR_COLS, y, 0, pairs, k_dim_p, rows_p);
+    gemv_m_dispatch<1, false, EPI_SCALE, 1>(a, rows_of(a, geo, m_p), 0, LDS, ws);
+}
+extern "C" __global__ void __launch_bounds__(512) gemv_nvfp4_gum_one(const unsigned char* __restrict__ wg, const unsigned char* __restrict__ wu,
+                                                                       const float* __restrict__ x, const float* __restrict__ gs_g,
+                                                                       const float* __restrict__ gs_u, float* __restrict__ y,
+                                                                       const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
+                                                                       const int* __restrict__ m_p, int geo, const Workspace ws) {
+    ENTER(wg, wu, x, gs_g, gs_u, y, k_dim_p, rows_p, m_p, geo);
+    const int pairs = geo & 0xFFFFF;
+    GemvArgs a = gemv_args(wg, wu, gs_g, gs_u, x, (size_t)pairs * CROW_PAIR_COLS, y, 0, pairs, k_dim_p, rows_p);
+    gemv_m_dispatch<2, false, EPI_SILU_GU, 1>(a, rows_of(a, geo, m_p), 0, LDS, ws);
+}
 // bf16-activation twins of the two verify kernels (X [M][k_dim] bf16, outputs f32)
 extern "C" __global__ void __launch_bounds__(512) gemv_nvfp4_wm_bf16(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x,
                                                                       const float* __restrict__ gs_ptr, float* __restrict__ y,

@@ -406,6 +406,34 @@ def test_record_kernel_entry_points_by_their_own_names(eng):
     eng.check()
 
 
+# the edges of the rules that shorten a wave's walk (512 strips, 7 groups) and take one strip per block (256 strips; 512 and 12 groups)
+@pytest.mark.parametrize("rows,cols", [(17, 64), (4096, 1792), (4097, 1856), (8192, 3072), (8177, 3136), (8193, 2048), (250, 5120)])
+@pytest.mark.parametrize("gu", [False, True])
+def test_verify_rows_keep_the_decode_rows_bits_under_every_split(eng, rows, cols, gu):
+    """Rows of an M-row launch equal one-row launches bit for bit, with one strip per block and with two."""
+    from crow_nest_amd.kernels import launch_dims, launch_v
+    ws = [_load(random_nvfp4(rows + i, rows, cols), rows, cols, 1.1e-3) for i in range(2 if gu else 1)]
+    x = _dev(normal_f32(9, rows, 3 * cols).reshape(3, cols))
+    p, one, many = eng.p, ("gemv_nvfp4_gu" if gu else "gemv_nvfp4_w"), ("gemv_nvfp4_gum" if gu else "gemv_nvfp4_wm")
+    head = [w.w_ptr for w in ws]
+
+    def run(name, dims, xv, m):
+        y = torch.full((m, rows), float("nan"), device="cuda")
+        launch_v(eng.k.f(name), *dims, head + [xv.data_ptr()] + [w.gs_ptr for w in ws] + [y.data_ptr(), p.i32(cols), p.i32(rows)] + ([p.i32(m)] if name == many else []))
+        eng.check()
+        return y
+
+    ref = torch.cat([run(one, launch_dims(one, rows, cols), x[i], 1) for i in range(3)])
+    gx, gy, gz, bx = launch_dims(many, rows, cols, 3)
+    strips = (rows + 15) // 16
+    assert gy >> 24 in (1, 0x81) and gx == (strips if gy >> 24 == 0x81 else (strips + 1) // 2)
+    assert torch.equal(run(many, (gx, gy, gz, bx), x, 3), ref)
+    assert torch.equal(run(many, (strips, (gy & 0xFFFFFF) | (0x81 << 24), gz, bx), x, 3), ref)
+    assert torch.equal(run(many, ((strips + 1) // 2, (gy & 0xFFFFFF) | (1 << 24), gz, bx), x, 3), ref)
+    if not gu:
+        assert rel_err(ref[0].cpu().numpy(), orc.gemv(random_nvfp4(rows, rows, cols), rows, cols, 1.1e-3, x[0].cpu().numpy())[0], floor_of(rows)) <= TOL
+
+
 # ---------------------------------------------------------------- head
 
 def test_lm_head_logits_and_greedy_token(eng):
