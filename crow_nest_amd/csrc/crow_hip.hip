@@ -408,6 +408,7 @@ const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) {
     const char* best = nullptr;
     double best_t = 0.0;
     for (const auto& c : cand) {
+        if (c.mt == 32 && (m + 31ull) / 32 > 65535) continue;  // its token blocks are the grid's second dimension
         const unsigned long long blocks = ((strips + c.strips - 1) / c.strips) * ((m + c.mt - 1) / c.mt);
         const double t = c.start + c.each * (double)((blocks + cus - 1) / cus);
         if (best == nullptr || t < best_t) {
@@ -550,7 +551,7 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         if (name[15] == '_' && name[16] == 't') {  // gemm_nvfp4_bf16_t<tokens per block>: four waves of five strips
             const uint32_t mtt = (uint32_t)atoi(name + 17);
             const unsigned long long tiles = (unsigned long long)((strips + 19) / 20) * ((z + mtt - 1) / mtt);
-            if (tiles > 0x7FFFFFFFull) return CROW_ERR_SHAPE;
+            if (tiles > 0x7FFFFFFFull || k_dim >= 1u << 25) return CROW_ERR_SHAPE;
             *out = crow_dims{(uint32_t)tiles, 1, 1, 256};
             return CROW_OK;
         }

@@ -422,8 +422,9 @@ struct TallTile {
     u32x4 B[2];
     f32x4 acc[TBK][NJ];
     const unsigned char* wp[NJ];
-    unsigned xrow, xlast, kd;  // element offsets of this thread's first row of X and of the last row; the row stride
-    const unsigned short* x;
+    unsigned xrow, xlast, kd;  // element offsets, from the block's first token row, of this thread's first row of X and of the last
+                               // row; the row stride.  A block's rows fit 32 bits (K < 2^25), all of X need not.
+    const unsigned short* x;   // the block's first token row
     const __bf16 *cur, *nxt;  // this lane's view of the X tile that is being multiplied / of the next one
     __bf16* put;              // this thread's first chunk of the next X tile
     f32x2 pair;               // the decode under way: two values, their scale, the first product
@@ -503,7 +504,6 @@ struct TallTile {
     __device__ __forceinline__ void run(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x_, const float* __restrict__ gs_ptr,
                                         float* __restrict__ y, int k_dim, int rows, int m_total, __bf16* xs2) {
         lane = lane_id();
-        x = x_;
         const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
         const int strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
         const int panels = (k_dim + CROW_PANEL_COLS - 1) / CROW_PANEL_COLS;
@@ -525,8 +525,9 @@ struct TallTile {
         // chunk c = i * 256 + thread: token row c / 32, 8 columns from 8 (c % 32)
         const int xq = ((int)threadIdx.x & 31) * 8;
         kd = (unsigned)k_dim;
-        xlast = (unsigned)(m_total - 1) * kd;
-        xrow = (unsigned)(m0 + ((int)threadIdx.x >> 5)) * kd;
+        x = x_ + (size_t)m0 * k_dim;
+        xlast = (unsigned)(m_total - m0 < MT ? m_total - m0 - 1 : MT - 1) * kd;
+        xrow = (threadIdx.x >> 5) * kd;
         auto next_panel = [&](int p, int buf) {  // the X tile that load_x and store_x move
             const int k = p * CROW_PANEL_COLS + xq;
             from = k < k_dim ? x : (const unsigned short*)gemm_zeros;
@@ -625,8 +626,8 @@ extern "C" __global__ void __launch_bounds__(256) gemm_nvfp4_bf16_m16(const unsi
                                                            const float* __restrict__ gs_ptr, float* __restrict__ y,            \
                                                            const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,    \
                                                            const int* __restrict__ m_p) {                                      \
-        /* 256 threads; X is addressed with 32-bit element offsets */                                                         \
-        if (block_threads() != 256 || *m_p < 1 || (unsigned long long)*m_p * (unsigned long long)*k_dim_p > 0xffffffffull) {   \
+        /* 256 threads; a block's rows of X are addressed with 32-bit element offsets */                                      \
+        if (block_threads() != 256 || *m_p < 1 || (unsigned)*k_dim_p >= 1u << 25) {                                            \
             if (threadIdx.x == 0) atomicOr(crow::g_ws.status, crow::STATUS_BAD_SHAPE);                                         \
             return;                                                                                                            \
         }                                                                                                                      \
@@ -659,8 +660,8 @@ CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w96, 6)
                                                          const float* __restrict__ gs_ptr, float* __restrict__ y,              \
                                                          const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,      \
                                                          const int* __restrict__ m_p) {                                        \
-        /* 256 threads; X is addressed with 32-bit element offsets */                                                         \
-        if (block_threads() != 256 || *m_p < 1 || (unsigned long long)*m_p * (unsigned long long)*k_dim_p > 0xffffffffull) {   \
+        /* 256 threads; a block's rows of X are addressed with 32-bit element offsets */                                      \
+        if (block_threads() != 256 || *m_p < 1 || (unsigned)*k_dim_p >= 1u << 25) {                                            \
             if (threadIdx.x == 0) atomicOr(crow::g_ws.status, crow::STATUS_BAD_SHAPE);                                         \
             return;                                                                                                            \
         }                                                                                                                      \

@@ -1116,6 +1116,19 @@ def test_launches_with_a_wrong_block_shape_are_refused(eng):
     eng.check()
 
 
+def test_gemm_tall_tiles_on_more_than_2_to_the_32_activations(eng):
+    """Token rows on both sides of element 2^32 of X equal the same rows on their own, bit for bit."""
+    rows, cols = 16, 17408
+    m = 2 ** 32 // cols + 200
+    f = _load(random_nvfp4(5, rows, cols), rows, cols, 6.0e-4)
+    x = torch.zeros((m, cols), dtype=torch.bfloat16, device="cuda")
+    x[-400:] = torch.from_numpy(normal_f32(13, rows, 400 * cols).reshape(400, cols)).cuda().to(torch.bfloat16)
+    got = eng.gemm(f, m, x, kernel="gemm_nvfp4_bf16_t128")
+    ref = eng.gemm(f, 400, x[-400:], kernel="gemm_nvfp4_bf16_t128")
+    eng.check()
+    assert ref.any(dim=1).all() and torch.equal(got[-400:], ref) and not got[:-400].any()
+
+
 def test_a_refused_routing_launch_leaves_no_pointers(eng):
     """The fused routing launch under a geometry it does not take (none set) writes zeros over whatever its pointer buffer held:
     the engine hands it uninitialised memory, and the down kernel behind it must not follow that."""
