@@ -396,19 +396,22 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
 // Measured on MI355X at K = 5120 over rows 1024..17408 and 17..2048 tokens: n blocks of m32 on one compute unit take
 // 5.8 + 10.7 n microseconds (within 10 %), a round of t64 / t96 / t128 60 / 72 / 86; at K = 1024 and 17408 all scale
 // alike.  So few row tiles stay with m32 far beyond 96 tokens ([1024, 5120] x 512: 19.7 us against 57 for t64 and 52 for the
-// best of the other tilings), and [17408, 5120] leaves it at about 128 ([.., 5120] x 512: t128 86 us, w80 104).  The remaining
-// entry points (m48 .. w96) are not the fastest anywhere in that range by more than 1 us; they stay callable by name.
+// best of the other tilings), and [17408, 5120] leaves it at about 96 ([.., 5120] x 512: t128 86 us, w80 104).  Between the two
+// stand blocks of 256 rows x 48 tokens while they fit one round: within 1 us of t64 at K = 5120 ([17408, 5120] x 128: m48 57.9 us,
+// m32 58.5, t64 57.1) and ahead at small K ([17408, 1024] x 144: 14.9 against 20.2 / 17.4; [8192, 2048] x 288: 22.7 against 26.9 /
+// 27.4); a second round adds 45.  The remaining entry points (m64 .. w96) are not the fastest anywhere in that range by more than 1 us; they stay
+// callable by name.
 const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) {
     if (m <= 16) return "gemm_nvfp4_bf16_m16";
     static const struct { const char* name; uint32_t mt, strips; double start, each; } cand[] = {
-        {"gemm_nvfp4_bf16_m32", 32, 4, 5.8, 10.7},  {"gemm_nvfp4_bf16_t64", 64, 20, 0.0, 60.0},
-        {"gemm_nvfp4_bf16_t96", 96, 20, 0.0, 72.0}, {"gemm_nvfp4_bf16_t128", 128, 20, 0.0, 86.0}};
+        {"gemm_nvfp4_bf16_m32", 32, 4, 5.8, 10.7},  {"gemm_nvfp4_bf16_m48", 48, 16, 12.0, 45.0},
+        {"gemm_nvfp4_bf16_t64", 64, 20, 0.0, 60.0}, {"gemm_nvfp4_bf16_t96", 96, 20, 0.0, 72.0}, {"gemm_nvfp4_bf16_t128", 128, 20, 0.0, 86.0}};
     const unsigned long long strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
     const unsigned long long cus = g.cus > 0 ? (unsigned long long)g.cus : 256ull;
     const char* best = nullptr;
     double best_t = 0.0;
     for (const auto& c : cand) {
-        if (c.mt == 32 && (m + 31ull) / 32 > 65535) continue;  // its token blocks are the grid's second dimension
+        if (c.mt < 64 && (m + c.mt - 1ull) / c.mt > 65535) continue;  // their token blocks are the grid's second dimension
         const unsigned long long blocks = ((strips + c.strips - 1) / c.strips) * ((m + c.mt - 1) / c.mt);
         const double t = c.start + c.each * (double)((blocks + cus - 1) / cus);
         if (best == nullptr || t < best_t) {

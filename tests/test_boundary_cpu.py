@@ -84,6 +84,7 @@ def test_gemm_kernel_choice_by_the_fullest_compute_unit():
     lib = L.lib()
     pick = lambda rows, m: lib.crow_hip_gemm_kernel(rows, m).decode()[len("gemm_nvfp4_bf16_"):]
     assert [pick(1024, m) for m in (17, 512, 1024)] == ["m32"] * 3
+    assert pick(17408, 96) == "m32" and [pick(17408, m) for m in (97, 128, 144)] == ["m48"] * 3  # one round of 256 x 48 blocks
     assert pick(5120, 1024) == "t64" and pick(2816, 2048) == "t96" and pick(17408, 512) == pick(5120, 1999) == "t128"
     assert pick(16, 32 * 65535) == "m32" and pick(16, 32 * 65535 + 1) != "m32"  # the end of a grid's second dimension
     for name, mt in (("t64", 64), ("t96", 96), ("t128", 128)):
