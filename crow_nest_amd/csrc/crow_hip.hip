@@ -394,13 +394,15 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
 // four waves (m32: two of them share a compute unit, short, but a decoded weight serves 32 tokens only) and blocks of 320 rows
 // whose waves each walk all of K (t64 / t96 / t128: one per compute unit, long, a decoded weight serves 64 to 128 tokens).
 // Measured on MI355X at K = 5120 over rows 1024..17408 and 17..2048 tokens: n blocks of m32 on one compute unit take
-// 5.8 + 10.7 n microseconds (within 10 %), a round of t64 / t96 / t128 60 / 72 / 86; at K = 1024 and 17408 all scale
-// alike.  So few row tiles stay with m32 far beyond 96 tokens ([1024, 5120] x 512: 19.7 us against 57 for t64 and 52 for the
+// 5.8 + 10.7 n microseconds (within 10 %), a round of t64 / t96 / t128 60 / 72 / 86; from K = 2048 on all scale
+// about alike.  So few row tiles stay with m32 far beyond 96 tokens ([1024, 5120] x 512: 19.7 us against 57 for t64 and 52 for the
 // best of the other tilings), and [17408, 5120] leaves it at about 96 ([.., 5120] x 512: t128 86 us, w80 104).  Between the two
 // stand blocks of 256 rows x 48 tokens while they fit one round: within 1 us of t64 at K = 5120 ([17408, 5120] x 128: m48 57.9 us,
 // m32 58.5, t64 57.1) and ahead at small K ([17408, 1024] x 144: 14.9 against 20.2 / 17.4; [8192, 2048] x 288: 22.7 against 26.9 /
-// 27.4); a second round adds 45.  The remaining entry points (m64 .. w96) are not the fastest anywhere in that range by more than 1 us; they stay
-// callable by name.
+// 27.4); a second round adds 45.  The remaining entry points (m64 .. w96) stay callable by name: at K = 2048 the choice is ahead
+// of the best of them at nearly every size (1.03 to 1.23 times; [17408, 2048] x 1999: w96 157 us, t128 160).  K is not an argument
+// here, and at K = 1024, where a long wave's start weighs more, the line lies up to 10 % off: [5120, 1024] x 300 m48 13.0, m32 14.4;
+// [17408, 1024] x 300 w48 21.5, t96 22.8; x 1999 w96 93.7, t128 100.2.
 const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) {
     if (m <= 16) return "gemm_nvfp4_bf16_m16";
     static const struct { const char* name; uint32_t mt, strips; double start, each; } cand[] = {
