@@ -626,8 +626,8 @@ extern "C" __global__ void __launch_bounds__(256) gemm_nvfp4_bf16_m16(const unsi
                                                            const float* __restrict__ gs_ptr, float* __restrict__ y,            \
                                                            const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,    \
                                                            const int* __restrict__ m_p) {                                      \
-        /* 256 threads; a block's rows of X are addressed with 32-bit element offsets */                                      \
-        if (block_threads() != 256 || *m_p < 1 || (unsigned)*k_dim_p >= 1u << 25) {                                            \
+        /* 256 threads; X is addressed with 32-bit element offsets */                                                         \
+        if (block_threads() != 256 || *m_p < 1 || (unsigned long long)*m_p * (unsigned long long)*k_dim_p > 0xffffffffull) {   \
             if (threadIdx.x == 0) atomicOr(crow::g_ws.status, crow::STATUS_BAD_SHAPE);                                         \
             return;                                                                                                            \
         }                                                                                                                      \

@@ -1129,6 +1129,29 @@ def test_gemm_tall_tiles_on_more_than_2_to_the_32_activations(eng):
     assert ref.any(dim=1).all() and torch.equal(got[-400:], ref) and not got[:-400].any()
 
 
+def test_gemm_entry_points_on_more_than_2_to_the_32_activations(eng):
+    """Every entry point that takes this many token rows, on both sides of element 2^32 of X: the rows' own results, or a
+    refusal that the status names - never other rows' results with a clean status."""
+    from crow_nest_amd.lib import CrowHipError
+    rows, cols = 16, 17408
+    m = 2 ** 32 // cols + 200
+    f = _load(random_nvfp4(5, rows, cols), rows, cols, 6.0e-4)
+    x = torch.zeros((m, cols), dtype=torch.bfloat16, device="cuda")
+    x[-400:] = torch.from_numpy(normal_f32(13, rows, 400 * cols).reshape(400, cols)).cuda().to(torch.bfloat16)
+    for name in ("m32", "m48", "m64", "m96", "", "w48", "w64", "w80", "w96", "t64", "t96", "t128"):
+        kernel = "gemm_nvfp4_bf16" + ("_" + name if name else "")
+        print(kernel, flush=True)
+        got = eng.gemm(f, m, x, kernel=kernel)
+        try:
+            eng.check()
+        except CrowHipError as e:
+            assert e.code == -7 and name[:1] != "t", kernel
+            continue
+        ref = eng.gemm(f, 400, x[-400:], kernel=kernel)
+        eng.check()
+        assert torch.equal(got[-400:], ref) and not got[:-400].any(), kernel
+
+
 def test_a_refused_routing_launch_leaves_no_pointers(eng):
     """The fused routing launch under a geometry it does not take (none set) writes zeros over whatever its pointer buffer held:
     the engine hands it uninitialised memory, and the down kernel behind it must not follow that."""
