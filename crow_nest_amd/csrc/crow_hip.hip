@@ -403,7 +403,10 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
 // of the best of them at nearly every size (1.03 to 1.23 times; [17408, 2048] x 1999: w96 157 us, t128 160).  K is not an argument
 // here, and at K = 1024, where a long wave's start weighs more, the line lies up to 10 % off: [5120, 1024] x 300 m48 13.0, m32 14.4;
 // [17408, 1024] x 300 w48 21.5, t96 22.8; x 1999 w96 93.7, t128 100.2.
-const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) {
+// An entry point that would refuse the product is left out: m32 / m48 address X with 32-bit element offsets from its start (m K up
+// to 2^32 - 1) and count token blocks in the grid's second dimension; the tall tiles count from a block's first token row (K < 2^25).
+// If none takes it, m32 is named, whose refusal the status reports.  k_dim = 0: K is not known, only rows and tokens decide.
+static const char* gemm_choice(uint32_t rows, uint32_t m, uint32_t k_dim) {
     if (m <= 16) return "gemm_nvfp4_bf16_m16";
     static const struct { const char* name; uint32_t mt, strips; double start, each; } cand[] = {
         {"gemm_nvfp4_bf16_m32", 32, 4, 5.8, 10.7},  {"gemm_nvfp4_bf16_m48", 48, 16, 12.0, 45.0},
@@ -413,16 +416,19 @@ const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) {
     const char* best = nullptr;
     double best_t = 0.0;
     for (const auto& c : cand) {
-        if (c.mt < 64 && (m + c.mt - 1ull) / c.mt > 65535) continue;  // their token blocks are the grid's second dimension
-        const unsigned long long blocks = ((strips + c.strips - 1) / c.strips) * ((m + c.mt - 1) / c.mt);
+        const unsigned long long token_blocks = (m + c.mt - 1ull) / c.mt, blocks = ((strips + c.strips - 1) / c.strips) * token_blocks;
+        const bool tall = c.name[16] == 't';
+        if (tall ? k_dim >= 1u << 25 || blocks > 0x7FFFFFFFull : token_blocks > 65535 || (unsigned long long)m * k_dim > 0xffffffffull) continue;
         const double t = c.start + c.each * (double)((blocks + cus - 1) / cus);
         if (best == nullptr || t < best_t) {
             best_t = t;
             best = c.name;
         }
     }
-    return best;
+    return best != nullptr ? best : cand[0].name;
 }
+const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) { return gemm_choice(rows, m, 0); }
+const char* crow_hip_gemm_kernel_for(uint32_t rows, uint32_t m, uint32_t k_dim) { return gemm_choice(rows, m, k_dim); }
 
 // Split of a [rows, k_dim] product over the chip.  A block owns one 16-row strip; the strip's 256-column groups are dealt
 // to W waves of the block (combined in LDS) and, only when a strip has more groups than one block's waves can hold, to S

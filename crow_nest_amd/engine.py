@@ -272,19 +272,19 @@ class Engine:
     # ------------------------------------------------------------------ prefill GEMM (M >= 16)
     def gemm(self, w: Fp4, m: int, x: torch.Tensor, y: torch.Tensor | None = None, kernel: str | None = None) -> torch.Tensor:
         """Y[m][rows] = X[m][cols] W^T on the matrix cores (bf16 X, exact bf16 weight tiles, f32 accumulate).
-        `kernel` forces one entry point (gemm_nvfp4_bf16_m16 takes m <= 16, the others any m); default: gemm_kernel_for(m, rows)."""
+        `kernel` forces one entry point (gemm_nvfp4_bf16_m16 takes m <= 16, the others any m); default: gemm_kernel_for(m, rows, cols)."""
         rows, k = w.rows, w.cols
         assert x.is_cuda and x.is_contiguous() and x.dtype == torch.bfloat16 and x.numel() == m * k
         if y is None:
             y = torch.empty((m, rows), dtype=torch.float32, device=self.dev)
-        name = kernel or gemm_kernel_for(m, rows)
+        name = kernel or gemm_kernel_for(m, rows, k)
         p = self.p
         self.k.run(name, rows, k, m, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m))
         return y
 
 
-def gemm_kernel_for(m: int, rows: int = 17408) -> str:
-    """Which GEMM entry point serves m token rows of a [rows, *] tensor: the library's choice (crow_hip_gemm_kernel), which
+def gemm_kernel_for(m: int, rows: int = 17408, k: int = 5120) -> str:
+    """Which GEMM entry point serves m token rows of a [rows, k] tensor: the library's choice (crow_hip_gemm_kernel_for), which
     weighs how the blocks of each tiling fall on the device's compute units."""
     from . import lib as _l
-    return _l.lib().crow_hip_gemm_kernel(rows, m).decode()
+    return _l.lib().crow_hip_gemm_kernel_for(rows, m, k).decode()

@@ -302,7 +302,7 @@ void Engine::f32_proj(uint64_t w_f32, int rows, int kd, int t, uint64_t x, uint6
     launch_v(k.f("gemv_b"), launch_dims("gemv_b", (uint32_t)rows, (uint32_t)kd, (uint32_t)t), {w_f32, x, y, p.i32(kd), p.i32(rows)});
 }
 void Engine::gemm(const Fp4& w, int m, uint64_t x_bf16, uint64_t y) {
-    const char* name = crow_hip_gemm_kernel((uint32_t)w.rows, (uint32_t)m);
+    const char* name = crow_hip_gemm_kernel_for((uint32_t)w.rows, (uint32_t)m, (uint32_t)w.cols);
     launch_v(k.f(name), launch_dims(name, (uint32_t)w.rows, (uint32_t)w.cols, (uint32_t)m), {w.w.ptr(), x_bf16, w.gs.ptr(), y, p.i32(w.cols), p.i32(w.rows), p.i32(m)});
 }
 

@@ -116,8 +116,11 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
  * made for a larger tensor make them read beyond the allocation. */
 #define CROW_DIMS_COUNT_FROM_MEMORY 0x80000000u
 int crow_hip_launch_dims(const char* name, uint32_t rows, uint32_t k_dim, uint32_t z, crow_dims* out);
-/* the GEMM entry point (a name of the kernel table) that serves `m` token rows fastest on a tensor of `rows` rows: the
- * choice depends on how the blocks of each tiling fall on this device's compute units */
+/* the GEMM entry point (a name of the kernel table) that serves `m` token rows fastest on a [rows, k_dim] tensor: the choice
+ * depends on how the blocks of each tiling fall on this device's compute units, and leaves out an entry point that would
+ * refuse the product (more than 2^32 - 1 activations, or k_dim of 2^25 and more, depending on the tiling) */
+const char* crow_hip_gemm_kernel_for(uint32_t rows, uint32_t m, uint32_t k_dim);
+/* the same without k_dim, as for k_dim around 5120: the entry point it names may refuse the product */
 const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m);
 /* reads and clears the device status word (waits for the whole device first: every stream): CROW_OK or CROW_ERR_* */
 int crow_hip_status(void);

@@ -95,14 +95,14 @@ CROW_KERNEL(moe_down_grouped, 9)
 /* ---- batched GEMM on the matrix cores (bf16 x, f32 y) ------------------------------------------------------------- */
 /* w, x, gs, y, k_dim_p, rows_p, m_p.  The dense NVFP4 GEMM of kernels_glm5_moe.cu:310-543 (gemm_fp4_dense's list minus
  * the quantised-activation buffer: x is bf16).  gemm_nvfp4_bf16_m16 serves *m_p <= 16 only; the others take any m
- * and differ in tiling (32, 48, 64, 96, 128 tokens per block); crow_hip_gemm_kernel names the one to use. */
+ * and differ in tiling (32, 48, 64, 96, 128 tokens per block); crow_hip_gemm_kernel_for names the one to use. */
 CROW_KERNEL(gemm_nvfp4_bf16, 7)
 /* the same product in blocks of eight waves (two per SIMD) x 48 / 64 / 80 / 96 tokens */
 CROW_KERNEL(gemm_nvfp4_bf16_w48, 7)
 CROW_KERNEL(gemm_nvfp4_bf16_w64, 7)
 CROW_KERNEL(gemm_nvfp4_bf16_w80, 7)
 CROW_KERNEL(gemm_nvfp4_bf16_w96, 7)
-/* ... and in blocks of four waves (one per SIMD), five 16-row strips each, x 64 / 96 / 128 tokens: what crow_hip_gemm_kernel
+/* ... and in blocks of four waves (one per SIMD), five 16-row strips each, x 64 / 96 / 128 tokens: what crow_hip_gemm_kernel_for
  * picks for large products */
 CROW_KERNEL(gemm_nvfp4_bf16_t64, 7)
 CROW_KERNEL(gemm_nvfp4_bf16_t96, 7)

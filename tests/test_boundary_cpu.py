@@ -94,6 +94,21 @@ def test_gemm_kernel_choice_by_the_fullest_compute_unit():
             assert (d.gx, d.gy, d.gz, d.bx) == (-(-rows // 320) * -(-m // mt), 1, 1, 256)
 
 
+def test_gemm_kernel_choice_names_an_entry_point_that_takes_the_product():
+    """Where any entry point does: the K-split and shared-X kernels count activations from the start of X in 32 bits and token
+    blocks in the grid's second dimension, the tall tiles count from a block's first token row (K < 2^25)."""
+    lib = L.lib()
+    for rows in (16, 64, 256, 1024, 17408, 151936):
+        for m in (17, 64, 128, 129, 12288, 246923, 839000, 32 * 65535 + 1, 1 << 22):
+            for k in (64, 1024, 5120, 17408, (1 << 32) // m // 64 * 64, ((1 << 32) // m // 64 + 1) * 64, (1 << 25) - 64, 1 << 25):
+                name = lib.crow_hip_gemm_kernel_for(rows, m, k).decode()[len("gemm_nvfp4_bf16_"):]
+                counted = m * k <= 0xFFFFFFFF
+                if name[0] == "t":
+                    assert k < 1 << 25, (rows, m, k, name)
+                elif counted or k < 1 << 25:  # (else none takes it, and the one named refuses)
+                    assert counted and -(-m // int(name[1:])) <= 65535, (rows, m, k, name)
+
+
 def test_native_launch_call_arguments():
     """The package's native launch call hands its integers to the library and returns the library's codes; what is not an
     integer, or too much, raises.  (Nothing is launched: the library is not initialised here.)"""

@@ -1129,6 +1129,21 @@ def test_gemm_tall_tiles_on_more_than_2_to_the_32_activations(eng):
     assert ref.any(dim=1).all() and torch.equal(got[-400:], ref) and not got[:-400].any()
 
 
+def test_gemm_choice_takes_more_than_2_to_the_32_activations(eng):
+    """The same product through the entry point that the library names for it: computed, not refused (the K-split kernel that
+    suits so few rows counts activations in 32 bits)."""
+    rows, cols = 16, 17408
+    m = 2 ** 32 // cols + 200
+    f = _load(random_nvfp4(5, rows, cols), rows, cols, 6.0e-4)
+    x = torch.zeros((m, cols), dtype=torch.bfloat16, device="cuda")
+    x[-400:] = torch.from_numpy(normal_f32(13, rows, 400 * cols).reshape(400, cols)).cuda().to(torch.bfloat16)
+    got = eng.dense_proj(f, m, x)
+    eng.check()
+    ref = eng.gemm(f, 400, x[-400:], kernel="gemm_nvfp4_bf16_t128")  # same order of sums: same bits
+    eng.check()
+    assert torch.equal(got[-400:], ref) and not got[:-400].any()
+
+
 def test_gemm_entry_points_on_more_than_2_to_the_32_activations(eng):
     """Every entry point that takes this many token rows, on both sides of element 2^32 of X: the rows' own results, or a
     refusal that the status names - never other rows' results with a clean status."""
