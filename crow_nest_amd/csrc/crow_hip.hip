@@ -389,37 +389,38 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
     return launch_entry(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream, g.ws_static);
 }
 
-// Which GEMM entry point for m token rows on a [rows, *] tensor.  Up to 16 rows: the K-split body over blocks.  Beyond that
-// the launch lasts as long as the fullest compute unit, and the choice is between blocks that deal one 64-row tile's K over
-// four waves (m32: two of them share a compute unit, short, but a decoded weight serves 32 tokens only) and blocks of 320 rows
-// whose waves each walk all of K (t64 / t96 / t128: one per compute unit, long, a decoded weight serves 64 to 128 tokens).
-// Measured on MI355X at K = 5120 over rows 1024..17408 and 17..2048 tokens: n blocks of m32 on one compute unit take
-// 5.8 + 10.7 n microseconds (within 10 %), a round of t64 / t96 / t128 60 / 72 / 86; from K = 2048 on all scale
-// about alike.  So few row tiles stay with m32 far beyond 96 tokens ([1024, 5120] x 512: 19.7 us against 57 for t64 and 52 for the
-// best of the other tilings), and [17408, 5120] leaves it at about 96 ([.., 5120] x 512: t128 86 us, w80 104).  Between the two
-// stand blocks of 256 rows x 48 tokens while they fit one round: within 1 us of t64 at K = 5120 ([17408, 5120] x 128: m48 57.9 us,
-// m32 58.5, t64 57.1) and ahead at small K ([17408, 1024] x 144: 14.9 against 20.2 / 17.4; [8192, 2048] x 288: 22.7 against 26.9 /
-// 27.4); a second round adds 45.  The remaining entry points (m64 .. w96) stay callable by name: at K = 2048 the choice is ahead
-// of the best of them at nearly every size (1.03 to 1.23 times; [17408, 2048] x 1999: w96 157 us, t128 160).  K is not an argument
-// here, and at K = 1024, where a long wave's start weighs more, the line lies up to 10 % off: [5120, 1024] x 300 m48 13.0, m32 14.4;
-// [17408, 1024] x 300 w48 21.5, t96 22.8; x 1999 w96 93.7, t128 100.2.
-// An entry point that would refuse the product is left out: m32 / m48 address X with 32-bit element offsets from its start (m K up
+// Which GEMM entry point for m token rows on a [rows, k_dim] tensor.  Up to 16 rows: the K-split body over blocks.  Beyond that the
+// launch lasts as long as the fullest compute unit, which takes `rounds` = ceil(blocks / compute units) blocks: one behind the other
+// where a block fills the unit (eight waves, or four that keep most registers), some of them together for m32 / m48 / m64.  Short
+// blocks that deal one 64-row tile's K over four waves (m32) win while there are few; large products go to the blocks whose
+// decoded weights serve the most tokens (t64 .. t128, 320 rows each), unless the last round is nearly empty with them and full with
+// others ([8192, 5120] x 1536: w96 has 256 blocks, one round, 114 us; t96 416, two, 140).
+//   us = rounds (a + b K / 1024) + blocks / compute units (c + d K / 1024) + (alone + alone_k K / 1024, one block on a unit)
+// was fitted to every entry point's time on MI355X at 1,122 sizes (rows 512 .. 17408, K 256 .. 17408, 17 .. 1999 tokens) and
+// names one within 3 % of the fastest at all but 9 of them (0.1 % on average); 96- and 128-token blocks of the shared-X body
+// (m96, the general name) are never ahead by more than that and are left to callers by name.
+// An entry point that would refuse the product is left out: those that address X with 32-bit element offsets from its start (m K up
 // to 2^32 - 1) and count token blocks in the grid's second dimension; the tall tiles count from a block's first token row (K < 2^25).
-// If none takes it, m32 is named, whose refusal the status reports.  k_dim = 0: K is not known, only rows and tokens decide.
-static const char* gemm_choice(uint32_t rows, uint32_t m, uint32_t k_dim) {
+// If none takes it, m32 is named, whose refusal the status reports.
+static const char* gemm_choice(uint32_t rows, uint32_t m, uint32_t k_dim, bool k_known) {
     if (m <= 16) return "gemm_nvfp4_bf16_m16";
-    static const struct { const char* name; uint32_t mt, strips; double start, each; } cand[] = {
-        {"gemm_nvfp4_bf16_m32", 32, 4, 5.8, 10.7},  {"gemm_nvfp4_bf16_m48", 48, 16, 12.0, 45.0},
-        {"gemm_nvfp4_bf16_t64", 64, 20, 0.0, 60.0}, {"gemm_nvfp4_bf16_t96", 96, 20, 0.0, 72.0}, {"gemm_nvfp4_bf16_t128", 128, 20, 0.0, 86.0}};
+    static const struct { const char* name; uint32_t mt, strips; double a, b, c, d, alone, alone_k; } cand[] = {
+        {"gemm_nvfp4_bf16_m32", 32, 4, 2.31, 1.46, 0.0, 0.44, 2.43, 0.48},    {"gemm_nvfp4_bf16_m48", 48, 16, 2.03, 6.56, 0.84, 1.81, 1.58, 2.46},
+        {"gemm_nvfp4_bf16_m64", 64, 16, 3.03, 5.5, 0.84, 4.96, 1.01, 4.51},   {"gemm_nvfp4_bf16_w48", 48, 32, 3.94, 12.93, 2.54, 1.31, 0.0, 0.0},
+        {"gemm_nvfp4_bf16_w64", 64, 32, 3.96, 15.51, 4.16, 1.61, 0.0, 0.0},   {"gemm_nvfp4_bf16_w80", 80, 32, 4.92, 16.17, 3.8, 2.45, 0.0, 0.0},
+        {"gemm_nvfp4_bf16_w96", 96, 32, 6.1, 17.18, 6.18, 3.24, 0.0, 0.0},    {"gemm_nvfp4_bf16_t64", 64, 20, 5.53, 10.69, 1.98, 0.0, 0.0, 0.0},
+        {"gemm_nvfp4_bf16_t96", 96, 20, 4.69, 12.31, 5.31, 0.0, 0.0, 0.0},    {"gemm_nvfp4_bf16_t128", 128, 20, 9.56, 12.71, 1.44, 1.72, 0.0, 0.0}};
     const unsigned long long strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
     const unsigned long long cus = g.cus > 0 ? (unsigned long long)g.cus : 256ull;
+    const double k = (double)k_dim / 1024.0;
     const char* best = nullptr;
     double best_t = 0.0;
     for (const auto& c : cand) {
         const unsigned long long token_blocks = (m + c.mt - 1ull) / c.mt, blocks = ((strips + c.strips - 1) / c.strips) * token_blocks;
         const bool tall = c.name[16] == 't';
-        if (tall ? k_dim >= 1u << 25 || blocks > 0x7FFFFFFFull : token_blocks > 65535 || (unsigned long long)m * k_dim > 0xffffffffull) continue;
-        const double t = c.start + c.each * (double)((blocks + cus - 1) / cus);
+        if (tall ? k_dim >= 1u << 25 || blocks > 0x7FFFFFFFull : token_blocks > 65535 || (k_known && (unsigned long long)m * k_dim > 0xffffffffull)) continue;
+        const unsigned long long rounds = (blocks + cus - 1) / cus;
+        const double t = (double)rounds * (c.a + c.b * k) + (double)blocks / (double)cus * (c.c + c.d * k) + (rounds == 1 ? c.alone + c.alone_k * k : 0.0);
         if (best == nullptr || t < best_t) {
             best_t = t;
             best = c.name;
@@ -427,8 +428,8 @@ static const char* gemm_choice(uint32_t rows, uint32_t m, uint32_t k_dim) {
     }
     return best != nullptr ? best : cand[0].name;
 }
-const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) { return gemm_choice(rows, m, 0); }
-const char* crow_hip_gemm_kernel_for(uint32_t rows, uint32_t m, uint32_t k_dim) { return gemm_choice(rows, m, k_dim); }
+const char* crow_hip_gemm_kernel(uint32_t rows, uint32_t m) { return gemm_choice(rows, m, 5120, false); }
+const char* crow_hip_gemm_kernel_for(uint32_t rows, uint32_t m, uint32_t k_dim) { return gemm_choice(rows, m, k_dim, true); }
 
 // Split of a [rows, k_dim] product over the chip.  A block owns one 16-row strip; the strip's 256-column groups are dealt
 // to W waves of the block (combined in LDS) and, only when a strip has more groups than one block's waves can hold, to S
