@@ -243,13 +243,11 @@ class Params:
 
     def __init__(self):
         self._dev = _device()
-        self._cache: dict[int, torch.Tensor] = {}
-        self._ptr: dict[int, int] = {}
+        self._words: dict[int, tuple[int, torch.Tensor]] = {}  # address and the tensor that keeps it, as one value: the words live as long as this object
 
     def i32(self, v: int) -> int:
-        ptr = self._ptr.get(v)
-        if ptr is None:
+        word = self._words.get(v)
+        if word is None:
             t = torch.tensor([v], dtype=torch.int32, device=self._dev)
-            self._cache[v] = t  # kept: the words live as long as this object
-            ptr = self._ptr[v] = t.data_ptr()
-        return ptr
+            word = self._words.setdefault(v, (t.data_ptr(), t))  # another thread's, if it was first
+        return word[0]

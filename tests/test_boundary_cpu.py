@@ -119,6 +119,27 @@ def test_gemm_kernel_choice_knows_k(rows, m, k, want):
     assert name in ((want,) if isinstance(want, str) else want)
 
 
+def test_a_shape_word_made_by_two_threads_at_once_is_one_word(monkeypatch):
+    """A second thread asks for the same value while the first is making its word: both get the same address, of a tensor that
+    the object keeps - never one that nothing holds any more."""
+    import weakref
+    import torch
+    from crow_nest_amd import weights as W
+    monkeypatch.setattr(W, "_device", lambda: torch.device("cpu"))
+    p, made, other, make = W.Params(), [], [], torch.tensor
+
+    def tensor(*a, **k):
+        t = make(*a, **k)
+        made.append((t.data_ptr(), weakref.ref(t)))
+        if len(made) == 1:
+            other.append(p.i32(7))  # what the second thread does meanwhile
+        return t
+
+    monkeypatch.setattr(torch, "tensor", tensor)
+    assert p.i32(7) == other[0] == p.i32(7) and len(made) == 2
+    assert [ref() is not None for ptr, ref in made if ptr == other[0]] == [True]
+
+
 def test_native_launch_call_arguments():
     """The package's native launch call hands its integers to the library and returns the library's codes; what is not an
     integer, or too much, raises.  (Nothing is launched: the library is not initialised here.)"""
