@@ -510,11 +510,13 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
             // [6151, 3008] 5.9 -> 4.8 (three rows 8.9 -> 7.0), [1024, 5120] 5.4 -> 5.0 (three rows 10.1 -> 8.6), 64 rows 52.5 -> 47.2 at
             // [4096, 5120].  Eight would win again up to four rows (4.3) and lose from sixteen on (60 against 47); at 1088 strips and 8
             // groups four waves lose (one row 8.1 against 7.1, five 13.6 against 12.3).  Up to seven groups a wave walks the strip
-            // alone, here and in the grouped expert kernels.
+            // alone, here and in the grouped expert kernels.  The routed kernels keep the long walks: their launch is that many strips
+            // per combo or tile, which fills the chip (gemv_fp4_ptrb [4096, 2048] x 512 combos 250 us, 332 with four waves, x 32 21 / 26;
+            // moe_down_grouped [2048, 2560] x 64 tiles 52 / 61).
             // (The split depends on the tensor's shape only, never on the number of tokens or experts in the launch: a token's
-            // bits are the same in every batch, and the grouped expert kernels reproduce them.  Four waves per tensor at
+            // bits are the same in every batch, and the grouped expert kernels reproduce the per-combo ones'.  Four waves per tensor at
             // batch 1 would take routed gate|up [1024, 2048] x 8 experts from 8.0 to 7.2 us and give that up.)
-            if (e->nr == 1 && strips <= 512 && groups > 7 && w < 4) w = 4;
+            if (e->nr == 1 && !routed && strips <= 512 && groups > 7 && w < 4) w = 4;
         } else {
             w = 4;
             s = (groups + 13) / 14;

@@ -183,6 +183,17 @@ def test_launch_dims_depend_on_the_matrix_only():
     assert lib.crow_hip_launch_dims(b"gemv_nvfp4_w", 8, 96, 1, C.byref(d1)) == -7  # 96 columns: not whole blocks
 
 
+@pytest.mark.parametrize("rows,cols", [(512, 2048), (4096, 2560), (8192, 3584), (2048, 5120)])
+def test_routed_launches_keep_long_walks(rows, cols):
+    """One wave per seven groups of a strip: a routed launch has a strip per combo or tile and needs no more waves."""
+    import ctypes as C
+    d = L.Dims()
+    for name in (b"gemv_fp4_ptrb", b"moe_down_grouped"):
+        assert L.lib().crow_hip_launch_dims(name, rows, cols, 64, C.byref(d)) == 0
+        assert d.bx == 64 * -(-cols // (7 * 256)), name
+    assert L.lib().crow_hip_launch_dims(b"gemv_nvfp4_w", rows, cols, 1, C.byref(d)) == 0 and d.bx == 64 * 4
+
+
 def test_matrix_shapes_are_checked_like_the_reference():
     b = np.zeros(Nvfp4Matrix.byte_len(3, 128), np.uint8)
     Nvfp4Matrix.new(b, 3, 128, 1.0)
