@@ -31,10 +31,12 @@ struct FnEntry {
     const void* tile_stub;
     bool takes_geo;  // the launcher appends the model geometry (crow_hip_set_geo) by value, last
     const void* one_stub = nullptr;  // a twin of `stub` with one strip per block, started in its place when S = CROW_ONE_STRIP
+    const void* two_stub = nullptr;  // ... and one with two runs of columns per wave, when S = CROW_TWO_RUNS
 };
-// value of S in a launch's `gy` word (GEMV family, K up to 16384): one slice, and one strip per block where the kernel otherwise
-// takes `ns` of them.  A strip of at most 64 groups never has that many slices.
+// values of S in a launch's `gy` word (GEMV family, K up to 16384; a strip of at most 64 groups never has that many slices): one
+// slice, and one strip per block where the kernel otherwise takes `ns` of them / two runs of columns per wave of the block
 #define CROW_ONE_STRIP 0x81u
+#define CROW_TWO_RUNS 0x82u
 
 // The launcher builds a kernel's argument array from the fields of its table entry: the caller's `nargs` values, then the
 // geometry word (GEMV family), the scratch descriptor (takes_ws), the model geometry (takes_geo).  A kernel that gains a
@@ -62,6 +64,9 @@ constexpr int checked_nargs(F) {
 // ... with a twin for one strip per block
 #define CROW_GEMV_ONE(name, nargs, NR, MMAX) \
     {#name, (const void*)&name, checked_nargs<nargs, 2>(&name) + 0 * checked_nargs<nargs, 2>(&name##_one), 0u, NR, 8, crow::crow_gemv_lds_per_wave(MMAX, false), CROW_MULTI_STRIPS, true, nullptr, false, (const void*)&name##_one}
+// ... for two runs per wave
+#define CROW_GEMV_TWO(name, nargs, twin) \
+    {#name, (const void*)&name, checked_nargs<nargs, 2>(&name) + 0 * checked_nargs<nargs, 2>(&twin), 0u, 1, 8, crow::crow_gemv_lds_per_wave(4, false), CROW_MULTI_STRIPS, true, nullptr, false, nullptr, (const void*)&twin}
 #define CROW_GEMV_GEO(name, nargs, NR, MMAX, XBF16) \
     {#name, (const void*)&name, checked_nargs<nargs, 3>(&name), 0u, NR, 16, crow::crow_gemv_lds_per_wave(MMAX, XBF16), 1, true, nullptr, true}
 const FnEntry g_table[] = {
@@ -69,7 +74,7 @@ const FnEntry g_table[] = {
     CROW_GEMV(gemv_nvfp4_gu, 8, 2, 1, false),      CROW_GEMV(gemv_nvfp4_gu_bf16, 8, 2, 1, true),
     CROW_GEMV_ONE(gemv_nvfp4_wm, 7, 1, 4),         CROW_GEMV_ONE(gemv_nvfp4_gum, 9, 2, 4),
     CROW_GEMV(gemv_nvfp4_wm_bf16, 7, 1, 4, true),  CROW_GEMV(gemv_nvfp4_gum_bf16, 9, 2, 4, true), CROW_GEMV(gemv_fp4, 6, 1, 1, false),
-    CROW_GEMV(gemv_fp4_b, 7, 1, 4, false),         CROW_GEMV(gemv_fp4_b1k, 7, 1, 4, false),      CROW_GEMV(gemv_fp4_bs, 8, 1, 4, false),
+    CROW_GEMV_TWO(gemv_fp4_b, 7, gemv_fp4_b_two),  CROW_GEMV_TWO(gemv_fp4_b1k, 7, gemv_fp4_b_two), CROW_GEMV_TWO(gemv_fp4_bs, 8, gemv_fp4_bs_two),
     CROW_GEMV(gemv_fp4_ptrb, 8, 1, 1, false),      CROW_GEMV(moe_gate_up_silu, 8, 2, 1, false),  CROW_GEMV_GEO(moe_down_combine, 7, 1, 1, false),
     CROW_GEMV_GEO(moe_route_gate_up_silu, 11, 2, 1, false),
     {"moe_gate_up_silu_grouped", (const void*)&moe_gate_up_silu_grouped, checked_nargs<11, 2>(&moe_gate_up_silu_grouped) + 0 * checked_nargs<11, 2>(&moe_gate_up_silu_grouped_tile), 0u, 2, 8, crow::crow_gemv_lds_per_wave(4, false), CROW_MULTI_STRIPS, true, (const void*)&moe_gate_up_silu_grouped_tile, false},
@@ -185,8 +190,10 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
             lds = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)tile_groups(e->nr, (unsigned)pairs) * (size_t)(e->lds_per_wave / 2);
         } else {
             const bool one = e->one_stub != nullptr && (word >> 24) == CROW_ONE_STRIP && pairs <= 64 * CROW_GROUP_PAIRS;
-            const int slices = one || (word >> 24) == 0 ? 1 : (int)(word >> 24);
+            const bool two = e->two_stub != nullptr && (word >> 24) == CROW_TWO_RUNS && pairs <= 64 * CROW_GROUP_PAIRS;
+            const int slices = one || two || (word >> 24) == 0 ? 1 : (int)(word >> 24);
             if (one) stub = e->one_stub;
+            if (two) stub = e->two_stub;
             lds = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)waves * (size_t)e->lds_per_wave;
             // a split launch must fit the scratch memory it is given (the kernels check again and report through the status word)
             if (slices > 1 && ((unsigned long long)grid.x * grid.z * (unsigned)slices * (unsigned)(e->nr * (one ? 1 : e->ns)) * 64ull > ws.partial_floats ||
@@ -265,9 +272,10 @@ int crow_hip_init(int device) {
         if (most > 48 * 1024 &&
             (e = hipFuncSetAttribute(g_table[i].stub, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most)) != hipSuccess)
             return fail(e);
-        if (g_table[i].one_stub != nullptr && most > 48 * 1024 &&
-            (e = hipFuncSetAttribute(g_table[i].one_stub, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most)) != hipSuccess)
-            return fail(e);
+        for (const void* twin : {g_table[i].one_stub, g_table[i].two_stub})
+            if (twin != nullptr && most > 48 * 1024 &&
+                (e = hipFuncSetAttribute(twin, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most)) != hipSuccess)
+                return fail(e);
         // the twin for short strips stages up to eight groups of twelve rows per block
         const size_t tile_most = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)CROW_TILE_MAX_GROUPS * (size_t)(g_table[i].lds_per_wave / 2);
         if (g_table[i].tile_stub != nullptr && tile_most > 48 * 1024 &&
@@ -509,7 +517,7 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
             // 512 to 17408 rows, K = 1024..5120 and 1 to 64 rows of activations (us, one row unless said): [512, 2048] 3.7 -> 3.3,
             // [6151, 3008] 5.9 -> 4.8 (three rows 8.9 -> 7.0), [1024, 5120] 5.4 -> 5.0 (three rows 10.1 -> 8.6), 64 rows 52.5 -> 47.2 at
             // [4096, 5120].  Eight would win again up to four rows (4.3) and lose from sixteen on (60 against 47); at 1088 strips and 8
-            // groups four waves lose (one row 8.1 against 7.1, five 13.6 against 12.3).  Up to seven groups a wave walks the strip
+            // groups four waves lose (one row 8.1 against 7.1, five 13.6 against 12.3; see also CROW_TWO_RUNS below).  Up to seven groups a wave walks the strip
             // alone, here and in the grouped expert kernels.  The routed kernels keep the long walks: their launch is that many strips
             // per combo or tile, which fills the chip (gemv_fp4_ptrb [4096, 2048] x 512 combos 250 us, 332 with four waves, x 32 21 / 26;
             // moe_down_grouped [2048, 2560] x 64 tiles 52 / 61).
@@ -535,9 +543,16 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         // up to two blocks a unit where a strip is short, one strip per block is faster (three rows, us, two / one strips per block:
         // [2048, 5120] 8.6 / 7.4, [4096, 5120] 8.7 / 8.3, [8192, 2048] 6.0 / 5.5, [6151, 3008] 7.0 / 6.7; [5120, 5120] 8.8 / 10.1,
         // [12288, 3072] 9.2 / 9.6; gate|up [4096, 5120] 13.3 / 11.3, [5120, 2048] 10.8 / 11.1).  Same bits.
+        // Four waves on a strip of up to 14 groups walk two to four groups each.  Many token groups fill the chip with such short walks:
+        // there two waves take the four runs between them (blocks of more than three per compute unit; us, four waves / two waves with
+        // two runs / two waves with a run each, which are other bits: [8192, 2560] x 257 208 / 169 / 170, [4096, 2048] x 257 75 / 66 / 66,
+        // [4096, 3072] x 32 16.3 / 14.4 / 14.1; below the line, [2048, 3072] x 32, 9.6 / 13.7 / 13.3).
+        const bool two = e->two_stub != nullptr && s == 1 && w == 4 && groups > 7 && groups <= 14 && force_w == 0 && force_s == 0 &&
+                         (unsigned long long)((strips + 1) / 2) * gz > 768;
+        if (two) w = 2;
         const bool one = e->one_stub != nullptr && s == 1 && (strips <= 256 || (e->nr == 1 && strips <= 512 && groups <= 12));
         const uint32_t ns = one ? 1u : (uint32_t)e->ns, gx = (strips + ns - 1) / ns;
-        *out = crow_dims{gx, pairs | (hint << 20) | ((one ? CROW_ONE_STRIP : s) << 24), gz, 64u * w * (uint32_t)e->nr};
+        *out = crow_dims{gx, pairs | (hint << 20) | ((one ? CROW_ONE_STRIP : (two ? CROW_TWO_RUNS : s)) << 24), gz, 64u * w * (uint32_t)e->nr};
         if (s > 1 && ((unsigned long long)gx * gz * s * (unsigned)(e->nr * ns) * 64 > PARTIAL_FLOATS || (unsigned long long)gx * gz > COUNTER_SLOTS)) return CROW_ERR_WORKSPACE;
         return CROW_OK;
     }

@@ -569,7 +569,10 @@ struct StripWalkPairs {
 // activation row the operation sequence is StripWalk's, so the sums are the same bits.
 //   wl[s]   the lane's view of the wave's first group of strip s (a strip beyond the tensor: any strip that exists; its
 //           sums are never stored)
-template <int M, bool XBF16, int NS>
+// RUNS = 2: the wave walks the groups of two runs in one go: `cut` groups, then - `jump` groups further on - the second run's.
+// Between them the first run's sums move to `head` and the second run starts from zero, so each run's operations, and its bits,
+// are those of a wave of its own.
+template <int M, bool XBF16, int NS, int RUNS = 1>
 struct MultiWalk {
     typedef Staging<M, XBF16> St;
     static constexpr int NSET = XBF16 ? 1 : (3 * M + 3) / 4;
@@ -582,12 +585,14 @@ struct MultiWalk {
     const unsigned char* wl[NS];
     const unsigned char* xl;
     size_t xoff[M];
-    int col_lane, k_dim, lane;
-    float acc[NS][M];
+    int col_lane, k_dim, lane, cut, jump;
+    float acc[NS][M], head[NS][M];
 
-    __device__ __forceinline__ void init(const unsigned char* const (&strip)[NS], int first, int k_dim_, const void* x, const size_t (&xoff_elems)[M],
-                                         lds_p xw_, lds_p zero) {
+    __device__ __forceinline__ void init(const unsigned char* const (&strip)[NS], int first, int cut_, int jump_, int k_dim_, const void* x,
+                                         const size_t (&xoff_elems)[M], lds_p xw_, lds_p zero) {
         lane = lane_id();
+        cut = cut_;
+        jump = jump_;
         xw = xw_;
         k_dim = k_dim_;
 #pragma unroll
@@ -598,7 +603,7 @@ struct MultiWalk {
         for (int m = 0; m < M; m++) {
             xoff[m] = xoff_elems[m] * (XBF16 ? 2 : 4);
 #pragma unroll
-            for (int s = 0; s < NS; s++) acc[s][m] = 0.0f;
+            for (int s = 0; s < NS; s++) acc[s][m] = head[s][m] = 0.0f;
         }
         const int g = lane >> 4, i = lane & 15, r4 = i & 3;
         const bool half_ok = (g >> 1) == (i >> 3);
@@ -614,9 +619,11 @@ struct MultiWalk {
                 a2[sl][q] = (live && second) ? data + 64 : zero + 16 * g;
             }
     }
+    // group g of the wave's walk, counted from the first run's first group
+    __device__ __forceinline__ int at(int g) const { return RUNS == 2 && g >= cut ? g + jump : g; }
     template <int J>
     __device__ __forceinline__ void issue_x(int g) {
-        const int col = col_lane + g * CROW_GROUP_COLS;
+        const int col = col_lane + at(g) * CROW_GROUP_COLS;
         const size_t o = (size_t)(col < k_dim ? col : k_dim - 4) * (XBF16 ? 2 : 4);
 #pragma unroll
         for (int t = 0; t < M; t++) xv[J][t] = *(const __attribute__((address_space(1))) XV*)(xl + xoff[t] + o);
@@ -625,7 +632,7 @@ struct MultiWalk {
     __device__ __forceinline__ void issue_w(int g) {
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            const unsigned char* p = wl[s] + (size_t)g * CROW_GROUP_BYTES;
+            const unsigned char* p = wl[s] + (size_t)at(g) * CROW_GROUP_BYTES;
             sc[J][s] = stream_load_u32((const unsigned*)p + lane);
             cd[J][s][0] = stream_load_v((const uint4*)(p + CROW_GROUP_SCALE_BYTES) + lane);
             cd[J][s][1] = stream_load_v((const uint4*)(p + CROW_GROUP_SCALE_BYTES + 1024) + lane);
@@ -633,7 +640,7 @@ struct MultiWalk {
     }
     template <int J>
     __device__ __forceinline__ void stage(int g) {
-        const bool in = col_lane + g * CROW_GROUP_COLS < k_dim;
+        const bool in = col_lane + at(g) * CROW_GROUP_COLS < k_dim;
         lds_p slot = xw + J * St::SLOT + 8 * lane;
 #pragma unroll
         for (int t = 0; t < M; t++) {
@@ -654,10 +661,20 @@ struct MultiWalk {
         __builtin_amdgcn_wave_barrier();
     }
     template <int J>
-    __device__ __forceinline__ void multiply() {
+    __device__ __forceinline__ void multiply(int g) {
         group_multiply<M, XBF16, NS>(sc[J], cd[J], a1[J], a2[J], acc);
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (RUNS == 2) {  // (selects: a branch here costs 0.1 us per group)
+            const bool end = g + 1 == cut;
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+                    head[s][m] = end ? acc[s][m] : head[s][m];
+                    acc[s][m] = end ? 0.0f : acc[s][m];
+                }
+        }
     }
     // On entry: the weights of groups g0, g0 + 1 are in (or on their way to) slots 0, 1; group g0 is staged; the activations of
     // g0 + 1 and g0 + 2 are in (or on their way to) x slots 1 and 0.  Requests for groups beyond the wave's run read columns
@@ -666,13 +683,13 @@ struct MultiWalk {
     __device__ __forceinline__ void duo(int g0) {
         stage<1>(g0 + 1);
         issue_x<1>(g0 + 3);
-        multiply<0>();
+        multiply<0>(g0);
         if (REFILL) {
             issue_w<0>(g0 + 2);
             stage<0>(g0 + 2);
             issue_x<0>(g0 + 4);
         }
-        multiply<1>();
+        multiply<1>(g0 + 1);
         if (REFILL) issue_w<1>(g0 + 3);
     }
     // (one copy of each body, and no branch whose two sides begin alike: see StripWalk::go)
@@ -694,25 +711,26 @@ struct MultiWalk {
                 issue_x<0>(even);
                 issue_w<0>(even);
                 stage<0>(even);
-                multiply<0>();
+                multiply<0>(even);
             }
         } else if (count == 1) {
             issue_x<0>(0);
             issue_w<0>(0);
             mid();
             stage<0>(0);
-            multiply<0>();
+            multiply<0>(0);
         } else {
             mid();
         }
     }
+    // (two runs: the first one's sums end in lanes 0..31, the second one's in lanes 32..63)
     __device__ __forceinline__ void finish(float (&out)[NS][M]) const {
 #pragma unroll
         for (int s = 0; s < NS; s++)
 #pragma unroll
             for (int m = 0; m < M; m++) {
                 const unsigned a = __float_as_uint(acc[s][m]);
-                const u32x2 sw = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+                const u32x2 sw = __builtin_amdgcn_permlane32_swap(RUNS == 2 ? __float_as_uint(head[s][m]) : a, a, false, false);
                 const unsigned b = __float_as_uint(__fadd_rn(__uint_as_float(sw.x), __uint_as_float(sw.y)));
                 const u32x2 sq = __builtin_amdgcn_permlane16_swap(b, b, false, false);
                 out[s][m] = __fadd_rn(__uint_as_float(sq.x), __uint_as_float(sq.y));
@@ -940,11 +958,13 @@ typedef __attribute__((address_space(3))) float* lds_f;
 // sized by the launcher for M_ALLOC rows: entry points that dispatch over M size it for their widest body.
 // NS = strips per block: 1 for the one-row kernels (StripWalk); the kernels for several activation rows take NS adjacent strips
 // per block, every wave all NS of them over its run of columns (MultiWalk), blockIdx.x = strip / NS.
-template <int NR, int M, bool XBF16, int EPI, int M_ALLOC = M, int NS = 1>
+// RUNS = runs of columns per wave (one tensor, NS > 1): with 2, half the waves make the same runs' sums.
+template <int NR, int M, bool XBF16, int EPI, int M_ALLOC = M, int NS = 1, int RUNS = 1>
 __device__ __forceinline__ void gemv_body(const GemvArgs& a, unsigned z, lds_p lds, const Workspace& ws) {
     static_assert(M <= M_ALLOC, "the allocation covers this body");
     constexpr int AREA = crow_gemv_lds_per_wave(M_ALLOC, XBF16);
-    static_assert(NS * M * 64 <= AREA, "a wave's sums fit its staging area");
+    static_assert(RUNS * NS * M * 64 <= AREA, "a wave's sums fit its staging area");
+    static_assert(RUNS == 1 || (RUNS == 2 && NR == 1 && NS > 1), "two runs per wave: MultiWalk, one tensor");
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = block_threads() >> 6;  // wave-uniform on purpose
     CROW_STAMP(0);
@@ -954,13 +974,16 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, unsigned z, lds_p l
     const int groups = (a.pairs + CROW_GROUP_PAIRS - 1) / CROW_GROUP_PAIRS;
     const int wpt = NR == 2 ? waves >> 1 : waves;            // waves per tensor
     const int r_own = (NR == 2 && wave >= wpt) ? 1 : 0;      // wave-uniform
-    const int unit = slice * wpt + (wave - r_own * wpt), units = slices * wpt;
+    const int unit = slice * wpt + (wave - r_own * wpt), units = slices * wpt * RUNS;  // (two runs per wave: `unit` and the one `half` on)
     // the strip's groups in runs of floor(groups / units), the first groups % units runs one longer
     const int base = groups / units, rem = groups - base * units;
     // (a two-tensor block launched with an odd number of waves has one wave too many: it takes nothing, and the launch is
     // refused at the store - not here, where the refusal would sit between a wave's start and its first weight load)
     const bool extra_wave = NR == 2 && wave - r_own * wpt >= wpt;
-    const int count = extra_wave ? 0 : base + (unit < rem ? 1 : 0), first = unit * base + (unit < rem ? unit : rem);
+    const int half = slices * wpt, second = unit + half;
+    const int first_run = base + (unit < rem ? 1 : 0), first = unit * base + (unit < rem ? unit : rem);
+    const int count = extra_wave ? 0 : first_run + (RUNS == 2 ? base + (second < rem ? 1 : 0) : 0);
+    const int jump = second * base + (second < rem ? second : rem) - first - first_run;  // from behind the first run to the second
     const unsigned char* wsel = r_own != 0 ? a.w[1] : a.w[0];  // a select, never an indexed read
     // element offsets of this launch's activation rows, and which output row each of them writes
     size_t xoff[M];
@@ -1002,28 +1025,48 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, unsigned z, lds_p l
         const unsigned char* sp[NS];
 #pragma unroll
         for (int s = 0; s < NS; s++) sp[s] = wsel + (size_t)(strip + (s < have ? s : 0)) * groups * CROW_GROUP_BYTES;
-        MultiWalk<M, XBF16, NS> walk;
-        walk.init(sp, first, k_dim, a.x, xoff, areas + wave * AREA, zero);
+        MultiWalk<M, XBF16, NS, RUNS> walk;
+        walk.init(sp, first, first_run, jump, k_dim, a.x, xoff, areas + wave * AREA, zero);
         walk.go(count, mid);
         walk.finish(part);
     }
 
-    // waves of the block -> wave 0: lane l of wave 0 takes output (m = l / 16, n = l % 16) of every strip and adds the waves'
-    // sums in wave order
+    // waves of the block -> wave 0: lane l of wave 0 takes output (m = l / 16, n = l % 16) of every strip and adds the runs'
+    // sums in order
     float v[NR * NS];
 #pragma unroll
     for (int r = 0; r < NR * NS; r++) v[r] = 0.0f;
     const int mo = lane >> 4, n = lane & 15;
-    if (waves > 1) {
-        if (lane < 16) {
+    if (waves * RUNS > 1) {
+        if (RUNS == 2 ? (lane & 16) == 0 : lane < 16) {  // (lane 32 + i: the second run's sum)
+            const int at = RUNS == 2 ? (lane >> 5) * NS * M * 16 + n : lane;
 #pragma unroll
             for (int s = 0; s < NS; s++)
 #pragma unroll
-                for (int m = 0; m < M; m++) ((lds_f)(areas + wave * AREA))[(s * M + m) * 16 + lane] = part[s][m];
+                for (int m = 0; m < M; m++) ((lds_f)(areas + wave * AREA))[(s * M + m) * 16 + at] = part[s][m];
         }
         __syncthreads();
         if (wave > 0) return;
-        if (mo < M) {
+        if (RUNS == 2) {  // the waves' first runs, then their second ones; two of these sums on their way at a time
+            if (mo < M) {
+#pragma unroll
+                for (int q = 0; q < RUNS; q++)
+                    for (int w = 0; w < wpt; w += 2) {
+                        float t[2][NS];
+#pragma unroll
+                        for (int i = 0; i < 2; i++)
+#pragma unroll
+                            for (int s = 0; s < NS; s++) t[i][s] = ((lds_f)(areas + (w + i < wpt ? w + i : w) * AREA))[(q * NS + s) * M * 16 + lane];
+#pragma unroll
+                        for (int i = 0; i < 2; i++)
+#pragma unroll
+                            for (int s = 0; s < NS; s++) {
+                                if (q + w + i == 0) v[s] = t[i][s];
+                                else if (w + i < wpt) v[s] += t[i][s];
+                            }
+                    }
+            }
+        } else if (mo < M) {
 #pragma unroll
             for (int r = 0; r < NR; r++)
 #pragma unroll

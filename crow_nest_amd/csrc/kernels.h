@@ -116,7 +116,7 @@ extern "C" __global__ void __launch_bounds__(1024) gemv_nvfp4_gu_bf16(const unsi
 #ifndef CROW_MULTI_STRIPS_BF16
 #define CROW_MULTI_STRIPS_BF16 1
 #endif
-template <int NR, bool XBF16, int EPI, int NS = CROW_MULTI_STRIPS>
+template <int NR, bool XBF16, int EPI, int NS = CROW_MULTI_STRIPS, int RUNS = 1>
 __device__ __forceinline__ void gemv_m_dispatch(const GemvArgs& a, int m, unsigned z, lds_p lds, const Workspace& ws) {
     if (m < 1 || m > 4) {  // the reference's NVFP4_MMAX (engine/src/kernels_p2.rs:397-400); uniform over the launch
         if (threadIdx.x == 0) atomicOr(ws.status, STATUS_BAD_SHAPE);
@@ -124,10 +124,10 @@ __device__ __forceinline__ void gemv_m_dispatch(const GemvArgs& a, int m, unsign
     }
     // one body per M keeps each row's operation sequence identical to the one-row kernel
     switch (m) {
-        case 1: gemv_body<NR, 1, XBF16, EPI, 4, NS>(a, z, lds, ws); break;
-        case 2: gemv_body<NR, 2, XBF16, EPI, 4, NS>(a, z, lds, ws); break;
-        case 3: gemv_body<NR, 3, XBF16, EPI, 4, NS>(a, z, lds, ws); break;
-        default: gemv_body<NR, 4, XBF16, EPI, 4, NS>(a, z, lds, ws); break;
+        case 1: gemv_body<NR, 1, XBF16, EPI, 4, NS, RUNS>(a, z, lds, ws); break;
+        case 2: gemv_body<NR, 2, XBF16, EPI, 4, NS, RUNS>(a, z, lds, ws); break;
+        case 3: gemv_body<NR, 3, XBF16, EPI, 4, NS, RUNS>(a, z, lds, ws); break;
+        default: gemv_body<NR, 4, XBF16, EPI, 4, NS, RUNS>(a, z, lds, ws); break;
     }
 }
 // The activation row count of a verify launch: from the geometry word when the launcher put it there (then the word behind
@@ -208,6 +208,7 @@ extern "C" __global__ void __launch_bounds__(512) gemv_nvfp4_gum_bf16(const unsi
 // :1022-1058.  grid.z = ceil(T / 4): each block decodes its weights once for up to 4 token rows.
 // (gemv_fp4_b1k is the reference's 1024-thread variant of gemv_fp4_b for tensors of few rows; here the block shape follows
 // K alone, so both names run the same body.)
+template <int RUNS = 1>
 __device__ __forceinline__ void gemv_tokens(const unsigned char* w, const float* x, const float* gs, float* y, int geo, const int* k_dim_p,
                                             const int* rows_p, const int* t_p, size_t y_stride, const Workspace& ws) {
     const int pairs = geo & 0xFFFFF, hint = (geo >> 20) & 0xF;
@@ -225,7 +226,7 @@ __device__ __forceinline__ void gemv_tokens(const unsigned char* w, const float*
         if (t0 >= t_total) return;
         m = t_total - t0 < 4 ? t_total - t0 : 4;
     }
-    gemv_m_dispatch<1, false, EPI_SCALE>(a, m, blockIdx.z, LDS, ws);
+    gemv_m_dispatch<1, false, EPI_SCALE, CROW_MULTI_STRIPS, RUNS>(a, m, blockIdx.z, LDS, ws);
 }
 extern "C" __global__ void __launch_bounds__(512) gemv_fp4_b(const unsigned char* __restrict__ w, const float* __restrict__ x,
                                                               const float* __restrict__ gs_ptr, float* __restrict__ y,
@@ -252,6 +253,27 @@ extern "C" __global__ void __launch_bounds__(512) gemv_fp4_bs(const unsigned cha
         return;
     }
     gemv_tokens(w, x, gs_ptr, y, geo, k_dim_p, rows_p, t_p, (size_t)y_stride, ws);
+}
+// The three kernels above with two runs of columns per wave, which the launcher starts in their place when the launch dimensions
+// say so (crow_hip_launch_dims: many token groups of a tensor of few strips).  Same bits: the runs are the same.
+extern "C" __global__ void __launch_bounds__(512) gemv_fp4_b_two(const unsigned char* __restrict__ w, const float* __restrict__ x,
+                                                                  const float* __restrict__ gs_ptr, float* __restrict__ y,
+                                                                  const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
+                                                                  const int* __restrict__ t_p, int geo, const Workspace ws) {
+    ENTER(w, x, gs_ptr, y, k_dim_p, rows_p, t_p, geo);
+    gemv_tokens<2>(w, x, gs_ptr, y, geo, k_dim_p, rows_p, t_p, 0, ws);
+}
+extern "C" __global__ void __launch_bounds__(512) gemv_fp4_bs_two(const unsigned char* __restrict__ w, const float* __restrict__ x,
+                                                                   const float* __restrict__ gs_ptr, float* __restrict__ y,
+                                                                   const int* __restrict__ k_dim_p, const int* __restrict__ y_stride_p,
+                                                                   const int* __restrict__ rows_p, const int* __restrict__ t_p, int geo, const Workspace ws) {
+    ENTER(w, x, gs_ptr, y, k_dim_p, y_stride_p, rows_p, t_p, geo);
+    const int y_stride = *y_stride_p;
+    if (y_stride < *rows_p) {  // as gemv_fp4_bs
+        if (threadIdx.x == 0) atomicOr(ws.status, STATUS_BAD_SHAPE);
+        return;
+    }
+    gemv_tokens<2>(w, x, gs_ptr, y, geo, k_dim_p, rows_p, t_p, (size_t)y_stride, ws);
 }
 
 // ------------------------------------------------------------------ routed experts

@@ -48,7 +48,7 @@ enum crow_status {
 /* launch geometry chosen by the library for a kernel and a problem (wave64 shapes stay out of the caller).  The four words
  * are to be handed to crow_hip_launch unchanged.  For the NVFP4 GEMV family `gy` is not a grid extent: it carries the problem
  * (bits 0..19 = k_dim / 64, bits 20..23 = activation rows of the last token group or 0, bits 24..31 = column slices per
- * strip, or 0x81: one slice and one strip per block); crow_hip_launch launches (gx, slices, gz) blocks and hands the low 24 bits to the kernel by value, so that a wave
+ * strip, or 0x81 / 0x82: one slice, and one strip per block / two runs of columns per wave); crow_hip_launch launches (gx, slices, gz) blocks and hands the low 24 bits to the kernel by value, so that a wave
  * can address its weights before the words behind k_dim_p / m_p have arrived from memory. */
 typedef struct crow_dims {
     uint32_t gx, gy, gz, bx;

@@ -434,6 +434,39 @@ def test_verify_rows_keep_the_decode_rows_bits_under_every_split(eng, rows, cols
         assert rel_err(ref[0].cpu().numpy(), orc.gemv(random_nvfp4(rows, rows, cols), rows, cols, 1.1e-3, x[0].cpu().numpy())[0], floor_of(rows)) <= TOL
 
 
+# many token groups of a tensor of few strips: two waves take four runs between them (partial last groups of columns, an odd number
+# of strips, last token groups of one to four rows)
+@pytest.mark.parametrize("rows,cols,t", [(8161, 1856, 13), (250, 2048, 401), (8192, 2560, 16), (2049, 3520, 51), (8177, 3584, 14)])
+def test_token_rows_keep_the_decode_rows_bits_with_two_runs_per_wave(eng, rows, cols, t):
+    from crow_nest_amd.kernels import COUNT_FROM_MEMORY, launch_dims, launch_v
+    w = random_nvfp4(rows, rows, cols)
+    f = _load(w, rows, cols, 1.1e-3)
+    xs = normal_f32(9, rows, t * cols).reshape(t, cols)
+    x, p = _dev(xs), eng.p
+
+    def run(dims, name="gemv_fp4_b", stride=rows):
+        y = torch.full((t, stride), float("nan"), device="cuda")
+        words = [p.i32(cols)] + ([p.i32(stride)] if name == "gemv_fp4_bs" else []) + [p.i32(rows), p.i32(t)]
+        launch_v(eng.k.f(name), *dims, [f.w_ptr, x.data_ptr(), f.gs_ptr, y.data_ptr()] + words)
+        eng.check()
+        assert torch.isnan(y[:, rows:]).all()
+        return y[:, :rows].contiguous()
+
+    d = launch_dims("gemv_fp4_b", rows, cols, t)
+    assert d[1] >> 24 == 0x82 and d[3] == 128
+    four = launch_dims("gemv_fp4_b", rows, cols, t, split=(1, 4))
+    assert four[1] >> 24 == 1 and four[3] == 256
+    ref = run(four)
+    assert torch.equal(run(d), ref)
+    assert torch.equal(run(launch_dims("gemv_fp4_b1k", rows, cols, t), "gemv_fp4_b1k"), ref)
+    assert torch.equal(run(launch_dims("gemv_fp4_bs", rows, cols, t), "gemv_fp4_bs", rows + 5), ref)
+    assert torch.equal(run(launch_dims("gemv_fp4_b", rows, cols, COUNT_FROM_MEMORY | (t + 9))), ref)
+    for i in (0, t - 1):
+        assert torch.equal(eng.dense_proj(f, 1, x[i:i + 1])[0], ref[i])
+    n = min(rows, 300)
+    assert rel_err(ref[-1, :n].cpu().numpy(), orc.gemv(w[:n * cols // 64 * 36], n, cols, 1.1e-3, xs[-1])[0], floor_of(n)) <= TOL
+
+
 # ---------------------------------------------------------------- head
 
 def test_lm_head_logits_and_greedy_token(eng):
