@@ -524,7 +524,10 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
             // (The split depends on the tensor's shape only, never on the number of tokens or experts in the launch: a token's
             // bits are the same in every batch, and the grouped expert kernels reproduce the per-combo ones'.  Four waves per tensor at
             // batch 1 would take routed gate|up [1024, 2048] x 8 experts from 8.0 to 7.2 us and give that up.)
-            if (e->nr == 1 && !routed && strips <= 512 && groups > 7 && w < 4) w = 4;
+            // bf16 activations cost a wave less, so from 17 groups on three waves keep the chip as busy beyond 256 strips ([8192, 5376]
+            // three rows 6.9 us, 7.3 with four waves, one row 6.2 / 6.4; [6144, 4608] three rows 6.2 / 6.4).
+            const bool long_bf16 = strstr(name, "_bf16") != nullptr && groups > 16 && strips > 256;
+            if (e->nr == 1 && !routed && !long_bf16 && strips <= 512 && groups > 7 && w < 4) w = 4;
         } else {
             w = 4;
             s = (groups + 13) / 14;

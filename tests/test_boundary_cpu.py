@@ -194,6 +194,15 @@ def test_routed_launches_keep_long_walks(rows, cols):
     assert L.lib().crow_hip_launch_dims(b"gemv_nvfp4_w", rows, cols, 1, C.byref(d)) == 0 and d.bx == 64 * 4
 
 
+def test_bf16_rows_keep_three_waves_on_long_strips():
+    """Decode row and verify rows alike (they share the order of the sums)."""
+    import ctypes as C
+    d = L.Dims()
+    for rows, cols, waves in ((8192, 4608, 3), (4112, 5376, 3), (4096, 5376, 4), (8192, 4096, 4), (8208, 4096, 3), (512, 5376, 4)):
+        for name, m in ((b"gemv_nvfp4_w_bf16", 1), (b"gemv_nvfp4_wm_bf16", 3)):
+            assert L.lib().crow_hip_launch_dims(name, rows, cols, m, C.byref(d)) == 0 and d.bx == 64 * waves, (name, rows, cols)
+
+
 def test_matrix_shapes_are_checked_like_the_reference():
     b = np.zeros(Nvfp4Matrix.byte_len(3, 128), np.uint8)
     Nvfp4Matrix.new(b, 3, 128, 1.0)
