@@ -32,11 +32,13 @@ struct FnEntry {
     bool takes_geo;  // the launcher appends the model geometry (crow_hip_set_geo) by value, last
     const void* one_stub = nullptr;  // a twin of `stub` with one strip per block, started in its place when S = CROW_ONE_STRIP
     const void* two_stub = nullptr;  // ... and one with two runs of columns per wave, when S = CROW_TWO_RUNS
+    const void* ahead_stub = nullptr;  // unquantised GEMVs: a twin that requests weights alone ahead, when the launch's gz = CROW_KEEP_AHEAD
 };
 // values of S in a launch's `gy` word (GEMV family, K up to 16384; a strip of at most 64 groups never has that many slices): one
 // slice, and one strip per block where the kernel otherwise takes `ns` of them / two runs of columns per wave of the block
 #define CROW_ONE_STRIP 0x81u
 #define CROW_TWO_RUNS 0x82u
+#define CROW_KEEP_AHEAD 2u  // (the grid of those kernels has no third dimension)
 
 // The launcher builds a kernel's argument array from the fields of its table entry: the caller's `nargs` values, then the
 // geometry word (GEMV family), the scratch descriptor (takes_ws), the model geometry (takes_geo).  A kernel that gains a
@@ -56,6 +58,8 @@ constexpr int checked_nargs(F) {
     return NARGS;
 }
 #define CROW_FN(name, nargs) {#name, (const void*)&name, checked_nargs<nargs, 0>(&name), 0u, 0, 16, 0, 1, false, nullptr, false}
+#define CROW_FN_KEEP(name, nargs, twin) \
+    {#name, (const void*)&name, checked_nargs<nargs, 0>(&name) + 0 * checked_nargs<nargs, 0>(&twin), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, (const void*)&twin}
 #define CROW_FN_GEO(name, nargs) {#name, (const void*)&name, checked_nargs<nargs, 1>(&name), 0u, 0, 16, 0, 1, false, nullptr, true}
 // NR tensors per block, bodies for 1 .. MMAX activation rows, bf16 or f32 activations
 // (the bodies for several rows need more registers than a block of sixteen waves leaves each: they run in blocks of eight)
@@ -95,8 +99,9 @@ const FnEntry g_table[] = {
     {"gemm_nvfp4_bf16_t64", (const void*)&gemm_nvfp4_bf16_t64, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t64), 2u * 64u * 528u, 0, 4, 0, 1, false},
     {"gemm_nvfp4_bf16_t96", (const void*)&gemm_nvfp4_bf16_t96, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t96), 2u * 96u * 528u, 0, 4, 0, 1, false},
     {"gemm_nvfp4_bf16_t128", (const void*)&gemm_nvfp4_bf16_t128, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t128), 2u * 128u * 528u, 0, 4, 0, 1, false},
-    CROW_FN(gemm_nvfp4_bf16_m32, 7), CROW_FN(gemm_nvfp4_bf16_m16, 7), CROW_FN(gemv_bf16_w, 5),
-    CROW_FN(gemv_bf16, 5), CROW_FN(gemv_bf16_b, 5), CROW_FN(gemv_b, 5), CROW_FN(gemv_bf16_ws, 5), CROW_FN(gemv_bf16_bs, 6),
+    CROW_FN(gemm_nvfp4_bf16_m32, 7), CROW_FN(gemm_nvfp4_bf16_m16, 7), CROW_FN_KEEP(gemv_bf16_w, 5, gemv_bf16_ahead),
+    CROW_FN_KEEP(gemv_bf16, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_bf16_b, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_b, 5, gemv_b_ahead),
+    CROW_FN_KEEP(gemv_bf16_ws, 5, gemv_bf16_ws_ahead), CROW_FN_KEEP(gemv_bf16_bs, 6, gemv_bf16_bs_ahead),
     CROW_FN(gemv_nvfp4_w_valu1, 6), CROW_FN(gemv_nvfp4_w_valu2, 6), CROW_FN(gemv_nvfp4_w_valu4, 6),  // measurement only
 };
 const int g_table_n = (int)(sizeof(g_table) / sizeof(g_table[0]));
@@ -204,6 +209,10 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
         }
         if (lds > g.lds_cap) return CROW_ERR_SHAPE;
         args[na++] = (void*)&geo;
+    }
+    if (e->ahead_stub != nullptr && grid.z == CROW_KEEP_AHEAD) {
+        stub = e->ahead_stub;
+        grid.z = 1;
     }
     if (e->takes_ws) args[na++] = (void*)&ws_arg;
     crow::Geo model_arg = g.model;
@@ -469,11 +478,14 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         if (k_dim == 0 || k_dim % (strcmp(name, "gemv_b") == 0 ? 4 : 8) != 0) return CROW_ERR_SHAPE;
         if (strcmp(name, "gemv_bf16") == 0 && z != 1) return CROW_ERR_SHAPE;  // the one-token form
         // short tensors: a block of four waves per (row, token); force_w = 4 / 1 asks for one shape or the other
-        if (force_w == 4 || (force_w == 0 && (unsigned long long)rows * z <= 2048)) {
-            *out = crow_dims{rows, z, 1, 256};
-            return CROW_OK;
-        }
-        *out = crow_dims{(rows + 3) / 4, z, 1, 256};
+        const bool f32 = strcmp(name, "gemv_b") == 0, block_per_row = force_w == 4 || (force_w == 0 && (unsigned long long)rows * z <= 2048);
+        // Several rows against weights that the 256 MB memory-side cache cannot hold from one row to the next, and long bf16 rows in
+        // more than three blocks per compute unit, are bound by memory: weights alone ahead (us, so / weights and activations together,
+        // f32 [20000, 5120] x 4 231 / 258, [10240, 8192] x 2 103 / 109; bf16 [40000, 5120] x 2 141 / 150, [2048, 8192] x 1 8.5 / 9.0;
+        // up to 256 MB together is ahead by up to 1.4 times: bf16 [10240, 8192] x 16 356 / 290)
+        const bool ahead = (z > 1 && (unsigned long long)rows * k_dim * (f32 ? 4 : 2) > (256ull << 20)) ||
+                           (!f32 && block_per_row && k_dim >= 4096 && (unsigned long long)rows * z > 768);
+        *out = crow_dims{block_per_row ? rows : (rows + 3) / 4, z, ahead ? CROW_KEEP_AHEAD : 1u, 256};
         return CROW_OK;
     }
     if (e->nr != 0) {  // the NVFP4 GEMV family

@@ -769,7 +769,9 @@ extern "C" __global__ void __launch_bounds__(1024) argmax_finish(int* __restrict
 //   gemv_b        engine/src/kernels.rs:97-115   (f32 weights, the router projection of gen.rs:4182; + rows_p; k_dim % 4 == 0)
 //   gemv_bf16_ws  engine/src/kernels.rs:1430-1458 (gemv_bf16_w with y = 1 / (1 + expf(-sum)) at the store)
 //   gemv_bf16_bs  engine/src/kernels.rs:1100-1124 (gemv_bf16_b with an explicit y row stride; + rows_p)
-template <bool WBF16, bool SIGMOID = false>
+// AHEAD: where the memory is the bound, the weights of four steps alone are requested ahead, non-temporal, and each step's
+// activations behind them (`.._ahead`, started in a kernel's place when the launch dimensions say so: crow_hip_launch_dims).  Same bits.
+template <bool WBF16, bool SIGMOID = false, bool AHEAD = false>
 __device__ __forceinline__ void keep_gemv_body(const void* __restrict__ w, const float* __restrict__ x, float* __restrict__ y, int k, int rows,
                                                size_t y_stride) {
     constexpr int PER = WBF16 ? 8 : 4;  // weights per 16-byte load
@@ -801,45 +803,65 @@ __device__ __forceinline__ void keep_gemv_body(const void* __restrict__ w, const
         }
     };
     int i0 = (part * 64 + lane) * PER;
-    // four steps at a time, weights and activations requested together: one round trip a trip, not two.  With several
-    // activation rows in the launch the weights are read again (from the die's L2): plain loads
-    const bool reread = gridDim.y > 1;  // uniform
-    for (; i0 + 3 * run < k; i0 += 4 * run) {
-        uint4 v[4];
-        float4 a[4], b[4];
+    if constexpr (AHEAD) {
+        for (; i0 < k; i0 += 4 * run) {
+            uint4 v[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = i0 + j * run;
-            a[j] = *(const float4*)(xp + i);
-            b[j] = WBF16 ? *(const float4*)(xp + i + 4) : a[j];
-        }
-        if (reread) {
+            for (int j = 0; j < 4; j++) {
+                const int i = i0 + j * run;
+                v[j] = make_uint4(0, 0, 0, 0);
+                if (i < k) v[j] = stream_load((const uint4*)(wp + (size_t)i * (WBF16 ? 2 : 4)));
+            }
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = *(const uint4*)(wp + (size_t)(i0 + j * run) * (WBF16 ? 2 : 4));
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = stream_load((const uint4*)(wp + (size_t)(i0 + j * run) * (WBF16 ? 2 : 4)));
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) add(v[j], a[j], b[j]);
-    }
-    if (i0 < k) {  // up to three steps more, requested together as well
-        uint4 v[3];
-        float4 a[3], b[3];
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const int i = i0 + j * run;
-            v[j] = make_uint4(0, 0, 0, 0);
-            a[j] = b[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (i < k) {
-                v[j] = stream_load((const uint4*)(wp + (size_t)i * (WBF16 ? 2 : 4)));
-                a[j] = *(const float4*)(xp + i);
-                if (WBF16) b[j] = *(const float4*)(xp + i + 4);
+            for (int j = 0; j < 4; j++) {
+                const int i = i0 + j * run;
+                if (i < k) {
+                    const float4 a = *(const float4*)(xp + i);
+                    add(v[j], a, WBF16 ? *(const float4*)(xp + i + 4) : a);
+                }
             }
         }
+    } else {
+        // four steps at a time, weights and activations requested together: one round trip a trip, not two.  With several
+        // activation rows in the launch the weights are read again, from the caches: plain loads (in a last, partial trip non-temporal ones)
+        const bool reread = gridDim.y > 1;  // uniform
+        for (; i0 + 3 * run < k; i0 += 4 * run) {
+            uint4 v[4];
+            float4 a[4], b[4];
 #pragma unroll
-        for (int j = 0; j < 3; j++)
-            if (i0 + j * run < k) add(v[j], a[j], b[j]);
+            for (int j = 0; j < 4; j++) {
+                const int i = i0 + j * run;
+                a[j] = *(const float4*)(xp + i);
+                b[j] = WBF16 ? *(const float4*)(xp + i + 4) : a[j];
+            }
+            if (reread) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = *(const uint4*)(wp + (size_t)(i0 + j * run) * (WBF16 ? 2 : 4));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = stream_load((const uint4*)(wp + (size_t)(i0 + j * run) * (WBF16 ? 2 : 4)));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) add(v[j], a[j], b[j]);
+        }
+        if (i0 < k) {  // up to three steps more, requested together as well
+            uint4 v[3];
+            float4 a[3], b[3];
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const int i = i0 + j * run;
+                v[j] = make_uint4(0, 0, 0, 0);
+                a[j] = b[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (i < k) {
+                    v[j] = stream_load((const uint4*)(wp + (size_t)i * (WBF16 ? 2 : 4)));
+                    a[j] = *(const float4*)(xp + i);
+                    if (WBF16) b[j] = *(const float4*)(xp + i + 4);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                if (i0 + j * run < k) add(v[j], a[j], b[j]);
+        }
     }
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
     auto finish = [](float v) { return SIGMOID ? 1.0f / (1.0f + expf(-v)) : v; };
@@ -851,37 +873,45 @@ __device__ __forceinline__ void keep_gemv_body(const void* __restrict__ w, const
     __syncthreads();
     if (threadIdx.x == 0) y[(size_t)t * y_stride + row] = finish(((wave_sum[0] + wave_sum[1]) + wave_sum[2]) + wave_sum[3]);
 }
-#define CROW_KEEP_GEMV(NAME, WT, WBF16)                                                                                              \
+#define CROW_KEEP_GEMV(NAME, WT, WBF16, AHEAD)                                                                                              \
     extern "C" __global__ void __launch_bounds__(256) NAME(const WT* __restrict__ w, const float* __restrict__ x, float* __restrict__ y, \
                                                            const int* __restrict__ k_dim_p, const int* __restrict__ rows_p) {        \
         if (block_threads() != 256) {                                                                                                \
             if (threadIdx.x == 0) atomicOr(g_ws.status, STATUS_BAD_SHAPE);                                                           \
             return;                                                                                                                  \
         }                                                                                                                            \
-        keep_gemv_body<WBF16>(w, x, y, *k_dim_p, *rows_p, (size_t)*rows_p);                                                          \
+        keep_gemv_body<WBF16, false, AHEAD>(w, x, y, *k_dim_p, *rows_p, (size_t)*rows_p);                                            \
     }
-CROW_KEEP_GEMV(gemv_bf16_w, unsigned short, true)
-CROW_KEEP_GEMV(gemv_bf16, unsigned short, true)
-CROW_KEEP_GEMV(gemv_bf16_b, unsigned short, true)
-CROW_KEEP_GEMV(gemv_b, float, false)
+CROW_KEEP_GEMV(gemv_bf16_w, unsigned short, true, false)
+CROW_KEEP_GEMV(gemv_bf16, unsigned short, true, false)
+CROW_KEEP_GEMV(gemv_bf16_b, unsigned short, true, false)
+CROW_KEEP_GEMV(gemv_b, float, false, false)
+CROW_KEEP_GEMV(gemv_bf16_ahead, unsigned short, true, true)
+CROW_KEEP_GEMV(gemv_b_ahead, float, false, true)
 
-extern "C" __global__ void __launch_bounds__(256) gemv_bf16_ws(const unsigned short* __restrict__ w, const float* __restrict__ x, float* __restrict__ y,
-                                                               const int* __restrict__ k_dim_p, const int* __restrict__ rows_p) {
-    if (block_threads() != 256) {
-        if (threadIdx.x == 0) atomicOr(g_ws.status, STATUS_BAD_SHAPE);
-        return;
+#define CROW_KEEP_GEMV_WS(NAME, AHEAD)                                                                                                          \
+    extern "C" __global__ void __launch_bounds__(256) NAME(const unsigned short* __restrict__ w, const float* __restrict__ x,                   \
+                                                           float* __restrict__ y, const int* __restrict__ k_dim_p, const int* __restrict__ rows_p) { \
+        if (block_threads() != 256) {                                                                                                           \
+            if (threadIdx.x == 0) atomicOr(g_ws.status, STATUS_BAD_SHAPE);                                                                      \
+            return;                                                                                                                             \
+        }                                                                                                                                       \
+        keep_gemv_body<true, true, AHEAD>(w, x, y, *k_dim_p, *rows_p, (size_t)*rows_p);                                                         \
     }
-    keep_gemv_body<true, true>(w, x, y, *k_dim_p, *rows_p, (size_t)*rows_p);
-}
-extern "C" __global__ void __launch_bounds__(256) gemv_bf16_bs(const unsigned short* __restrict__ w, const float* __restrict__ x, float* __restrict__ y,
-                                                               const int* __restrict__ k_dim_p, const int* __restrict__ y_stride_p,
-                                                               const int* __restrict__ rows_p) {
-    if (block_threads() != 256 || *y_stride_p < *rows_p) {
-        if (threadIdx.x == 0) atomicOr(g_ws.status, STATUS_BAD_SHAPE);
-        return;
+CROW_KEEP_GEMV_WS(gemv_bf16_ws, false)
+CROW_KEEP_GEMV_WS(gemv_bf16_ws_ahead, true)
+#define CROW_KEEP_GEMV_BS(NAME, AHEAD)                                                                                                          \
+    extern "C" __global__ void __launch_bounds__(256) NAME(const unsigned short* __restrict__ w, const float* __restrict__ x,                   \
+                                                           float* __restrict__ y, const int* __restrict__ k_dim_p,                              \
+                                                           const int* __restrict__ y_stride_p, const int* __restrict__ rows_p) {                \
+        if (block_threads() != 256 || *y_stride_p < *rows_p) {                                                                                  \
+            if (threadIdx.x == 0) atomicOr(g_ws.status, STATUS_BAD_SHAPE);                                                                      \
+            return;                                                                                                                             \
+        }                                                                                                                                       \
+        keep_gemv_body<true, false, AHEAD>(w, x, y, *k_dim_p, *rows_p, (size_t)*y_stride_p);                                                    \
     }
-    keep_gemv_body<true>(w, x, y, *k_dim_p, *rows_p, (size_t)*y_stride_p);
-}
+CROW_KEEP_GEMV_BS(gemv_bf16_bs, false)
+CROW_KEEP_GEMV_BS(gemv_bf16_bs_ahead, true)
 
 // ------------------------------------------------------------------ measurement only: the one-row GEMV without matrix instructions
 // The reference's own shape for this product (kernels_p2.rs:304-368: a warp per few rows, lanes across the columns, f32

@@ -1392,6 +1392,33 @@ def test_f32_keep_gemv_router_projection(eng, rows, cols, t):
     assert np.array_equal(eng.f32_proj(wd, t, xd).cpu().numpy(), eng._keep_proj("gemv_b", wd, t, xd, None, 0).cpu().numpy())
 
 
+# beyond what the memory-side cache holds from one row to the next, and long bf16 rows a block each: the kernels that request weights alone ahead
+@pytest.mark.parametrize("name,rows,cols,t", [("gemv_b", 13108, 5124, 2), ("gemv_bf16_w", 16385, 8200, 3), ("gemv_bf16", 801, 4104, 1),
+                                              ("gemv_bf16_b", 401, 8192, 2), ("gemv_bf16_ws", 1000, 6152, 2), ("gemv_bf16_bs", 999, 4104, 2)])
+def test_unquantised_gemvs_with_weights_ahead_keep_the_bits(eng, name, rows, cols, t):
+    from crow_nest_amd.kernels import launch_dims, launch_v
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    w = torch.empty((rows, cols), device="cuda", dtype=torch.float32 if name == "gemv_b" else torch.bfloat16).normal_(0.0, 0.05, generator=gen)
+    x = torch.empty((t, cols), device="cuda").normal_(generator=gen)
+    p, out = eng.p, []
+    gx, gy, gz, bx = launch_dims(name, rows, cols, t)
+    assert gz == 2
+    for z in (2, 1):
+        y = torch.full((t, rows + 3), float("nan"), device="cuda")
+        words = [p.i32(cols)] + ([p.i32(rows + 3)] if name == "gemv_bf16_bs" else []) + [p.i32(rows)]
+        launch_v(eng.k.f(name), gx, gy, z, bx, [w.data_ptr(), x.data_ptr(), y.data_ptr()] + words)
+        eng.check()
+        out.append(y if name == "gemv_bf16_bs" else y.view(-1)[:t * rows].view(t, rows))
+    assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
+    n = min(rows, 500)
+    ref = x.double() @ w[-n:].double().T  # (to the f32 bound of the kept summation order: gamma of cols + 6 additions)
+    got = out[0][:, :rows][:, -n:].double()
+    bound = orc.gamma(16 * (cols + 6)) * (x.double().abs() @ w[-n:].double().abs().T)
+    if name == "gemv_bf16_ws":  # the sigmoid's slope is at most a quarter; 2e-7: expf in the last place
+        ref, bound = torch.sigmoid(ref), bound / 4 + 2e-7
+    assert ((got - ref).abs() <= bound).all()
+
+
 # ---------------------------------------------------------------- the ABI from plain C
 
 def test_c_abi_from_a_plain_c_program():
