@@ -279,13 +279,15 @@ extern "C" __global__ void __launch_bounds__(256) quantize_nvfp4_amax(const floa
     }
 }
 // pass 2: one thread per sub-block: its scale byte and its sixteen codes; thread 0 also leaves the global scale.  The blocks run
-// from the end of the tensor to its start: what pass 1 read last is still in the memory-side cache.
+// from the end of the tensor to its start, what pass 1 read last is still in the memory-side cache; by eights, so that a block reads
+// what pass 1 read on its own die (block % 8) and small tensors come out of that die's L2 ([1000, 5120]: 5.7 us, 7.0 when reversed singly).
 extern "C" __global__ void __launch_bounds__(256) quantize_nvfp4_encode(const float* __restrict__ values, unsigned long long n_sub,
                                                                          const unsigned* __restrict__ max_bits, unsigned char* __restrict__ blocks,
                                                                          float* __restrict__ global_out) {
     const float max_scale = __fdiv_rn(__uint_as_float(*max_bits), 6.0f);  // the largest raw scale (see pass 1)
     const float global = max_scale > 0.0f ? __fdiv_rn(max_scale, 448.0f) : 1.0f;
-    const unsigned long long i = (unsigned long long)(gridDim.x - 1 - blockIdx.x) * blockDim.x + threadIdx.x;
+    const unsigned eights = gridDim.x >> 3, b = blockIdx.x, at = b < 8 * eights ? 8 * (eights - 1 - (b >> 3)) + (b & 7) : b;
+    const unsigned long long i = (unsigned long long)at * blockDim.x + threadIdx.x;
     if (i == 0) global_out[0] = global;
     if (i >= n_sub) return;
     const float4* p = (const float4*)(values + 16 * i);
