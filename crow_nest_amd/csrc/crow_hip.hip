@@ -900,12 +900,13 @@ static int layout_launch(const char* name, const void* a, const void* b, const v
     vals[n++] = (uint64_t)(sc + 1);
     rc = launch_entry(find(name), dim3(d.gx, d.gy, d.gz), dim3(d.bx), vals, n, g.stream, g.ws);
     if (rc != CROW_OK) return rc;
-    // both status words come back in pinned memory behind the kernel, so that one wait for the device is all the host does; what
-    // they say when one is raised is crow_hip_status's to report (a bit raised meanwhile on another stream stays for the next call)
+    // every stream idle, as in crow_hip_status; then a kernel puts both status words into pinned memory (two copies to pageable
+    // memory take longer), and what they say when one is raised is crow_hip_status's to report
+    if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
     unsigned* said = g.said + 2 * turn;
     void* a1[3] = {(void*)&g.ws.status, (void*)&g.ws_static.status, (void*)&said};
     if ((e = hipLaunchKernel((const void*)&status_words, dim3(1), dim3(1), a1, 0, g.stream)) != hipSuccess) return (int)e;
-    if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
+    if ((e = hipStreamSynchronize(g.stream)) != hipSuccess) return (int)e;
     return (said[0] | said[1]) == 0 ? CROW_OK : crow_hip_status();
 }
 

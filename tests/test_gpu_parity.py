@@ -82,6 +82,29 @@ def test_encode_repack_dequant_at_the_edges_of_their_blocks(eng, rows, cols):
     assert np.array_equal(got[1:1 + rows * cols].view(np.uint32), ref.view(np.uint32)) and got[0] == -1.0 and (got[1 + rows * cols:] == -1.0).all()
 
 
+def test_a_layout_call_reports_what_another_stream_is_about_to_raise(eng):
+    """A layout call waits for the device: a refusal of a launch still queued behind 50 ms of other work on another stream is
+    reported by it, not left for a later call."""
+    import ctypes as C
+    from crow_nest_amd import lib
+    from crow_nest_amd.kernels import launch_dims
+    from crow_nest_amd.weights import dequant
+    f = _load(random_nvfp4(7, 16, 256), 16, 256, 1.0e-3)
+    x, y, p = torch.ones(256, device="cuda"), torch.full((16,), 7.0, device="cuda"), eng.p
+    vals = [f.w_ptr, x.data_ptr(), f.gs_ptr, y.data_ptr(), p.i32(320), p.i32(16)]  # K of the word is not K of the dimensions: refused
+    dims = launch_dims("gemv_nvfp4_w", 16, 256)
+    eng.check()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(5_000_000)  # cycles of a 100 MHz counter
+    lib.check(lib.lib().crow_hip_launch(eng.k.f("gemv_nvfp4_w"), *dims, (C.c_uint64 * 6)(*vals), 6, side.cuda_stream), "crow_hip_launch")
+    with pytest.raises(lib.CrowHipError) as ei:
+        dequant(f)
+    assert ei.value.code == -7 and bool((y == 7.0).all())
+    eng.check()
+
+
 def test_dequant_every_scale_byte_and_the_refused_one(eng):
     from crow_nest_amd.lib import CrowHipError
     from crow_nest_amd.weights import dequant
