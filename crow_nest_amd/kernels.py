@@ -15,6 +15,7 @@ HIP error raises where the reference's ``cuda::ck`` panics.  Grid and block come
 from __future__ import annotations
 
 import ctypes as C
+import warnings
 from dataclasses import dataclass
 
 from . import lib as _l
@@ -82,10 +83,16 @@ class Kernels:
         for i in range(L.crow_hip_function_count()):
             name = L.crow_hip_function_name(i).decode()
             self.map[name] = module.get(name)
-        from . import _launch  # built beside the library; missing = not built, like the library itself
+        self._native = {name: (name.encode(), f) for name, f in self.map.items()}
+        self._launch = self._launch_at = None
+        try:
+            from . import _launch  # built beside the library where the interpreter's headers are
+        except ImportError as e:
+            warnings.warn(f"crow_nest_amd._launch is not built for this interpreter ({e}): launches go through ctypes, about 5 us more each "
+                          "(make -C crow_nest_amd/csrc builds it where Python.h is)", RuntimeWarning, stacklevel=2)
+            return
         _launch.bind(C.cast(L.crow_hip_launch_dims_split, C.c_void_p).value, C.cast(L.crow_hip_launch, C.c_void_p).value)
         self._launch, self._launch_at = _launch.launch, _launch.launch_at
-        self._native = {name: (name.encode(), f) for name, f in self.map.items()}
 
     def run(self, name: str, rows: int, k_dim: int, z: int, *vals: int) -> None:
         """``launch_v(f(name), *launch_dims(name, rows, k_dim, z), vals)`` in one native call: same dimensions, same errors."""
@@ -93,6 +100,8 @@ class Kernels:
             native, f = self._native[name]
         except KeyError:
             raise KernelMissing(f"kernel missing: {name}") from None
+        if self._launch is None:
+            return launch_v(f, *launch_dims(name, rows, k_dim, z), vals)
         rc = self._launch(native, f, rows, k_dim, z, *vals)
         if rc:
             launch_dims(name, rows, k_dim, z)  # raises if the dimensions were refused
@@ -100,6 +109,8 @@ class Kernels:
 
     def run_at(self, name: str, gx: int, gy: int, gz: int, bx: int, *vals: int) -> None:
         """``launch_v(f(name), gx, gy, gz, bx, vals)`` in one native call."""
+        if self._launch_at is None:
+            return launch_v(self.f(name), gx, gy, gz, bx, vals)
         rc = self._launch_at(self.f(name), gx, gy, gz, bx, *vals)
         if rc:
             _l.check(rc, "launch_v")

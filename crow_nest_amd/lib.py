@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 import subprocess
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _SO = os.environ.get("CROW_HIP_LIBRARY") or os.path.join(_HERE, "libcrow_hip.so")
@@ -29,7 +30,7 @@ def library_path() -> str:
 
 
 def build(force: bool = True) -> None:
-    cmd = ["make", "-C", os.path.join(_HERE, "csrc")] + (["-B"] if force else [])
+    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), f"PYTHON={sys.executable}"] + (["-B"] if force else [])
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("building libcrow_hip.so failed:\n" + r.stdout[-4000:] + r.stderr[-4000:])

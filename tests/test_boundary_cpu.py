@@ -165,6 +165,41 @@ def test_native_launch_call_arguments():
             _launch.launch(b"gemv_nvfp4_w", f.value, bad, 256, 1, *vals)
 
 
+def test_launches_without_the_native_launch_module(monkeypatch):
+    """An interpreter that the module was not built for launches through ctypes, says so once, and gets the same errors."""
+    import ctypes as C
+    import sys
+    import warnings
+    import torch
+    import crow_nest_amd
+    from crow_nest_amd import kernels as K
+
+    class Loaded:
+        def get(self, name):
+            out = C.c_void_p()
+            assert L.lib().crow_hip_get_function(name.encode(), C.byref(out)) == 0
+            return out.value
+
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        native = K.Kernels(Loaded())
+    monkeypatch.setitem(sys.modules, "crow_nest_amd._launch", None)
+    monkeypatch.delattr(crow_nest_amd, "_launch", raising=False)
+    with pytest.warns(RuntimeWarning, match="launches go through ctypes"):
+        plain = K.Kernels(Loaded())
+    for k in (native, plain):
+        with pytest.raises(K.KernelMissing):
+            k.run("no_such_kernel", 16, 256, 1, *[16] * 6)
+        with pytest.raises(L.CrowHipError) as ei:
+            k.run("gemv_nvfp4_w", 16, 100, 1, *[16] * 6)
+        assert ei.value.code == -7
+        if not torch.cuda.is_available():
+            for call in (lambda: k.run("gemv_nvfp4_w", 16, 256, 1, *[16] * 6), lambda: k.run_at("gemv_nvfp4_w", 1, 4, 1, 64, *[16] * 6)):
+                with pytest.raises(L.CrowHipError) as ei:
+                    call()
+                assert ei.value.code == -1  # not initialised
+
+
 def test_launch_dims_depend_on_the_matrix_only():
     import ctypes as C
     lib = L.lib()
