@@ -406,7 +406,11 @@ __device__ __forceinline__ void gemm_wide_body(const unsigned char* __restrict__
 // instruction that only partly overlap, and the power of the matrix cores.
 // blockIdx.x counts tiles in an order that keeps the tiles of one compute die (blockIdx.x % 8) together: four row blocks by
 // as many token blocks as fall to the die, so that its L2 serves both operands.
-__device__ const unsigned gemm_zeros[4] = {0u, 0u, 0u, 0u};
+struct alignas(16) ZeroChunk {
+    unsigned words[4];
+};
+static_assert(alignof(ZeroChunk) >= alignof(u32x4), "load_x reads it as one vector");
+__device__ const ZeroChunk gemm_zeros = {{0u, 0u, 0u, 0u}};
 typedef float f32x4_dword __attribute__((ext_vector_type(4), aligned(4)));  // rows of Y start at any dword
 template <int TBK, int NJ>
 struct TallTile {
@@ -530,7 +534,7 @@ struct TallTile {
         xrow = (threadIdx.x >> 5) * kd;
         auto next_panel = [&](int p, int buf) {  // the X tile that load_x and store_x move
             const int k = p * CROW_PANEL_COLS + xq;
-            from = k < k_dim ? x : (const unsigned short*)gemm_zeros;
+            from = k < k_dim ? x : (const unsigned short*)gemm_zeros.words;
             inside = k < k_dim ? ~0u : 0u;
             at_k = k < k_dim ? (unsigned)k : 0u;
             put = xs2 + buf * XBUF + ((int)threadIdx.x >> 5) * CROW_GEMM_XS_STRIDE + xq;
