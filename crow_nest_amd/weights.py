@@ -15,6 +15,8 @@ PyTorch tensors are used as device allocations only.
 """
 from __future__ import annotations
 
+import ctypes as C
+import itertools
 from dataclasses import dataclass
 
 import numpy as np
@@ -238,16 +240,36 @@ def load_expert_slabs(data, experts: int, rows: int, cols: int, global_scale: fl
     return ExpertSlabs(w, gs, experts, rows, cols, slab)
 
 
+def _store_word(ptr: int, v: int) -> None:
+    """One 32-bit word into device memory, there when this returns: a launch on any stream may read it."""
+    if not -(1 << 31) <= v < 1 << 31:
+        raise RuntimeError(f"value cannot be converted to type int32 without overflow: {v}")
+    _l.ensure_init()
+    L, word = _l.lib(), C.c_int32(int(v))
+    _l.check(L.crow_hip_upload(ptr, C.byref(word), 4), "crow_hip_upload")
+    if L.crow_hip_cur_stream():  # (an upload on a stream of the caller's is not waited for)
+        _l.check(L.crow_hip_sync(), "crow_hip_sync")
+
+
 class Params:
-    """Device words for kernel scalars (``Params`` of engine/src/gen.rs:2913-2925), created on demand."""
+    """Device words for kernel scalars (``Params`` of engine/src/gen.rs:2913-2925), created on demand: in blocks that live as long as
+    this object (a tensor per word takes its allocation and torch's copy on the first pass: 20 us, 15 so)."""
+
+    BLOCK = 1024  # words
 
     def __init__(self):
         self._dev = _device()
-        self._words: dict[int, tuple[int, torch.Tensor]] = {}  # address and the tensor that keeps it, as one value: the words live as long as this object
+        self._words: dict[int, int] = {}
+        self._blocks: dict[int, torch.Tensor] = {0: torch.empty(self.BLOCK, dtype=torch.int32, device=self._dev)}
+        self._slots = itertools.count()
 
     def i32(self, v: int) -> int:
-        word = self._words.get(v)
-        if word is None:
-            t = torch.tensor([v], dtype=torch.int32, device=self._dev)
-            word = self._words.setdefault(v, (t.data_ptr(), t))  # another thread's, if it was first
-        return word[0]
+        ptr = self._words.get(v)
+        if ptr is None:
+            block, at = divmod(next(self._slots), self.BLOCK)
+            if block not in self._blocks:
+                self._blocks.setdefault(block, torch.empty(self.BLOCK, dtype=torch.int32, device=self._dev))
+            ptr = self._blocks[block].data_ptr() + 4 * at
+            _store_word(ptr, v)
+            ptr = self._words.setdefault(v, ptr)  # another thread's, if it was first; this one's slot then stays unused
+        return ptr

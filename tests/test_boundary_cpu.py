@@ -122,22 +122,26 @@ def test_gemm_kernel_choice_knows_k(rows, m, k, want):
 def test_a_shape_word_made_by_two_threads_at_once_is_one_word(monkeypatch):
     """A second thread asks for the same value while the first is making its word: both get the same address, of a tensor that
     the object keeps - never one that nothing holds any more."""
-    import weakref
+    import ctypes as C
     import torch
     from crow_nest_amd import weights as W
     monkeypatch.setattr(W, "_device", lambda: torch.device("cpu"))
-    p, made, other, make = W.Params(), [], [], torch.tensor
+    p, made, other = W.Params(), [], []
 
-    def tensor(*a, **k):
-        t = make(*a, **k)
-        made.append((t.data_ptr(), weakref.ref(t)))
+    def store(ptr, v):
+        made.append(ptr)
+        C.c_int32.from_address(ptr).value = v
         if len(made) == 1:
             other.append(p.i32(7))  # what the second thread does meanwhile
-        return t
 
-    monkeypatch.setattr(torch, "tensor", tensor)
-    assert p.i32(7) == other[0] == p.i32(7) and len(made) == 2
-    assert [ref() is not None for ptr, ref in made if ptr == other[0]] == [True]
+    monkeypatch.setattr(W, "_store_word", store)
+    ptr = p.i32(7)
+    assert ptr == other[0] == p.i32(7) and len(set(made)) == 2 and ptr in made
+    # every word stays what it is, in memory that the object keeps, across more than one block of words
+    words = {v: p.i32(v) for v in range(-3, 2 * p.BLOCK)}
+    assert words[7] == ptr and len(set(words.values())) == len(words)
+    assert all(C.c_int32.from_address(at).value == v == C.c_int32.from_address(p.i32(v)).value for v, at in words.items())
+    assert all(any(0 <= at - t.data_ptr() < 4 * p.BLOCK for t in p._blocks.values()) for at in words.values())
 
 
 def test_native_launch_call_arguments():

@@ -105,6 +105,26 @@ def test_a_layout_call_reports_what_another_stream_is_about_to_raise(eng):
     eng.check()
 
 
+def test_shape_words_made_while_launches_go_to_a_stream_of_the_callers(eng):
+    """New words are in device memory when their address is handed out, whatever stream the library launches on."""
+    from crow_nest_amd import lib
+    from crow_nest_amd.weights import Params
+    f = _load(random_nvfp4(8, 48, 320), 48, 320, 1.0e-3)
+    x, side, old = torch.ones((1, 320), device="cuda"), torch.cuda.Stream(), eng.p
+    want = eng.dense_proj(f, 1, x)
+    torch.cuda.synchronize()
+    try:
+        lib.lib().crow_hip_set_stream(side.cuda_stream)
+        for _ in range(20):
+            eng.p = Params()
+            got = eng.dense_proj(f, 1, x)
+            eng.check()
+            assert torch.equal(got, want)
+    finally:
+        eng.p = old
+        lib.lib().crow_hip_set_stream(None)
+
+
 def test_dequant_every_scale_byte_and_the_refused_one(eng):
     from crow_nest_amd.lib import CrowHipError
     from crow_nest_amd.weights import dequant
