@@ -973,7 +973,8 @@ def test_config3_full_size_head(eng):
 # ---------------------------------------------------------------- batched GEMM on the matrix cores (config 4)
 
 @pytest.mark.parametrize("kernel", ["gemm_nvfp4_bf16_m16", "gemm_nvfp4_bf16_m32", "gemm_nvfp4_bf16_m48", "gemm_nvfp4_bf16_m64", "gemm_nvfp4_bf16_m96",
-                                    "gemm_nvfp4_bf16", "gemm_nvfp4_bf16_w48", "gemm_nvfp4_bf16_w64", "gemm_nvfp4_bf16_w80", "gemm_nvfp4_bf16_w96"])
+                                    "gemm_nvfp4_bf16", "gemm_nvfp4_bf16_w48", "gemm_nvfp4_bf16_w64", "gemm_nvfp4_bf16_w80", "gemm_nvfp4_bf16_w96",
+                                    "gemm_nvfp4_bf16_t64", "gemm_nvfp4_bf16_t96", "gemm_nvfp4_bf16_t128"])
 @pytest.mark.parametrize("m,rows,cols", [(16, 320, 1024), (5, 100, 320), (17, 100, 320), (33, 256, 512), (128, 512, 2048), (200, 192, 5120)])
 def test_gemm_bf16_against_the_cpu_path(eng, m, rows, cols, kernel):
     """Weights decode to exact bf16, X is bf16, products are exact in f32: only the summation order
@@ -1003,6 +1004,35 @@ def test_gemm_ragged_shapes_drawn_at_random(eng):
             eng.check()
             assert rel_err(y, ref, floor_of(y.size)) <= TOL, (case, kernel)
             assert gamma_ratio(y[:2], w, rows, cols, gs, xw.reshape(m, cols)[:2]) <= 1.0, (case, kernel)
+
+
+def test_gemm_large_ragged_shapes_through_the_choice(eng):
+    """Shapes drawn with a fixed seed whose product the library gives to a shared-X, eight-wave or tall-tile kernel (all nine
+    that it names beside the K-split ones), and through every tall tile: all tokens by the bits of one reference kernel - the kernels with a wave per
+    weight row add in the same order - and that kernel's first, a middle and last token against the CPU path."""
+    from crow_nest_amd.engine import gemm_kernel_for
+    g, named = np.random.default_rng(4243), set()
+    while len(named) < 9:
+        rows, m, cols = int(g.integers(700, 12000)), int(g.integers(150, 1700)), 64 * int(g.integers(1, 40))
+        name = gemm_kernel_for(m, rows, cols)[len("gemm_nvfp4_bf16_"):]
+        if name in named or name == "m32":
+            continue
+        named.add(name)
+        print(f"m={m} rows={rows} cols={cols} {name}", flush=True)
+        w, gs = random_nvfp4(700 + len(named), rows, cols), 6.0e-4
+        f = _load(w, rows, cols, gs)
+        xb, xw = _bf16_dev(normal_f32(18, len(named), m * cols))
+        x, xw = xb.reshape(m, cols).contiguous(), xw.reshape(m, cols)
+        ref = eng.gemm(f, m, x, kernel="gemm_nvfp4_bf16_w48")
+        for kernel in (None, "gemm_nvfp4_bf16_t64", "gemm_nvfp4_bf16_t96", "gemm_nvfp4_bf16_t128"):
+            got = eng.gemm(f, m, x, kernel=kernel)
+            eng.check()
+            assert torch.equal(got, ref), (name, kernel)
+        picks = [0, m // 2, m - 1]
+        y = ref[picks].cpu().numpy()
+        assert rel_err(y, orc.gemv(w, rows, cols, gs, xw[picks], threads=8), floor_of(y.size)) <= TOL, name
+        assert gamma_ratio(y, w, rows, cols, gs, xw[picks]) <= 1.0, name
+    assert named == {"m48", "m64", "w48", "w64", "w80", "w96", "t64", "t96", "t128"}
 
 
 @pytest.mark.parametrize("kernel,m,rows,cols", [
