@@ -119,6 +119,7 @@ struct State {
     crow::Geo model{0, 0, 0, 0};  // the routed geometry (crow_hip_set_geo): appended by value to the kernels that take it
     size_t lds_cap = 64u * 1024u;  // most LDS one workgroup may take on this device
 } g;
+std::atomic<bool> g_other_streams{false};  // a launch has gone to a stream that is not the null stream (or been captured from one)
 
 // Scratch memory of crow_hip_launch_noalloc: part of the code object, so it exists on a device from the moment the library
 // is loaded there until the process ends, and no call ever allocates it.  Words [0, NOALLOC_PARTIAL_FLOATS) hold the partial
@@ -220,6 +221,7 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
     const bool head = e->stub == (const void*)&gemv_nvfp4_w_argmax;
     // the fused head keeps one key per strip (the kernel checks again and reports through the status word)
     if (head && grid.x > ws.head_words) return CROW_ERR_WORKSPACE;
+    if (s != nullptr) g_other_streams.store(true);  // (before the launch: see layout_launch)
     hipError_t rc = hipLaunchKernel(stub, grid, block, args, lds, s);
     if (rc == hipSuccess && head) {  // ... and its finishing kernel right behind it: the token out of the strips' keys
         unsigned strips = grid.x;
@@ -556,7 +558,7 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         const uint32_t hint = from_memory ? 0 : (verify ? z : (tokens ? (z - 1) % 4 + 1 : 0));
         // Two strips per block share the operand reads of several f32 rows; where that leaves compute units without a block, and
         // up to two blocks a unit where a strip is short, one strip per block is faster (three rows, us, two / one strips per block:
-        // [2048, 5120] 8.6 / 7.4, [4096, 5120] 8.7 / 8.3, [8192, 2048] 6.0 / 5.5, [6151, 3008] 7.0 / 6.7; [5120, 5120] 8.8 / 10.1,
+        // [2048, 5120] 8.6 / 7.4, [4096, 5120] 8.7 / 8.3, [8192, 2048] 6.0 / 5.5, [6144, 3072] 6.9 / 6.5, [8192, 3072] 7.2 / 6.5; one group more, [6144, 3328] 7.2 / 7.6; [5120, 5120] 8.8 / 10.1,
         // [12288, 3072] 9.2 / 9.6; gate|up [4096, 5120] 13.3 / 11.3, [5120, 2048] 10.8 / 11.1).  Same bits.
         // Four waves on a strip of up to 14 groups walk two to four groups each.  Many token groups fill the chip with such short walks:
         // there two waves take the four runs between them (blocks of more than three per compute unit; us, four waves / two waves with
@@ -900,13 +902,16 @@ static int layout_launch(const char* name, const void* a, const void* b, const v
     vals[n++] = (uint64_t)(sc + 1);
     rc = launch_entry(find(name), dim3(d.gx, d.gy, d.gz), dim3(d.bx), vals, n, g.stream, g.ws);
     if (rc != CROW_OK) return rc;
-    // every stream idle, as in crow_hip_status; then a kernel puts both status words into pinned memory (two copies to pageable
-    // memory take longer), and what they say when one is raised is crow_hip_status's to report
-    if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
+    // A kernel puts both status words into pinned memory (two copies to pageable memory take longer); what they say when one is
+    // raised is crow_hip_status's to report.  It must run when every stream is idle, as crow_hip_status reads them: behind a wait for the
+    // device - but while all launches so far went to the null stream, it is behind all of them where it stands, and one wait does
+    // (a small layout call 18 us, 27 with two waits).
+    const bool elsewhere = g_other_streams.load();
+    if (elsewhere && (e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
     unsigned* said = g.said + 2 * turn;
     void* a1[3] = {(void*)&g.ws.status, (void*)&g.ws_static.status, (void*)&said};
     if ((e = hipLaunchKernel((const void*)&status_words, dim3(1), dim3(1), a1, 0, g.stream)) != hipSuccess) return (int)e;
-    if ((e = hipStreamSynchronize(g.stream)) != hipSuccess) return (int)e;
+    if ((e = elsewhere ? hipStreamSynchronize(g.stream) : hipDeviceSynchronize()) != hipSuccess) return (int)e;
     return (said[0] | said[1]) == 0 ? CROW_OK : crow_hip_status();
 }
 
