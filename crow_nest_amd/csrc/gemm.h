@@ -399,9 +399,9 @@ __device__ __forceinline__ void gemm_wide_body(const unsigned char* __restrict__
 //     decoded: half a panel of matrix work covers the round trip with a single register set;
 //   * the next X tile travels through registers, one 16-byte chunk requested per unit and one written per unit to the other LDS
 //     buffer, and the panel's only barrier stands before segment 7, whose operands are in registers by then.
-// Measured ([17408, 5120] x 512 tokens / [5120, 17408] x 1999, TBK = 8): 82 us / 289 us against 107 / 342 for the eight-wave
-// body at 80 tokens, 1.11 / 1.23 PFLOP/s; a library bf16 product of the first shape takes 100 us, and 8192^3 runs at 1.07 to
-// 1.39.  A panel takes 8250 cycles at 1.9 to 2.0 GHz where its matrix instructions alone take 5280; without the decode 7000, without
+// Measured ([17408, 5120] x 512 tokens / [5120, 17408] x 1999, TBK = 8): 81 to 90 us / 281 to 308 us by the session against 107 to 111 /
+// 342 to 354 for the eight-wave body at 80 tokens, 1.0 to 1.13 / 1.16 to 1.27 PFLOP/s; a library bf16 product of the first shape takes
+// 100 us, and 8192^3 runs at 1.31 to 1.41.  A panel takes 8250 cycles at 1.9 to 2.0 GHz where its matrix instructions alone take 5280; without the decode 7000, without
 // the matrix instructions 5000, with all activations zero the same cycles at 2.2 GHz: what remains is the two kinds of
 // instruction that only partly overlap, and the power of the matrix cores.
 // blockIdx.x counts tiles in an order that keeps the tiles of one compute die (blockIdx.x % 8) together: four row blocks by
