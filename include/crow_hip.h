@@ -99,7 +99,9 @@ int crow_hip_launch(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, uint32_t
 int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, uint32_t bx, const uint64_t* vals,
                             uint32_t n_vals, void* stream);
 /* grid/block for `name` on a [rows, k_dim] tensor with `z` token rows (batched and verify kernels: the value *t_p / *m_p
- * will hold) or combos (routed kernels); 1 otherwise.  The split of the work depends on (rows, k_dim) only, never on z.
+ * will hold) or combos (routed kernels); 1 otherwise.  How a row's columns are split into sums, and so its bits, depends on
+ * (rows, k_dim) only, never on z.  (Which waves make the sums may: see the values of `gy` above.  For the unquantised GEMVs
+ * gz = 2 asks for the form that requests weights alone ahead; a caller's own grid with gz = 1 serves every size.)
  *
  * Dimensions made for a row count are BOUND to it: the count rides in `gy`, the kernel works with it from its first
  * instruction and stores nothing (CROW_ERR_SHAPE from crow_hip_status) if the word behind m_p / t_p says otherwise - so a
