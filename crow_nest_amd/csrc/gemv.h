@@ -974,16 +974,19 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, unsigned z, lds_p l
     const int groups = (a.pairs + CROW_GROUP_PAIRS - 1) / CROW_GROUP_PAIRS;
     const int wpt = NR == 2 ? waves >> 1 : waves;            // waves per tensor
     const int r_own = (NR == 2 && wave >= wpt) ? 1 : 0;      // wave-uniform
-    const int unit = slice * wpt + (wave - r_own * wpt), units = slices * wpt * RUNS;  // (two runs per wave: `unit` and the one `half` on)
+    const int unit = slice * wpt + (wave - r_own * wpt), units = slices * wpt * RUNS;  // (two runs per wave: `unit` and the one slices * wpt on)
     // the strip's groups in runs of floor(groups / units), the first groups % units runs one longer
     const int base = groups / units, rem = groups - base * units;
     // (a two-tensor block launched with an odd number of waves has one wave too many: it takes nothing, and the launch is
     // refused at the store - not here, where the refusal would sit between a wave's start and its first weight load)
     const bool extra_wave = NR == 2 && wave - r_own * wpt >= wpt;
-    const int half = slices * wpt, second = unit + half;
-    const int first_run = base + (unit < rem ? 1 : 0), first = unit * base + (unit < rem ? unit : rem);
-    const int count = extra_wave ? 0 : first_run + (RUNS == 2 ? base + (second < rem ? 1 : 0) : 0);
-    const int jump = second * base + (second < rem ? second : rem) - first - first_run;  // from behind the first run to the second
+    const int run = extra_wave ? 0 : base + (unit < rem ? 1 : 0), first = unit * base + (unit < rem ? unit : rem);
+    int count = run, jump = 0;
+    if constexpr (RUNS == 2) {
+        const int second = unit + slices * wpt;
+        count = run + base + (second < rem ? 1 : 0);
+        jump = second * base + (second < rem ? second : rem) - first - run;  // from behind the first run to the second
+    }
     const unsigned char* wsel = r_own != 0 ? a.w[1] : a.w[0];  // a select, never an indexed read
     // element offsets of this launch's activation rows, and which output row each of them writes
     size_t xoff[M];
@@ -1026,7 +1029,7 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, unsigned z, lds_p l
 #pragma unroll
         for (int s = 0; s < NS; s++) sp[s] = wsel + (size_t)(strip + (s < have ? s : 0)) * groups * CROW_GROUP_BYTES;
         MultiWalk<M, XBF16, NS, RUNS> walk;
-        walk.init(sp, first, first_run, jump, k_dim, a.x, xoff, areas + wave * AREA, zero);
+        walk.init(sp, first, run, jump, k_dim, a.x, xoff, areas + wave * AREA, zero);
         walk.go(count, mid);
         walk.finish(part);
     }
