@@ -33,12 +33,16 @@ struct FnEntry {
     const void* one_stub = nullptr;  // a twin of `stub` with one strip per block, started in its place when S = CROW_ONE_STRIP
     const void* two_stub = nullptr;  // ... and one with two runs of columns per wave, when S = CROW_TWO_RUNS
     const void* ahead_stub = nullptr;  // unquantised GEMVs: a twin that requests weights alone ahead, when the launch's gz = CROW_KEEP_AHEAD
+    bool ksplit = false;  // GEMM for few token rows: one of g_ksplit starts in its place when the launch's gz says which (CROW_KSPLIT)
 };
 // values of S in a launch's `gy` word (GEMV family, K up to 16384; a strip of at most 64 groups never has that many slices): one
 // slice, and one strip per block where the kernel otherwise takes `ns` of them / two runs of columns per wave of the block
 #define CROW_ONE_STRIP 0x81u
 #define CROW_TWO_RUNS 0x82u
 #define CROW_KEEP_AHEAD 2u  // (the grid of those kernels has no third dimension)
+// A K-split GEMM in gz: this bit, bits 0..7 the column slices, 8..11 the strips per block, 12..15 the 16-token blocks per block, 16..23
+// the waves per block
+#define CROW_KSPLIT 0x80000000u
 
 // The launcher builds a kernel's argument array from the fields of its table entry: the caller's `nargs` values, then the
 // geometry word (GEMV family), the scratch descriptor (takes_ws), the model geometry (takes_geo).  A kernel that gains a
@@ -60,6 +64,8 @@ constexpr int checked_nargs(F) {
 #define CROW_FN(name, nargs) {#name, (const void*)&name, checked_nargs<nargs, 0>(&name), 0u, 0, 16, 0, 1, false, nullptr, false}
 #define CROW_FN_KEEP(name, nargs, twin) \
     {#name, (const void*)&name, checked_nargs<nargs, 0>(&name) + 0 * checked_nargs<nargs, 0>(&twin), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, (const void*)&twin}
+#define CROW_FN_KSPLIT(name, nargs) \
+    {#name, (const void*)&name, checked_nargs<nargs, 0>(&name), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, nullptr, true}
 #define CROW_FN_GEO(name, nargs) {#name, (const void*)&name, checked_nargs<nargs, 1>(&name), 0u, 0, 16, 0, 1, false, nullptr, true}
 // NR tensors per block, bodies for 1 .. MMAX activation rows, bf16 or f32 activations
 // (the bodies for several rows need more registers than a block of sixteen waves leaves each: they run in blocks of eight)
@@ -99,19 +105,31 @@ const FnEntry g_table[] = {
     {"gemm_nvfp4_bf16_t64", (const void*)&gemm_nvfp4_bf16_t64, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t64), 2u * 64u * 528u, 0, 4, 0, 1, false},
     {"gemm_nvfp4_bf16_t96", (const void*)&gemm_nvfp4_bf16_t96, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t96), 2u * 96u * 528u, 0, 4, 0, 1, false},
     {"gemm_nvfp4_bf16_t128", (const void*)&gemm_nvfp4_bf16_t128, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t128), 2u * 128u * 528u, 0, 4, 0, 1, false},
-    CROW_FN(gemm_nvfp4_bf16_m32, 7), CROW_FN(gemm_nvfp4_bf16_m16, 7), CROW_FN_KEEP(gemv_bf16_w, 5, gemv_bf16_ahead),
+    CROW_FN_KSPLIT(gemm_nvfp4_bf16_m32, 7), CROW_FN_KSPLIT(gemm_nvfp4_bf16_m16, 7), CROW_FN_KEEP(gemv_bf16_w, 5, gemv_bf16_ahead),
     CROW_FN_KEEP(gemv_bf16, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_bf16_b, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_b, 5, gemv_b_ahead),
     CROW_FN_KEEP(gemv_bf16_ws, 5, gemv_bf16_ws_ahead), CROW_FN_KEEP(gemv_bf16_bs, 6, gemv_bf16_bs_ahead),
     CROW_FN(gemv_nvfp4_w_valu1, 6), CROW_FN(gemv_nvfp4_w_valu2, 6), CROW_FN(gemv_nvfp4_w_valu4, 6),  // measurement only
 };
 const int g_table_n = (int)(sizeof(g_table) / sizeof(g_table[0]));
 
+// The K-split GEMM kernels (gemm.h) by [16-token blocks - 1][strips - 1] of a block
+struct KSplitEntry {
+    const void* stub;
+    int max_waves, lds_per_wave;
+};
+#define CROW_KSPLIT_ROW(TBK, NJ, MT, WAVES) \
+    {(const void*)&gemm_ksplit_##MT##x##NJ, WAVES + 0 * checked_nargs<7, 2>(&gemm_ksplit_##MT##x##NJ), crow::KSplitTile<TBK, NJ>::AREA},
+#define CROW_KSPLIT_NJ 5
+const KSplitEntry g_ksplit[4 * CROW_KSPLIT_NJ] = {CROW_GEMM_KSPLIT_ALL(CROW_KSPLIT_ROW)};
+
+const int STREAM_SLOTS = 4;
 struct State {
     bool ready = false;
     int device = -1;
     int cus = 256;
     hipStream_t stream = nullptr;
-    crow::Workspace ws{};
+    crow::Workspace ws{};  // the null stream's, and any stream's beyond the first STREAM_SLOTS others
+    crow::Workspace ws_more[STREAM_SLOTS] = {};  // those streams': same roles and sizes, the one status word
     crow::Workspace ws_static{};  // the same roles inside `scratch`, through the device address crow_hip_init asked for
     unsigned* said = nullptr;  // pinned host words: the two status words as the layout calls last read them, eight pairs in turn
     int* scalars = nullptr;  // device words for the library's own launches: (rows, k_dim) of the layout calls, the encoder's maxima
@@ -119,6 +137,7 @@ struct State {
     crow::Geo model{0, 0, 0, 0};  // the routed geometry (crow_hip_set_geo): appended by value to the kernels that take it
     size_t lds_cap = 64u * 1024u;  // most LDS one workgroup may take on this device
 } g;
+std::atomic<hipStream_t> g_slot_of[STREAM_SLOTS];  // which stream ws_more[i] belongs to; kept until crow_hip_shutdown (a graph captured there may outlive the stream)
 std::atomic<bool> g_other_streams{false};  // a launch has gone to a stream that is not the null stream (or been captured from one)
 
 // Scratch memory of crow_hip_launch_noalloc: part of the code object, so it exists on a device from the moment the library
@@ -157,6 +176,20 @@ const FnEntry* entry_of(crow_fn_t f) {
 }
 
 
+// The scratch memory of launches on stream s, and whether launches on other streams leave it alone
+const crow::Workspace& workspace_of(hipStream_t s, bool& own) {
+    own = true;
+    if (s == nullptr || s == hipStreamLegacy) return g.ws;
+    if (s != hipStreamPerThread)  // (one handle, a stream per thread)
+        for (int i = 0; i < STREAM_SLOTS; i++) {
+            hipStream_t at = g_slot_of[i].load();
+            if (at == nullptr && g_slot_of[i].compare_exchange_strong(at, s)) return g.ws_more[i];
+            if (at == s) return g.ws_more[i];
+        }
+    own = false;
+    return g.ws;
+}
+
 // Groups per strip if the grouped expert kernels take their twin for K / 64 = pairs (strips of two to eight groups that one
 // wave walks alone in the launch shapes chosen below: up to 7 groups for one tensor, 10 - here 8 - per tensor for two), else 0.
 unsigned tile_groups(int nr, unsigned pairs) {
@@ -167,8 +200,8 @@ unsigned tile_groups(int nr, unsigned pairs) {
 // The launch dimensions of the GEMV family carry the problem in `gy` (crow_hip_launch_dims writes it, callers pass it on
 // unchanged): bits 0..19 = K / 64, bits 20..23 = activation rows of the last token group (0 = not given), bits 24..31 = S, the
 // number of column slices per strip.  The real grid is (gx, S, gz); the low 24 bits reach the kernel by value.
-// `ws`: the scratch memory the launch may use, handed by value to the kernels that take one.
-int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, uint32_t n, hipStream_t s, const crow::Workspace& ws) {
+// `ws`: the scratch memory the launch may use, handed by value to the kernels that take one; `own_ws`: no launch on another stream uses it.
+int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, uint32_t n, hipStream_t s, const crow::Workspace& ws, bool own_ws) {
     if (!g.ready) return CROW_ERR_NOT_INITIALIZED;
     if (!e || !vals) return CROW_ERR_BAD_ARGUMENT;
     if ((int)n != e->nargs) return CROW_ERR_ARG_COUNT;
@@ -211,11 +244,30 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
         if (lds > g.lds_cap) return CROW_ERR_SHAPE;
         args[na++] = (void*)&geo;
     }
+    bool with_ws = e->takes_ws;
+    if (e->ksplit && (grid.z & CROW_KSPLIT) != 0) {
+        const unsigned word = grid.z, nj = (word >> 8) & 0xFu, tbk = (word >> 12) & 0xFu, most = (word >> 16) & 0xFFu;
+        if (nj < 1 || nj > CROW_KSPLIT_NJ || tbk < 1 || tbk > 4 || most == 0 || (word & 0xFFu) == 0) return CROW_ERR_BAD_ARGUMENT;
+        const KSplitEntry& k = g_ksplit[(tbk - 1) * CROW_KSPLIT_NJ + nj - 1];
+        if (block.x > 64u * (unsigned)k.max_waves) return CROW_ERR_BAD_ARGUMENT;
+        stub = k.stub;
+        // slices meet in scratch memory: a stream that has none of its own keeps the panels in one block (other bits, no slices)
+        grid.z = own_ws ? word & 0xFFu : 1u;
+        // (the kernel checks again and reports through the status word)
+        if (grid.z > 1 && ((unsigned long long)grid.x * grid.y * nj * grid.z * 256ull * tbk > ws.partial_floats ||
+                           (unsigned long long)grid.x * grid.y * nj > ws.counter_slots))
+            return CROW_ERR_WORKSPACE;
+        lds = (size_t)(block.x / 64) * (size_t)k.lds_per_wave;
+        if (lds > g.lds_cap) return CROW_ERR_SHAPE;
+        geo = (int)most;
+        args[na++] = (void*)&geo;
+        with_ws = true;
+    }
     if (e->ahead_stub != nullptr && grid.z == CROW_KEEP_AHEAD) {
         stub = e->ahead_stub;
         grid.z = 1;
     }
-    if (e->takes_ws) args[na++] = (void*)&ws_arg;
+    if (with_ws) args[na++] = (void*)&ws_arg;
     crow::Geo model_arg = g.model;
     if (e->takes_geo) args[na++] = (void*)&model_arg;
     const bool head = e->stub == (const void*)&gemv_nvfp4_w_argmax;
@@ -230,6 +282,12 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
     }
     if (rc != hipSuccess) (void)hipGetLastError();  // reported here: not left behind for an unrelated later call to find
     return hip_rc(rc);
+}
+int launch_on(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, uint32_t n, hipStream_t s) {
+    if (!g.ready) return CROW_ERR_NOT_INITIALIZED;
+    bool own;
+    const crow::Workspace& ws = workspace_of(s, own);
+    return launch_entry(e, grid, block, vals, n, s, ws, own);
 }
 
 }  // namespace
@@ -252,6 +310,7 @@ int crow_hip_init(int device) {
     crow::Workspace ws{};
     ws.partial_floats = PARTIAL_FLOATS;
     ws.counter_slots = COUNTER_SLOTS;
+    crow::Workspace more[STREAM_SLOTS] = {};
     int* scalars = nullptr;
     unsigned* said = nullptr;
     // one failure path: everything allocated so far is released again
@@ -259,6 +318,7 @@ int crow_hip_init(int device) {
         (void)hipFree(ws.partials);
         (void)hipFree(ws.counters);
         (void)hipFree(ws.head);
+        for (crow::Workspace& m : more) (void)hipFree(m.partials), (void)hipFree(m.counters), (void)hipFree(m.head);
         (void)hipFree(scalars);
         (void)hipHostFree(said);
         return (int)why;
@@ -272,6 +332,14 @@ int crow_hip_init(int device) {
     if ((e = hipHostMalloc((void**)&said, 16 * sizeof(unsigned), hipHostMallocDefault)) != hipSuccess) return fail(e);
     if ((e = hipMemset(ws.counters, 0, COUNTER_WORDS * sizeof(unsigned))) != hipSuccess) return fail(e);
     ws.status = ws.counters + COUNTER_SLOTS;
+    for (crow::Workspace& m : more) {
+        m = crow::Workspace{nullptr, nullptr, PARTIAL_FLOATS, COUNTER_SLOTS, ws.status, nullptr, HEAD_WORDS};
+        if ((e = hipMalloc((void**)&m.partials, PARTIAL_FLOATS * sizeof(float))) != hipSuccess) return fail(e);
+        if ((e = hipMalloc((void**)&m.counters, COUNTER_WORDS * sizeof(unsigned))) != hipSuccess) return fail(e);
+        if ((e = hipMalloc((void**)&m.head, HEAD_WORDS * sizeof(unsigned long long))) != hipSuccess) return fail(e);
+        if ((e = hipMemset(m.head, 0, HEAD_WORDS * sizeof(unsigned long long))) != hipSuccess) return fail(e);
+        if ((e = hipMemset(m.counters, 0, COUNTER_WORDS * sizeof(unsigned))) != hipSuccess) return fail(e);
+    }
     if ((e = hipMemcpyToSymbol(HIP_SYMBOL(crow::g_ws), &ws, sizeof ws)) != hipSuccess) return fail(e);
     // a GEMV block of 16 waves, and the GEMM's two staged X tiles, need more dynamic LDS than the default per-block limit
     for (int i = 0; i < g_table_n; i++) {
@@ -293,6 +361,10 @@ int crow_hip_init(int device) {
             (e = hipFuncSetAttribute(g_table[i].tile_stub, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tile_most)) != hipSuccess)
             return fail(e);
     }
+    for (const KSplitEntry& k : g_ksplit) {
+        const size_t most = (size_t)k.max_waves * (size_t)k.lds_per_wave;
+        if (most > 48 * 1024 && (e = hipFuncSetAttribute(k.stub, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(most < g.lds_cap ? most : g.lds_cap))) != hipSuccess) return fail(e);
+    }
     // `scratch` in host code is a stand-in, not a device address: ask for this device's copy once, and use only that
     unsigned* sp = nullptr;
     if ((e = hipGetSymbolAddress((void**)&sp, HIP_SYMBOL(scratch))) != hipSuccess || sp == nullptr) return fail(e != hipSuccess ? e : hipErrorInvalidSymbol);
@@ -310,6 +382,7 @@ int crow_hip_init(int device) {
     g.scalars = scalars;
     g.said = said;
     g.ws = ws;
+    for (int i = 0; i < STREAM_SLOTS; i++) g.ws_more[i] = more[i];
     g.ws_static = st;
     g.device = device;
     g.stream = nullptr;
@@ -323,6 +396,10 @@ int crow_hip_shutdown(void) {
     (void)hipFree(g.ws.partials);
     (void)hipFree(g.ws.counters);
     (void)hipFree(g.ws.head);
+    for (int i = 0; i < STREAM_SLOTS; i++) {
+        (void)hipFree(g.ws_more[i].partials), (void)hipFree(g.ws_more[i].counters), (void)hipFree(g.ws_more[i].head);
+        g_slot_of[i].store(nullptr);
+    }
     (void)hipFree(g.scalars);
     (void)hipHostFree(g.said);
     g = State{};
@@ -395,7 +472,7 @@ int crow_hip_launch(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, uint32_t
                     void* stream) {
     const FnEntry* e = entry_of(f);
     if (!e) return CROW_ERR_KERNEL_MISSING;
-    return launch_entry(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream, g.ws);
+    return launch_on(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream);
 }
 
 int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, uint32_t bx, const uint64_t* vals,
@@ -405,10 +482,67 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
     // only kernels that are handed their scratch memory as an argument can be pointed at the static array
     if (!e->takes_ws) return CROW_ERR_BAD_ARGUMENT;
     // launch_entry refuses (CROW_ERR_WORKSPACE) a split whose partial sums or counters do not fit what it is given
-    return launch_entry(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream, g.ws_static);
+    return launch_entry(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream, g.ws_static, false);
 }
 
-// Which GEMM entry point for m token rows on a [rows, k_dim] tensor.  Up to 16 rows: the K-split body over blocks.  Beyond that the
+// Waves, strips and column slices of a K-split GEMM block (gemm.h: KSplitTile) for m <= 64 token rows: what the following time is least
+// for, of 1 to 5 strips, 4 / 8 / 12 waves and 1 to 8 slices.  `rounds` of blocks one behind the other, as many of them together on a
+// compute unit as registers and LDS allow; panels per wave and per block; blocks per compute unit.
+//   us = c0 + (slices > 1) (c1 + c2 slices) + rounds (c3 + panels per wave (c4 + c5 strips)) + rounds together panels (c6 strips + c7)
+//        + blocks / compute units (panels (c8 strips + c9) + c10 strips) + c11 waves
+// was fitted to the times of all of them on MI355X at 104 tensors (rows 512 .. 17408, K 512 .. 17408) x 5, 16, 17, 32, 48 and 64 rows;
+// what it picks is 1 to 3 % behind the fastest on average, 28 % at worst, and between 0.99 and 4.4 times as fast as the kernels
+// that served these sizes before (m16, m32, m48, m64): 1.34 (64 rows) to 1.69 times (17 rows) on average.
+struct KSplitPlan {
+    double us;
+    uint32_t nj, waves, slices;
+};
+static KSplitPlan ksplit_search(uint32_t strips, uint32_t panels, uint32_t m, uint32_t force_s, uint32_t force_w) {
+    static const double coef[4][12] = {{2.452, 1.165, 0.201, 0.72, 0.099, 0.208, 0.028, 0.026, 0.056, 0.007, 0.0, 0.041},
+                                       {2.398, 1.281, 0.276, 0.914, 0.291, 0.211, 0.052, 0.036, 0.04, 0.048, 0.024, 0.079},
+                                       {2.745, 1.182, 0.383, 0.836, 0.164, 0.373, 0.028, 0.16, 0.049, 0.047, 0.07, 0.106},
+                                       {2.671, 1.108, 0.402, 1.149, 0.307, 0.321, 0.058, 0.147, 0.031, 0.097, 0.098, 0.145}};
+    static const unsigned char waves_per_simd[4][CROW_KSPLIT_NJ] = {{7, 5, 4, 4, 3}, {5, 4, 4, 3, 3}, {5, 4, 4, 3, 2}, {4, 3, 3, 2, 2}};  // (their registers)
+    const uint32_t tbk = (m + 15) / 16, cus = g.cus > 0 ? (uint32_t)g.cus : 256u;
+    const double* c = coef[tbk - 1];
+    KSplitPlan best{0.0, 0, 0, 0};
+    for (uint32_t nj = 1; nj <= CROW_KSPLIT_NJ; nj++) {
+        const KSplitEntry& k = g_ksplit[(tbk - 1) * CROW_KSPLIT_NJ + nj - 1];
+        const uint32_t tiles = (strips + nj - 1) / nj;
+        for (uint32_t w = 4; w <= 12; w += 4) {
+            if (w > (uint32_t)k.max_waves || w < nj || (force_w > 0 && w != force_w)) continue;
+            uint32_t fit = 4u * waves_per_simd[tbk - 1][nj - 1] / w;
+            const uint32_t by_lds = 163840u / (w * (uint32_t)k.lds_per_wave);
+            if (fit > by_lds) fit = by_lds;
+            if (fit < 1) fit = 1;
+            for (uint32_t s = 1; s <= 8; s += s < 4 ? 1 : 2) {
+                if (force_s > 0 && s != force_s) continue;
+                if (s > 1 && ((s - 1) * w >= panels || (unsigned long long)tiles * nj * s * 256ull * tbk > PARTIAL_FLOATS || (unsigned long long)tiles * nj > COUNTER_SLOTS)) continue;
+                const uint32_t blocks = tiles * s, n = (blocks + cus - 1) / cus, rounds = (n + fit - 1) / fit, together = n < fit ? n : fit;
+                const double own = (double)((panels + w * s - 1) / (w * s)), all = (double)panels / s, f = (double)blocks / cus, r = rounds;
+                const double us = c[0] + (s > 1 ? c[1] + c[2] * s : 0.0) + r * (c[3] + own * (c[4] + c[5] * nj)) + r * together * all * (c[6] * nj + c[7]) +
+                                  f * (all * (c[8] * nj + c[9]) + c[10] * nj) + c[11] * w;
+                if (best.nj == 0 || us < best.us) best = KSplitPlan{us, nj, w, s};
+            }
+        }
+    }
+    return best;
+}
+// The search takes 0.5 us, a tenth of a small call: each thread keeps what it found for the last shapes (a program has a few dozen).
+static KSplitPlan ksplit_plan(uint32_t strips, uint32_t panels, uint32_t m, uint32_t force_s, uint32_t force_w) {
+    if (force_s != 0 || force_w != 0) return ksplit_search(strips, panels, m, force_s, force_w);
+    struct Kept {
+        uint32_t strips, panels, m;
+        int cus;
+        KSplitPlan plan;
+    };
+    static thread_local Kept kept[64] = {};
+    Kept& k = kept[(strips * 0x9E3779B1u ^ panels * 0x85EBCA6Bu ^ m * 0xC2B2AE35u) >> 26];
+    if (k.strips != strips || k.panels != panels || k.m != m || k.cus != g.cus) k = Kept{strips, panels, m, g.cus, ksplit_search(strips, panels, m, 0, 0)};
+    return k.plan;
+}
+
+// Which GEMM entry point for m token rows on a [rows, k_dim] tensor.  Up to 64 rows: the K-split kernels.  Beyond that the
 // launch lasts as long as the fullest compute unit, which takes `rounds` = ceil(blocks / compute units) blocks: one behind the other
 // where a block fills the unit (eight waves, or four that keep most registers), some of them together for m32 / m48 / m64.  Short
 // blocks that deal one 64-row tile's K over four waves (m32) win while there are few; large products go to the blocks whose
@@ -423,6 +557,7 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
 // If none takes it, m32 is named, whose refusal the status reports.
 static const char* gemm_choice(uint32_t rows, uint32_t m, uint32_t k_dim, bool k_known) {
     if (m <= 16) return "gemm_nvfp4_bf16_m16";
+    if (m <= 64) return "gemm_nvfp4_bf16_m32";
     static const struct { const char* name; uint32_t mt, strips; double a, b, c, d, alone, alone_k; } cand[] = {
         {"gemm_nvfp4_bf16_m32", 32, 4, 2.31, 1.46, 0.0, 0.44, 2.43, 0.48},    {"gemm_nvfp4_bf16_m48", 48, 16, 2.03, 6.56, 0.84, 1.81, 1.58, 2.46},
         {"gemm_nvfp4_bf16_m64", 64, 16, 3.03, 5.5, 0.84, 4.96, 1.01, 4.51},   {"gemm_nvfp4_bf16_w48", 48, 32, 3.94, 12.93, 2.54, 1.31, 0.0, 0.0},
@@ -581,8 +716,17 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
     }
     if (strncmp(name, "gemm_nvfp4_bf16", 15) == 0) {  // z = M token rows
         if (k_dim == 0 || k_dim % CROW_BLOCK_VALUES != 0) return CROW_ERR_SHAPE;
-        if (strcmp(name, "gemm_nvfp4_bf16_m16") == 0) {  // one panel per wave where the workspace allows it
-            if (z > 16) return CROW_ERR_SHAPE;
+        const bool m16 = strcmp(name, "gemm_nvfp4_bf16_m16") == 0;
+        if (m16 && z > 16) return CROW_ERR_SHAPE;
+        if ((m16 || strcmp(name, "gemm_nvfp4_bf16_m32") == 0) && z >= 1 && z <= 64 && k_dim < 1u << 25) {
+            const KSplitPlan p = ksplit_plan(strips, panels, z, force_s, force_w);
+            if (p.nj != 0) {
+                const uint32_t tbk = (z + 15) / 16;
+                *out = crow_dims{(strips + p.nj - 1) / p.nj, 1, CROW_KSPLIT | p.slices | (p.nj << 8) | (tbk << 12) | (p.waves << 16), 64u * p.waves};
+                return CROW_OK;
+            }
+        }
+        if (m16) {  // one panel per wave where the workspace allows it
             uint32_t s = (panels + 3) / 4;
             if (s > 16) s = 16;
             while (s > 1 && ((unsigned long long)rt * s * 16 * 64 > PARTIAL_FLOATS || rt > COUNTER_SLOTS)) s--;
@@ -647,6 +791,7 @@ int crow_hip_status(void) {
         (void)hipMemset(g.ws.status, 0, sizeof st);
         // a launch that bailed out may have left arrival counters behind
         (void)hipMemset(g.ws.counters, 0, COUNTER_WORDS * sizeof(unsigned));
+        for (const crow::Workspace& m : g.ws_more) (void)hipMemset(m.counters, 0, COUNTER_WORDS * sizeof(unsigned));
     }
     if (st2 != 0) (void)hipMemset(g.ws_static.counters, 0, (NOALLOC_COUNTER_SLOTS + NOALLOC_TAIL_WORDS) * sizeof(unsigned));  // counters, status, key
     st |= st2;
@@ -663,6 +808,8 @@ int crow_hip_reset_workspace(void) {
     // arrival counters and the status word of both scratch areas (the head's keys need no clearing: every launch overwrites
     // the words it reads)
     if ((e = hipMemset(g.ws_static.counters, 0, (NOALLOC_COUNTER_SLOTS + 32) * sizeof(unsigned))) != hipSuccess) return (int)e;
+    for (const crow::Workspace& m : g.ws_more)
+        if ((e = hipMemset(m.counters, 0, COUNTER_WORDS * sizeof(unsigned))) != hipSuccess) return (int)e;
     return hip_rc(hipMemset(g.ws.counters, 0, COUNTER_WORDS * sizeof(unsigned)));
 }
 
@@ -724,7 +871,7 @@ int crow_hip_time_launches(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, u
     if ((rc = hipEventCreate(&b)) != hipSuccess) return (int)rc;
     int out = hip_rc(hipEventRecord(a, g.stream));
     for (uint32_t i = 0; i < iters && out == CROW_OK; i++)
-        out = launch_entry(e, dim3(gx, gy, gz), dim3(bx), vals + (size_t)(i % n_sets) * n_vals, n_vals, g.stream, g.ws);
+        out = launch_on(e, dim3(gx, gy, gz), dim3(bx), vals + (size_t)(i % n_sets) * n_vals, n_vals, g.stream);
     if (out == CROW_OK) out = hip_rc(hipEventRecord(b, g.stream));
     if (out == CROW_OK) out = hip_rc(hipEventSynchronize(b));
     float ms = 0.0f;
@@ -753,7 +900,7 @@ int crow_hip_time_sequence(uint32_t n_kernels, const crow_fn_t* fns, const crow_
     for (uint32_t i = 0; i < iters && out == CROW_OK; i++) {
         const uint64_t* v = vals + (size_t)(i % n_sets) * per_set;
         for (uint32_t k = 0; k < n_kernels && out == CROW_OK; k++) {
-            out = launch_entry((const FnEntry*)(void*)fns[k], dim3(dims[k].gx, dims[k].gy, dims[k].gz), dim3(dims[k].bx), v, n_vals[k], g.stream, g.ws);
+            out = launch_on((const FnEntry*)(void*)fns[k], dim3(dims[k].gx, dims[k].gy, dims[k].gz), dim3(dims[k].bx), v, n_vals[k], g.stream);
             v += n_vals[k];
         }
     }
@@ -900,7 +1047,7 @@ static int layout_launch(const char* name, const void* a, const void* b, const v
     if (c) vals[n++] = (uint64_t)c;
     vals[n++] = (uint64_t)sc;
     vals[n++] = (uint64_t)(sc + 1);
-    rc = launch_entry(find(name), dim3(d.gx, d.gy, d.gz), dim3(d.bx), vals, n, g.stream, g.ws);
+    rc = launch_on(find(name), dim3(d.gx, d.gy, d.gz), dim3(d.bx), vals, n, g.stream);
     if (rc != CROW_OK) return rc;
     // A kernel puts both status words into pinned memory (two copies to pageable memory take longer); what they say when one is
     // raised is crow_hip_status's to report.  It must run when every stream is idle, as crow_hip_status reads them: behind a wait for the

@@ -591,6 +591,211 @@ struct TallTile {
     }
 };
 
+
+// K-split body: up to 64 token rows, where the weights are a large part of the time.  A block is NJ adjacent strips and ONE token block
+// of MT = 16 TBK rows; its W waves divide the 256-column panels among themselves (and, if a tensor has too few strips for the
+// device, the S blocks of the grid's third dimension as well), each wave in runs of whole panels, and add their tiles through
+// LDS (slices: in slice order through the workspace).  Nothing is shared before that, so there is no barrier in the loop.
+//   * A decoded operand serves TBK matrix instructions only, and decoding it takes 17 vector instructions, so the instructions issued are a
+//     bound beside the memory: 5.6 us of them for [17408, 5120] at 16 tokens if every SIMD always finds one.  A wave that has a SIMD to
+//     itself issues a vector instruction every 8 cycles, two waves one every 4: eight to twelve waves per compute unit, in one round of blocks.
+//   * The activations are read by every block: 160 KB at 16 tokens and K = 5120, as much as the block's weights with NJ = 4.  More strips per
+//     block is less of that, and a chunk's operand reads from LDS serve all NJ strips.
+//   * vmcnt counts in order: what a wave waits for includes all it requested before.  Per panel the activations of the next one are
+//     requested first and its weights last, so that a wait for a chunk of activations never includes a load from memory that
+//     was requested less than a panel ago.
+// Measured ([17408, 5120], us; m16 / m32 before): 16 tokens 14.5 to 15.4 (18.5), 32 18.0 (24.7), 48 21.9 (35.0), 64 24.7 (36.8);
+// [4096, 4096]: 16 tokens 6.3 (8.8), 64 10.8 (14.4); [1024, 8192] x 64 9.9 (22.8).
+template <int TBK, int NJ>
+struct KSplitTile {
+    static constexpr int MT = 16 * TBK;
+    static constexpr int SEGS = TBK == 1 ? 8 : (TBK == 2 ? 4 : 2);  // 32-column segments per staged chunk of X: 32 registers of it at most
+    static constexpr int XCH = TBK * SEGS;                         // 16-byte pieces of a chunk per lane
+    static constexpr int PPR = SEGS * 4;                           // pieces per token row
+    static constexpr int STRIDE = SEGS * 64 + 16;                  // bytes per staged row: eight rows 16 bytes apart modulo the bank cycle
+    // LDS per wave: a chunk, and afterwards one token block's sums
+    static constexpr int AREA = MT * STRIDE > NJ * 1024 ? MT * STRIDE : NJ * 1024;
+    unsigned sc[NJ], even[NJ], odd[NJ];
+    u32x4 cd[NJ][2];
+    u32x4 xv[XCH];
+    // One token block: a panel's sums start from zero and are added behind its last instruction (four additions per strip and panel),
+    // which keeps the error of the long walks of few waves below that of one panel per wave over many slices ([17408, 5120] x 16
+    // against 64 bits: 6.9e-8; 9.0e-8 with one running sum; m16 7.4e-8).  More token blocks: m32's four walks are longer than these.
+    static constexpr bool BY_PANEL = TBK == 1;
+    f32x4 acc[TBK][NJ], total[BY_PANEL ? NJ : 1];
+    const unsigned char* wp[NJ];  // the wave's first group of each strip
+    unsigned rowoff[XCH];         // element offsets of this lane's rows of X, from the block's first token row (K < 2^25: 32 bits do)
+    const unsigned short* x;      // the block's first token row
+    int k_dim, lane, xq, count;
+    lds_p stage;
+
+    // panel p of the wave's run; behind the last one every lane asks for the same word of the first, never used (an address and not a
+    // branch, so that the loads in flight are the same on every path)
+    __device__ __forceinline__ void load_w(int p) {
+        const size_t at = p < count ? (size_t)p * CROW_GROUP_BYTES : 0;
+        const int l = p < count ? lane : 0;
+#pragma unroll
+        for (int J = 0; J < NJ; J++) {
+            const unsigned char* q = wp[J] + at;
+            sc[J] = stream_load_u32((const unsigned*)q + l);
+            cd[J][0] = stream_load_v((const uint4*)(q + CROW_GROUP_SCALE_BYTES) + l);
+            cd[J][1] = stream_load_v((const uint4*)(q + CROW_GROUP_SCALE_BYTES + 1024) + l);
+        }
+    }
+    // chunk c of panel p of the tensor; columns beyond K meet zero weights, but must not be NaN: their lanes read a word of zeros
+    __device__ __forceinline__ void load_x(int p, int c) {
+        const int col = p * CROW_PANEL_COLS + c * SEGS * 32 + xq;
+        const bool in = col < k_dim;
+        const unsigned short* from = in ? x : (const unsigned short*)gemm_zeros.words;
+        const unsigned mask = in ? ~0u : 0u, at = in ? (unsigned)col : 0u;
+#pragma unroll
+        for (int i = 0; i < XCH; i++) xv[i] = *(const __attribute__((address_space(1))) u32x4*)(from + (size_t)((rowoff[i] & mask) + at));
+    }
+    __device__ __forceinline__ void store_x() {
+#pragma unroll
+        for (int i = 0; i < XCH; i++) {
+            const int c = i * 64 + lane, r = c / PPR, q = c % PPR;
+            *(__attribute__((address_space(3))) u32x4*)(stage + r * STRIDE + q * 16) = xv[i];
+        }
+        __builtin_amdgcn_wave_barrier();  // (the wave's LDS accesses execute in order: this only keeps the compiler from reordering them)
+    }
+    template <int S>
+    __device__ __forceinline__ void segments(int p) {
+        if constexpr (S < 8) {
+            if constexpr (S % SEGS == 0) {
+                store_x();
+                if constexpr (S + SEGS < 8) load_x(p, S / SEGS + 1);
+                else load_x(p + 1, 0);
+            }
+            typedef __attribute__((address_space(3))) const u32x4* lds_v4;
+            const lds_p at = stage + (lane & 15) * STRIDE + (lane >> 4) * 16 + (S % SEGS) * 64;
+            bf16x8 A[TBK];
+#pragma unroll
+            for (int tb = 0; tb < TBK; tb++) A[tb] = __builtin_bit_cast(bf16x8, *(lds_v4)(at + tb * 16 * STRIDE));
+#pragma unroll
+            for (int J = 0; J < NJ; J++) {
+                const u32x4 q = cd[J][S >> 2];
+                const unsigned codes = (S & 3) == 0 ? q.x : ((S & 3) == 1 ? q.y : ((S & 3) == 2 ? q.z : q.w));
+                const bf16x8 B = decode8_scaled(codes, e4m3_to_f32<(S >> 1)>((S & 1) ? odd[J] : even[J]));
+#pragma unroll
+                for (int tb = 0; tb < TBK; tb++) acc[tb][J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B, A[tb], acc[tb][J], 0, 0, 0);
+            }
+            if constexpr (S % SEGS == SEGS - 1) __builtin_amdgcn_wave_barrier();  // the chunk is read before the next one overwrites it
+            segments<S + 1>(p);
+        }
+    }
+
+    __device__ __forceinline__ void run(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x_, const float* __restrict__ gs_ptr,
+                                        float* __restrict__ y, int k_dim_, int rows, int m_total, lds_p lds, const Workspace& ws) {
+        lane = lane_id();
+        k_dim = k_dim_;
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = block_threads() >> 6;
+        const int strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS, panels = (k_dim + CROW_PANEL_COLS - 1) / CROW_PANEL_COLS;
+        const int strip0 = (int)blockIdx.x * NJ, m0 = (int)blockIdx.y * MT;
+        if (strip0 >= strips || m0 >= m_total) return;  // a grid larger than the problem: the whole block leaves
+        // the panels in runs of floor(panels / units), the first ones one longer
+        const int slice = (int)blockIdx.z, slices = (int)gridDim.z, units = slices * waves, unit = slice * waves + wave;
+        const int base = panels / units, rem = panels - base * units, first = unit * base + (unit < rem ? unit : rem);
+        count = base + (unit < rem ? 1 : 0);
+        stage = lds + wave * AREA;
+#pragma unroll
+        for (int J = 0; J < NJ; J++)  // strips beyond the tensor re-read the last one (their rows are never stored)
+            wp[J] = w + ((size_t)(strip0 + J < strips ? strip0 + J : strips - 1) * panels + first) * CROW_GROUP_BYTES;
+        const int mlast = m_total - m0 - 1;  // rows beyond M read row M - 1 (never stored)
+#pragma unroll
+        for (int i = 0; i < XCH; i++) {
+            const int r = (i * 64 + lane) / PPR;
+            rowoff[i] = (unsigned)(r < mlast ? r : mlast) * (unsigned)k_dim;
+        }
+        xq = (lane % PPR) * 8;
+        x = x_ + (size_t)m0 * k_dim;
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < (BY_PANEL ? NJ : 1); j++) total[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (count > 0) {  // wave-uniform
+            load_x(first, 0);
+            load_w(0);
+            for (int p = 0; p < count; p++) {
+#pragma unroll
+                for (int J = 0; J < NJ; J++) {  // both segments' scale words of every pair, as in TileScales
+                    const u32x2 sw = __builtin_amdgcn_permlane16_swap(sc[J], sc[J], false, false);
+                    even[J] = sw.x;
+                    odd[J] = sw.y;
+                }
+                segments<0>(first + p);
+                __builtin_amdgcn_sched_barrier(0);
+                load_w(p + 1);
+                if constexpr (BY_PANEL) {
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+                        total[j] += acc[0][j];
+                        acc[0][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                }
+            }
+        }
+        if constexpr (BY_PANEL) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[0][j] = total[j];
+        }
+        // the waves' tiles, one token block of 16 rows at a time: wave j < NJ adds strip j's, by fours (in pairs), the fours in order
+        typedef __attribute__((address_space(3))) f32x4* lds_f4;
+        f32x4 v[TBK];
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++) {
+            if (tb > 0) __syncthreads();
+#pragma unroll
+            for (int j = 0; j < NJ; j++) *(lds_f4)(stage + j * 1024 + lane * 16) = acc[tb][j];
+            __syncthreads();
+            if (wave < NJ) {
+                for (int w0 = 0; w0 < waves; w0 += 4) {
+                    f32x4 t[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        t[i] = *(lds_f4)(lds + (w0 + i < waves ? w0 + i : 0) * AREA + wave * 1024 + lane * 16);
+                        if (w0 + i >= waves) t[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                    const f32x4 four = (t[0] + t[1]) + (t[2] + t[3]);
+                    v[tb] = w0 == 0 ? four : v[tb] + four;
+                }
+            }
+        }
+        if (wave >= NJ) return;
+        if (slices > 1) {
+            float q[4 * TBK];
+#pragma unroll
+            for (int tb = 0; tb < TBK; tb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) q[4 * tb + r] = v[tb][r];
+            if (!slice_hand_over<4 * TBK>(q, ((unsigned)blockIdx.y * gridDim.x + blockIdx.x) * NJ + wave, slice, slices, ws, lane)) return;
+#pragma unroll
+            for (int tb = 0; tb < TBK; tb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[tb][r] = q[4 * tb + r];
+        }
+        // v[tb][r] of lane (g, n): weight row 4 g + r of the strip, token m0 + 16 tb + n
+        const float gs = gs_ptr[0];
+        const int col = (strip0 + wave) * CROW_STRIP_ROWS + 4 * (lane >> 4);
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++) {
+            const int m = m0 + 16 * tb + (lane & 15);
+            if (m >= m_total) continue;
+            const f32x4 o = v[tb] * gs;
+            float* to = y + (size_t)m * rows + col;
+            if (col + 3 < rows) {
+                *(f32x4_dword*)to = o;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (col + r < rows) to[r] = o[r];
+            }
+        }
+    }
+};
+
 }  // namespace crow
 
 // Y[M][rows] f32 = X[M][k_dim] bf16 times the tiled NVFP4 tensor, times gs.  The argument list is
@@ -675,3 +880,24 @@ CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w96, 6)
 CROW_GEMM_TALL_ENTRY(gemm_nvfp4_bf16_t64, 4, 5)
 CROW_GEMM_TALL_ENTRY(gemm_nvfp4_bf16_t96, 6, 5)
 CROW_GEMM_TALL_ENTRY(gemm_nvfp4_bf16_t128, 8, 5)
+// The K-split body, which the launcher starts in the place of gemm_nvfp4_bf16_m16 / _m32 when the launch dimensions say so
+// (crow_hip_launch_dims): grid (ceil(strips / NJ), ceil(M / MT), slices), block of W >= NJ waves, MT = 16 TBK tokens; dynamic LDS = AREA
+// bytes per wave.  `waves` and the scratch memory come from the launcher.
+#define CROW_GEMM_KSPLIT_ENTRY(TBK, NJ, MT, WAVES)                                                                             \
+    extern "C" __global__ void __launch_bounds__(64 * WAVES) gemm_ksplit_##MT##x##NJ(                                           \
+        const unsigned char* __restrict__ w, const unsigned short* __restrict__ x, const float* __restrict__ gs_ptr,           \
+        float* __restrict__ y, const int* __restrict__ k_dim_p, const int* __restrict__ rows_p, const int* __restrict__ m_p, int waves, const Workspace ws) { \
+        static_assert(MT == 16 * TBK, "the name says the token rows of a block");                                              \
+        if (block_threads() != 64 * waves || waves < 2 || waves < NJ || *m_p < 1 || *m_p > MT * (int)gridDim.y || (unsigned)*k_dim_p >= 1u << 25) { \
+            if (threadIdx.x == 0) atomicOr(ws.status, crow::STATUS_BAD_SHAPE);                                                 \
+            return;                                                                                                            \
+        }                                                                                                                      \
+        crow::KSplitTile<TBK, NJ> t;                                                                                           \
+        t.run(w, x, gs_ptr, y, *k_dim_p, *rows_p, *m_p, LDS, ws);                                                              \
+    }
+#define CROW_GEMM_KSPLIT_ALL(E)                                                                    \
+    E(1, 1, 16, 12) E(1, 2, 16, 12) E(1, 3, 16, 12) E(1, 4, 16, 12) E(1, 5, 16, 12)                \
+    E(2, 1, 32, 12) E(2, 2, 32, 12) E(2, 3, 32, 12) E(2, 4, 32, 12) E(2, 5, 32, 12)                \
+    E(3, 1, 48, 12) E(3, 2, 48, 12) E(3, 3, 48, 8) E(3, 4, 48, 8) E(3, 5, 48, 8)                   \
+    E(4, 1, 64, 12) E(4, 2, 64, 8) E(4, 3, 64, 8) E(4, 4, 64, 8) E(4, 5, 64, 8)
+CROW_GEMM_KSPLIT_ALL(CROW_GEMM_KSPLIT_ENTRY)

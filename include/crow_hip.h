@@ -20,7 +20,9 @@
  * crow_kernels.h lists every kernel name with its value list and the reference kernel it stands for.
  *
  * Threading: like the reference engine (one engine thread, one process-global current stream)
- * the library keeps one workspace per process; launches that use it must be ordered on one stream.
+ * the library keeps one workspace per process; launches that use it must be ordered on one stream.  (The null stream and the first
+ * four others that launches go to have one each, until crow_hip_shutdown; beyond them the GEMM does without, the GEMVs share the null
+ * stream's.  A captured graph uses the capturing stream's, wherever it is replayed.)
  */
 #ifndef CROW_HIP_H
 #define CROW_HIP_H

@@ -1057,6 +1057,95 @@ def test_gemm_tall_tiles_at_their_edges(eng, kernel, m, rows, cols):
     assert torch.isnan(y[0]) and torch.isnan(y[1 + m * rows:]).all()
 
 
+def _ksplit(eng, f, x, y, m, rows, cols, tbk, nj, waves, slices, stream=None):
+    """One K-split launch of the kernel for blocks of `nj` strips x 16 `tbk` tokens, whatever the choice would say of this size."""
+    import ctypes as C
+    from crow_nest_amd import lib
+    p = eng.p
+    vals = (C.c_uint64 * 7)(f.w_ptr, x.data_ptr(), f.gs_ptr, y.data_ptr(), p.i32(cols), p.i32(rows), p.i32(m))
+    word = 0x80000000 | slices | nj << 8 | tbk << 12 | waves << 16
+    grid = (-(-(-(-rows // 16)) // nj), -(-m // (16 * tbk)), word, 64 * waves)
+    return lib.lib().crow_hip_launch(eng.k.f("gemm_nvfp4_bf16_m32"), *grid, vals, 7, stream)
+
+
+@pytest.mark.parametrize("tbk", [1, 2, 3, 4])
+@pytest.mark.parametrize("nj", [1, 2, 3, 4, 5])
+def test_gemm_k_split_kernels_at_their_edges(eng, tbk, nj):
+    """Every K-split kernel: a last strip of five rows and strips beyond the tensor, a last panel of 64 columns, one token block and
+    two with a single token in the last; waves with a panel more, one, and none; one slice and three.  All outputs against the CPU path,
+    Y at odd dwords with nothing written outside it."""
+    for case, (m, rows, cols, waves, slices) in enumerate([(16 * tbk - 3, 16 * nj + 5, 320, max(nj, 2), 1), (16 * tbk + 1, 16 * nj + 5, 64 * 37, 8, 1),
+                                                          (16 * tbk, 32 * nj - 16, 64 * 37, 5, 3), (1, 3, 64, 8, 2)]):
+        print(f"m={m} rows={rows} cols={cols} tbk={tbk} nj={nj} waves={waves} slices={slices}", flush=True)
+        w, gs = random_nvfp4(11 * tbk + nj + case, rows, cols), 6.0e-4
+        f = _load(w, rows, cols, gs)
+        xb, xw = _bf16_dev(normal_f32(19, case, m * cols))
+        x, xw = xb.reshape(m, cols).contiguous(), xw.reshape(m, cols)
+        y = torch.full((m * rows + 8,), float("nan"), device="cuda")
+        for _ in range(2):  # (a second launch finds the slices' counters as the first one found them)
+            y[1:1 + m * rows] = float("nan")
+            assert _ksplit(eng, f, x, y[1:], m, rows, cols, tbk, nj, waves, slices) == 0
+            eng.check()
+            got = y[1:1 + m * rows].view(m, rows).cpu().numpy()
+            assert rel_err(got, orc.gemv(w, rows, cols, gs, xw, threads=8), floor_of(got.size)) <= TOL
+            assert gamma_ratio(got, w, rows, cols, gs, xw) <= 1.0
+        assert torch.isnan(y[0]) and torch.isnan(y[1 + m * rows:]).all()
+
+
+def test_gemm_k_split_takes_infinities_where_they_are_and_refuses_other_launch_shapes(eng):
+    """Activations behind the last column and behind the last token row are not multiplied: they may be NaN.  More rows than the
+    grid covers, and another block than the dimensions say, are refused through the status; nothing is written."""
+    rows, cols, m = 37, 320, 18
+    w, gs = random_nvfp4(5, rows, cols), 6.0e-4
+    f = _load(w, rows, cols, gs)
+    xb, xw = _bf16_dev(normal_f32(20, 1, m * cols))
+    pool = torch.full(((m + 40) * cols,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    pool[:m * cols] = xb
+    pool[3 * cols + 7] = float("inf")
+    got = eng.gemm(f, m, pool[:m * cols].view(m, cols)).cpu().numpy()
+    eng.check()
+    assert not np.isfinite(got[3]).any() and np.isfinite(np.delete(got, 3, 0)).all()
+    ref = orc.gemv(w, rows, cols, gs, xw.reshape(m, cols), threads=8)
+    assert rel_err(np.delete(got, 3, 0), np.delete(ref, 3, 0)) <= TOL
+    from crow_nest_amd.kernels import launch_dims, launch_v
+    from crow_nest_amd.lib import CrowHipError
+    p, y = eng.p, torch.full((40, rows), 7.0, device="cuda")
+    gx, gy, gz, bx = launch_dims("gemm_nvfp4_bf16_m32", rows, cols, m)
+    for words, block in (((cols, rows, 40), bx), ((cols, rows, m), bx + 64), ((cols, rows, 0), bx)):
+        launch_v(eng.k.f("gemm_nvfp4_bf16_m32"), gx, gy, gz, block, [f.w_ptr, pool.data_ptr(), f.gs_ptr, y.data_ptr()] + [p.i32(v) for v in words])
+        with pytest.raises(CrowHipError) as ei:
+            eng.check()
+        assert ei.value.code == -7 and bool((y == 7.0).all())
+
+
+def test_gemm_k_split_slices_on_several_streams_at_once(eng):
+    """Split launches that overlap on the null stream and on six others: those that have scratch memory of their own give the split
+    product's bits, the others the unsplit one's."""
+    rows, cols, m = 1024, 8192, 48
+    f = _load(random_nvfp4(6, rows, cols), rows, cols, 6.0e-4)
+    xs = [_bf16_dev(normal_f32(21, i, m * cols))[0].reshape(m, cols).contiguous() for i in range(7)]
+    ys = [torch.empty((m, rows), device="cuda") for _ in range(7)]
+    want = []
+    for x in xs:
+        pair = []
+        for slices in (4, 1):
+            y = torch.empty((m, rows), device="cuda")
+            assert _ksplit(eng, f, x, y, m, rows, cols, 3, 1, 8, slices) == 0
+            pair.append(y)
+        want.append(pair)
+    eng.check()
+    streams = [None] + [torch.cuda.Stream() for _ in range(6)]
+    for r in range(20):
+        for x, y, s in zip(xs, ys, streams):
+            assert _ksplit(eng, f, x, y, m, rows, cols, 3, 1, 8, 4, None if s is None else s.cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(ys[0], want[0][0])
+        for y, (split, whole) in zip(ys, want):
+            assert torch.equal(y, split) or torch.equal(y, whole), r
+            y.fill_(-1.0)
+    eng.check()
+
+
 def test_gemm_m16_full_size_cross_block_split(eng):
     """[17408, 5120] at 16 tokens: the K-split kernel's five column slices meet through the workspace."""
     _gemm_case(eng, 16, 17408, 5120, "gemm_nvfp4_bf16_m16")
