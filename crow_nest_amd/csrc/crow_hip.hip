@@ -485,50 +485,58 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
     return launch_entry(e, dim3(gx, gy, gz), dim3(bx, 1, 1), vals, n_vals, stream ? (hipStream_t)stream : g.stream, g.ws_static, false);
 }
 
-// Waves, strips and column slices of a K-split GEMM block (gemm.h: KSplitTile) for m <= 64 token rows: what the following time is least
-// for, of 1 to 5 strips, 4 / 8 / 12 waves and 1 to 8 slices.  `rounds` of blocks one behind the other, as many of them together on a
+// Token rows, waves, strips and column slices of a K-split GEMM block (gemm.h: KSplitTile) for m token rows: what the following time is least
+// for, of 1 to 5 strips, 4 / 8 / 12 waves, 1 to 8 slices and, beyond 64 rows, 48 or 64 rows a block.  `rounds` of blocks one behind the other, as many of them together on a
 // compute unit as registers and LDS allow; panels per wave and per block; blocks per compute unit.
 //   us = c0 + (slices > 1) (c1 + c2 slices) + rounds (c3 + panels per wave (c4 + c5 strips)) + rounds together panels (c6 strips + c7)
 //        + blocks / compute units (panels (c8 strips + c9) + c10 strips) + c11 waves
-// was fitted to the times of all of them on MI355X at 104 tensors (rows 512 .. 17408, K 512 .. 17408) x 5, 16, 17, 32, 48 and 64 rows;
-// what it picks is 1 to 3 % behind the fastest on average, 28 % at worst, and between 0.99 and 4.4 times as fast as the kernels
-// that served these sizes before (m16, m32, m48, m64): 1.34 (64 rows) to 1.69 times (17 rows) on average.
+// was fitted to the times of all of them on MI355X at 104 tensors (rows 512 .. 17408, K 512 .. 17408) x 5, 16, 17, 32, 48 and 64 rows, and at
+// those for which gemm_choice names m32 x 96 .. 1999 rows; what it picks is 1 to 4 % behind the fastest on average.  Against the kernels
+// that served these sizes before: 1.34 (64 rows) to 1.69 times as fast (17 rows), 1.40 (96 rows) to 1.20 (1999 rows) on average, up to 4.4;
+// never behind by more than the noise of launches of 6 us.
 struct KSplitPlan {
     double us;
-    uint32_t nj, waves, slices;
+    uint32_t tbk, nj, waves, slices;
 };
 static KSplitPlan ksplit_search(uint32_t strips, uint32_t panels, uint32_t m, uint32_t force_s, uint32_t force_w) {
-    static const double coef[4][12] = {{2.452, 1.165, 0.201, 0.72, 0.099, 0.208, 0.028, 0.026, 0.056, 0.007, 0.0, 0.041},
+    static const double coef[6][12] = {{2.452, 1.165, 0.201, 0.72, 0.099, 0.208, 0.028, 0.026, 0.056, 0.007, 0.0, 0.041},
                                        {2.398, 1.281, 0.276, 0.914, 0.291, 0.211, 0.052, 0.036, 0.04, 0.048, 0.024, 0.079},
                                        {2.745, 1.182, 0.383, 0.836, 0.164, 0.373, 0.028, 0.16, 0.049, 0.047, 0.07, 0.106},
-                                       {2.671, 1.108, 0.402, 1.149, 0.307, 0.321, 0.058, 0.147, 0.031, 0.097, 0.098, 0.145}};
+                                       {2.671, 1.108, 0.402, 1.149, 0.307, 0.321, 0.058, 0.147, 0.031, 0.097, 0.098, 0.145},
+                                       {2.341, 0.991, 0.478, 0.925, 0.0, 0.405, 0.029, 0.093, 0.046, 0.101, 0.014, 0.138},   // several token blocks of 48 rows
+                                       {2.082, 0.79, 0.567, 1.506, 0.0, 0.423, 0.046, 0.09, 0.037, 0.155, 0.016, 0.175}};  // ... of 64
     static const unsigned char waves_per_simd[4][CROW_KSPLIT_NJ] = {{7, 5, 4, 4, 3}, {5, 4, 4, 3, 3}, {5, 4, 4, 3, 2}, {4, 3, 3, 2, 2}};  // (their registers)
-    const uint32_t tbk = (m + 15) / 16, cus = g.cus > 0 ? (uint32_t)g.cus : 256u;
-    const double* c = coef[tbk - 1];
-    KSplitPlan best{0.0, 0, 0, 0};
-    for (uint32_t nj = 1; nj <= CROW_KSPLIT_NJ; nj++) {
-        const KSplitEntry& k = g_ksplit[(tbk - 1) * CROW_KSPLIT_NJ + nj - 1];
-        const uint32_t tiles = (strips + nj - 1) / nj;
-        for (uint32_t w = 4; w <= 12; w += 4) {
-            if (w > (uint32_t)k.max_waves || w < nj || (force_w > 0 && w != force_w)) continue;
-            uint32_t fit = 4u * waves_per_simd[tbk - 1][nj - 1] / w;
-            const uint32_t by_lds = 163840u / (w * (uint32_t)k.lds_per_wave);
-            if (fit > by_lds) fit = by_lds;
-            if (fit < 1) fit = 1;
-            for (uint32_t s = 1; s <= 8; s += s < 4 ? 1 : 2) {
-                if (force_s > 0 && s != force_s) continue;
-                if (s > 1 && ((s - 1) * w >= panels || (unsigned long long)tiles * nj * s * 256ull * tbk > PARTIAL_FLOATS || (unsigned long long)tiles * nj > COUNTER_SLOTS)) continue;
-                const uint32_t blocks = tiles * s, n = (blocks + cus - 1) / cus, rounds = (n + fit - 1) / fit, together = n < fit ? n : fit;
-                const double own = (double)((panels + w * s - 1) / (w * s)), all = (double)panels / s, f = (double)blocks / cus, r = rounds;
-                const double us = c[0] + (s > 1 ? c[1] + c[2] * s : 0.0) + r * (c[3] + own * (c[4] + c[5] * nj)) + r * together * all * (c[6] * nj + c[7]) +
-                                  f * (all * (c[8] * nj + c[9]) + c[10] * nj) + c[11] * w;
-                if (best.nj == 0 || us < best.us) best = KSplitPlan{us, nj, w, s};
+    const uint32_t cus = g.cus > 0 ? (uint32_t)g.cus : 256u;
+    KSplitPlan best{0.0, 0, 0, 0, 0};
+    for (uint32_t tbk = m <= 64 ? (m + 15) / 16 : 3; tbk <= (m <= 64 ? (m + 15) / 16 : 4); tbk++) {
+        for (uint32_t nj = 1; nj <= CROW_KSPLIT_NJ; nj++) {
+            const double* c = coef[m <= 64 ? tbk - 1 : tbk + 1];
+            const KSplitEntry& k = g_ksplit[(tbk - 1) * CROW_KSPLIT_NJ + nj - 1];
+            const uint32_t token_blocks = (m + 16 * tbk - 1) / (16 * tbk);
+            const unsigned long long all_tiles = (unsigned long long)((strips + nj - 1) / nj) * token_blocks;
+            if (all_tiles > 0x0FFFFFFFull) continue;
+            const uint32_t tiles = (uint32_t)all_tiles;
+            for (uint32_t w = 4; w <= 12; w += 4) {
+                if (w > (uint32_t)k.max_waves || w < nj || (force_w > 0 && w != force_w)) continue;
+                uint32_t fit = 4u * waves_per_simd[tbk - 1][nj - 1] / w;
+                const uint32_t by_lds = 163840u / (w * (uint32_t)k.lds_per_wave);
+                if (fit > by_lds) fit = by_lds;
+                if (fit < 1) fit = 1;
+                for (uint32_t s = 1; s <= 8; s += s < 4 ? 1 : 2) {
+                    if (force_s > 0 && s != force_s) continue;
+                    if (s > 1 && ((s - 1) * w >= panels || (unsigned long long)tiles * nj * s * 256ull * tbk > PARTIAL_FLOATS || (unsigned long long)tiles * nj > COUNTER_SLOTS)) continue;
+                    const uint32_t blocks = tiles * s, n = (blocks + cus - 1) / cus, rounds = (n + fit - 1) / fit, together = n < fit ? n : fit;
+                    const double own = (double)((panels + w * s - 1) / (w * s)), all = (double)panels / s, f = (double)blocks / cus, r = rounds;
+                    const double us = c[0] + (s > 1 ? c[1] + c[2] * s : 0.0) + r * (c[3] + own * (c[4] + c[5] * nj)) + r * together * all * (c[6] * nj + c[7]) +
+                                      f * (all * (c[8] * nj + c[9]) + c[10] * nj) + c[11] * w;
+                    if (best.nj == 0 || us < best.us) best = KSplitPlan{us, tbk, nj, w, s};
+                }
             }
         }
     }
     return best;
 }
-// The search takes 0.5 us, a tenth of a small call: each thread keeps what it found for the last shapes (a program has a few dozen).
+// The search takes 0.5 to 1 us, a tenth of a small call: each thread keeps what it found for the last shapes (a program has a few dozen).
 static KSplitPlan ksplit_plan(uint32_t strips, uint32_t panels, uint32_t m, uint32_t force_s, uint32_t force_w) {
     if (force_s != 0 || force_w != 0) return ksplit_search(strips, panels, m, force_s, force_w);
     struct Kept {
@@ -718,11 +726,10 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         if (k_dim == 0 || k_dim % CROW_BLOCK_VALUES != 0) return CROW_ERR_SHAPE;
         const bool m16 = strcmp(name, "gemm_nvfp4_bf16_m16") == 0;
         if (m16 && z > 16) return CROW_ERR_SHAPE;
-        if ((m16 || strcmp(name, "gemm_nvfp4_bf16_m32") == 0) && z >= 1 && z <= 64 && k_dim < 1u << 25) {
+        if ((m16 || strcmp(name, "gemm_nvfp4_bf16_m32") == 0) && z >= 1 && z <= 48u * 65535u && k_dim < 1u << 25 && (unsigned long long)z * k_dim <= 0xffffffffull) {
             const KSplitPlan p = ksplit_plan(strips, panels, z, force_s, force_w);
             if (p.nj != 0) {
-                const uint32_t tbk = (z + 15) / 16;
-                *out = crow_dims{(strips + p.nj - 1) / p.nj, 1, CROW_KSPLIT | p.slices | (p.nj << 8) | (tbk << 12) | (p.waves << 16), 64u * p.waves};
+                *out = crow_dims{(strips + p.nj - 1) / p.nj, (z + 16 * p.tbk - 1) / (16 * p.tbk), CROW_KSPLIT | p.slices | (p.nj << 8) | (p.tbk << 12) | (p.waves << 16), 64u * p.waves};
                 return CROW_OK;
             }
         }

@@ -592,7 +592,7 @@ struct TallTile {
 };
 
 
-// K-split body: up to 64 token rows, where the weights are a large part of the time.  A block is NJ adjacent strips and ONE token block
+// K-split body: up to 64 token rows, and as many as there are where a tensor of few strips leaves the larger tiles' blocks fewer than compute units.  A block is NJ adjacent strips and ONE token block
 // of MT = 16 TBK rows; its W waves divide the 256-column panels among themselves (and, if a tensor has too few strips for the
 // device, the S blocks of the grid's third dimension as well), each wave in runs of whole panels, and add their tiles through
 // LDS (slices: in slice order through the workspace).  Nothing is shared before that, so there is no barrier in the loop.
@@ -605,7 +605,7 @@ struct TallTile {
 //     requested first and its weights last, so that a wait for a chunk of activations never includes a load from memory that
 //     was requested less than a panel ago.
 // Measured ([17408, 5120], us; m16 / m32 before): 16 tokens 14.5 to 15.4 (18.5), 32 18.0 (24.7), 48 21.9 (35.0), 64 24.7 (36.8);
-// [4096, 4096]: 16 tokens 6.3 (8.8), 64 10.8 (14.4); [1024, 8192] x 64 9.9 (22.8).
+// [4096, 4096]: 16 tokens 6.3 (8.8), 64 10.8 (14.4); [1024, 8192] x 64 9.9 (22.8); [5120, 17408] x 128 38.6 (67.8), x 256 62.6 (103); [1024, 5120] x 256 11.6 (16.2).
 template <int TBK, int NJ>
 struct KSplitTile {
     static constexpr int MT = 16 * TBK;

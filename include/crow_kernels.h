@@ -96,8 +96,8 @@ CROW_KERNEL(moe_down_grouped, 9)
 /* w, x, gs, y, k_dim_p, rows_p, m_p.  The dense NVFP4 GEMM of kernels_glm5_moe.cu:310-543 (gemm_fp4_dense's list minus
  * the quantised-activation buffer: x is bf16).  gemm_nvfp4_bf16_m16 serves *m_p <= 16 only; the others take any m
  * and differ in tiling (32, 48, 64, 96, 128 tokens per block); crow_hip_gemm_kernel_for names the one to use.  Under the dimensions that
- * crow_hip_launch_dims makes for up to 64 rows, m16 and m32 run in K-split blocks of 16 to 64 tokens and serve up to as many rows as the
- * grid's blocks hold (more: the status). */
+ * crow_hip_launch_dims makes (other grids run as before), m16 and m32 run in K-split blocks of 16 to 64 tokens and serve as many rows as
+ * the grid's blocks hold (more: the status). */
 CROW_KERNEL(gemm_nvfp4_bf16, 7)
 /* the same product in blocks of eight waves (two per SIMD) x 48 / 64 / 80 / 96 tokens */
 CROW_KERNEL(gemm_nvfp4_bf16_w48, 7)
