@@ -32,14 +32,15 @@ struct FnEntry {
     bool takes_geo;  // the launcher appends the model geometry (crow_hip_set_geo) by value, last
     const void* one_stub = nullptr;  // a twin of `stub` with one strip per block, started in its place when S = CROW_ONE_STRIP
     const void* two_stub = nullptr;  // ... and one with two runs of columns per wave, when S = CROW_TWO_RUNS
-    const void* ahead_stub = nullptr;  // unquantised GEMVs: a twin that requests weights alone ahead, when the launch's gz = CROW_KEEP_AHEAD
+    const void* twin_stub = nullptr;  // a twin started when the launch's gz = CROW_TWIN: unquantised GEMVs, weights alone requested ahead; acc_combo, y stored
     bool ksplit = false;  // GEMM for few token rows: one of g_ksplit starts in its place when the launch's gz says which (CROW_KSPLIT)
 };
 // values of S in a launch's `gy` word (GEMV family, K up to 16384; a strip of at most 64 groups never has that many slices): one
 // slice, and one strip per block where the kernel otherwise takes `ns` of them / two runs of columns per wave of the block
 #define CROW_ONE_STRIP 0x81u
 #define CROW_TWO_RUNS 0x82u
-#define CROW_KEEP_AHEAD 2u  // (the grid of those kernels has no third dimension)
+#define CROW_TWIN 2u  // (the grid of those kernels has no third dimension)
+#define CROW_STORE 0x83u  // moe_down_combine: y is stored, not added to
 // A K-split GEMM in gz: this bit, bits 0..7 the column slices, 8..11 the strips per block, 12..15 the 16-token blocks per block, 16..23
 // the waves per block
 #define CROW_KSPLIT 0x80000000u
@@ -66,6 +67,8 @@ constexpr int checked_nargs(F) {
     {#name, (const void*)&name, checked_nargs<nargs, 0>(&name) + 0 * checked_nargs<nargs, 0>(&twin), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, (const void*)&twin}
 #define CROW_FN_KSPLIT(name, nargs) \
     {#name, (const void*)&name, checked_nargs<nargs, 0>(&name), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, nullptr, true}
+#define CROW_FN_GEO_TWIN(name, nargs, twin) \
+    {#name, (const void*)&name, checked_nargs<nargs, 1>(&name) + 0 * checked_nargs<nargs, 1>(&twin), 0u, 0, 16, 0, 1, false, nullptr, true, nullptr, nullptr, (const void*)&twin}
 #define CROW_FN_GEO(name, nargs) {#name, (const void*)&name, checked_nargs<nargs, 1>(&name), 0u, 0, 16, 0, 1, false, nullptr, true}
 // NR tensors per block, bodies for 1 .. MMAX activation rows, bf16 or f32 activations
 // (the bodies for several rows need more registers than a block of sixteen waves leaves each: they run in blocks of eight)
@@ -90,7 +93,7 @@ const FnEntry g_table[] = {
     {"moe_gate_up_silu_grouped", (const void*)&moe_gate_up_silu_grouped, checked_nargs<11, 2>(&moe_gate_up_silu_grouped) + 0 * checked_nargs<11, 2>(&moe_gate_up_silu_grouped_tile), 0u, 2, 8, crow::crow_gemv_lds_per_wave(4, false), CROW_MULTI_STRIPS, true, (const void*)&moe_gate_up_silu_grouped_tile, false},
     {"moe_down_grouped", (const void*)&moe_down_grouped, checked_nargs<9, 2>(&moe_down_grouped) + 0 * checked_nargs<9, 2>(&moe_down_grouped_tile), 0u, 1, 8, crow::crow_gemv_lds_per_wave(4, false), CROW_MULTI_STRIPS, true, (const void*)&moe_down_grouped_tile, false},
     CROW_FN_GEO(moe_group, 6),
-    CROW_FN_GEO(router_top10, 10), CROW_FN_GEO(silu_mul_combo, 3),  CROW_FN_GEO(acc_combo, 3),
+    CROW_FN_GEO(router_top10, 10), CROW_FN_GEO(silu_mul_combo, 3),  CROW_FN_GEO_TWIN(acc_combo, 3, acc_combo_store),
     CROW_FN(argmax_k, 3),          CROW_FN(dequant_fp4_flat, 4),    CROW_FN(repack_nvfp4, 4),
     CROW_FN(unpack_nvfp4, 4),      CROW_FN(dequant_nvfp4_tiled, 5),
     // shared-X GEMM blocks: two staged X tiles of MT rows x 528 bytes
@@ -230,7 +233,8 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
         } else {
             const bool one = e->one_stub != nullptr && (word >> 24) == CROW_ONE_STRIP && pairs <= 64 * CROW_GROUP_PAIRS;
             const bool two = e->two_stub != nullptr && (word >> 24) == CROW_TWO_RUNS && pairs <= 64 * CROW_GROUP_PAIRS;
-            const int slices = one || two || (word >> 24) == 0 ? 1 : (int)(word >> 24);
+            const bool store = e->stub == (const void*)&moe_down_combine && (word >> 24) == CROW_STORE;
+            const int slices = one || two || store || (word >> 24) == 0 ? 1 : (int)(word >> 24);
             if (one) stub = e->one_stub;
             if (two) stub = e->two_stub;
             lds = (size_t)CROW_GEMV_ZERO_BYTES + (size_t)waves * (size_t)e->lds_per_wave;
@@ -239,6 +243,7 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
                                (unsigned long long)grid.x * grid.z > ws.counter_slots))
                 return CROW_ERR_WORKSPACE;
             geo = (int)(word & 0xFFFFFFu);
+            if (store) geo = pairs | CROW_GEO_STORE;
             grid.y = (unsigned)slices;
         }
         if (lds > g.lds_cap) return CROW_ERR_SHAPE;
@@ -263,8 +268,8 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
         args[na++] = (void*)&geo;
         with_ws = true;
     }
-    if (e->ahead_stub != nullptr && grid.z == CROW_KEEP_AHEAD) {
-        stub = e->ahead_stub;
+    if (e->twin_stub != nullptr && grid.z == CROW_TWIN) {
+        stub = e->twin_stub;
         grid.z = 1;
     }
     if (with_ws) args[na++] = (void*)&ws_arg;
@@ -604,6 +609,8 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
     // m_p / t_p, as the reference's kernels do; the low bits are then the capacity the grid is sized for
     const bool from_memory = (z & CROW_DIMS_COUNT_FROM_MEMORY) != 0 || z == 0;
     z &= ~CROW_DIMS_COUNT_FROM_MEMORY;
+    const bool combine = strcmp(name, "moe_down_combine") == 0 || strcmp(name, "acc_combo") == 0, store = combine && (z & CROW_DIMS_STORE) != 0;
+    if (combine) z &= ~CROW_DIMS_STORE;
     {
         const bool takes_count = strcmp(name, "gemv_nvfp4_wm") == 0 || strcmp(name, "gemv_nvfp4_gum") == 0 || strcmp(name, "gemv_nvfp4_wm_bf16") == 0 ||
                                  strcmp(name, "gemv_nvfp4_gum_bf16") == 0 || strcmp(name, "gemv_fp4_b") == 0 || strcmp(name, "gemv_fp4_b1k") == 0 ||
@@ -630,7 +637,7 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         // up to 256 MB together is ahead by up to 1.4 times: bf16 [10240, 8192] x 16 356 / 290)
         const bool ahead = (z > 1 && (unsigned long long)rows * k_dim * (f32 ? 4 : 2) > (256ull << 20)) ||
                            (!f32 && block_per_row && k_dim >= 4096 && (unsigned long long)rows * z > 768);
-        *out = crow_dims{block_per_row ? rows : (rows + 3) / 4, z, ahead ? CROW_KEEP_AHEAD : 1u, 256};
+        *out = crow_dims{block_per_row ? rows : (rows + 3) / 4, z, ahead ? CROW_TWIN : 1u, 256};
         return CROW_OK;
     }
     if (e->nr != 0) {  // the NVFP4 GEMV family
@@ -643,7 +650,7 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
                             strcmp(name, "gemv_nvfp4_gum_bf16") == 0;
         if (down_combine) {  // rows = hidden; one wave per picked expert, every wave all columns of its strip
             if (g.model.topk < 1 || g.model.topk > 16) return CROW_ERR_GEO;
-            *out = crow_dims{strips, pairs | (1u << 24), z, 64u * (uint32_t)g.model.topk};
+            *out = crow_dims{strips, pairs | ((store ? CROW_STORE : 1u) << 24), z, 64u * (uint32_t)g.model.topk};
             return CROW_OK;
         }
         if (e->tile_stub != nullptr && tile_groups(e->nr, pairs) != 0) {
@@ -772,7 +779,7 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
     if (strcmp(name, "router_top10") == 0) { *out = crow_dims{z, 1, 1, 64}; return CROW_OK; }
     if (strcmp(name, "moe_group") == 0) { *out = crow_dims{1, 1, 1, 1024}; return CROW_OK; }
     if (strcmp(name, "argmax_k") == 0) { *out = crow_dims{1, 1, 1, 1024}; return CROW_OK; }
-    if (strcmp(name, "acc_combo") == 0) { *out = crow_dims{(rows + 255) / 256, z, 1, 256}; return CROW_OK; }  // rows = hidden
+    if (strcmp(name, "acc_combo") == 0) { *out = crow_dims{(rows + 255) / 256, z, store ? CROW_TWIN : 1u, 256}; return CROW_OK; }  // rows = hidden
     if (strcmp(name, "silu_mul_combo") == 0 || strcmp(name, "dequant_fp4_flat") == 0) {  // rows = element count
         *out = crow_dims{(rows + 255) / 256, 1, 1, 256};
         return CROW_OK;

@@ -327,8 +327,10 @@ extern "C" __global__ void __launch_bounds__(1024) moe_gate_up_silu(const unsign
 
 // Fused routed down projection + weighted combine: y[t][row] += sum_j rw[t][j] * (gs * <down_{e(t,j)} row, h[t K + j]>),
 // j ascending, each product and each add rounded on its own - the arithmetic of gemv_fp4_ptrb(down)
-// followed by acc_combo (engine/src/gen.rs:4527-4531, engine/src/kernels.rs:1583-1592) in one launch.
+// followed by acc_combo (engine/src/gen.rs:4527-4531, engine/src/kernels.rs:1583-1592) in one launch.  CROW_GEO_STORE in the geometry
+// word: y = instead of y +=, so that nobody clears it first (a fill is 2.5 us on the device and 4 on the host; the kernel itself 4.7).
 // grid (ceil(H / 16), 1, T), block 64 * topk: wave j of a block takes combo t K + j and ALL columns of its strip.
+#define CROW_GEO_STORE (1 << 20)
 extern "C" __global__ void __launch_bounds__(1024) moe_down_combine(const unsigned long long* __restrict__ ptrs, const float* __restrict__ h,
                                                                     const float* __restrict__ gs_ptr, const float* __restrict__ rw,
                                                                     float* __restrict__ y, const int* __restrict__ k_dim_p,
@@ -337,7 +339,10 @@ extern "C" __global__ void __launch_bounds__(1024) moe_down_combine(const unsign
     const int pairs = geo & 0xFFFFF;
     constexpr int AREA = crow_gemv_lds_per_wave(1, false);
     const int topk = block_threads() >> 6;
+    const bool store = (geo & CROW_GEO_STORE) != 0;
     if (topk != model.topk || topk > 16) {
+        const int row = (int)(blockIdx.x * CROW_STRIP_ROWS + threadIdx.x), rows = *rows_p;
+        if (store && threadIdx.x < CROW_STRIP_ROWS && row < rows) y[(size_t)blockIdx.z * rows + row] = 0.0f;  // refused: what a cleared y would hold
         if (threadIdx.x == 0) atomicOr(ws.status, STATUS_BAD_GEO);
         return;
     }
@@ -356,7 +361,7 @@ extern "C" __global__ void __launch_bounds__(1024) moe_down_combine(const unsign
     const int row = strip * CROW_STRIP_ROWS + lane;
     const bool writer = j == 0 && lane < 16 && row < rows;
     float y_old = 0.0f;
-    if (writer) y_old = y[(size_t)t * rows + row];
+    if (writer && !store) y_old = y[(size_t)t * rows + row];
     const size_t xoff[1] = {0};
     StripWalk<1, false> walk;
     // a routing launch that refused its geometry left zeros behind: no weights to read; the wave still joins the barriers below
@@ -374,11 +379,12 @@ extern "C" __global__ void __launch_bounds__(1024) moe_down_combine(const unsign
     if (!writer) return;
     if (k_word != k) {
         if (lane == 0) atomicOr(ws.status, STATUS_BAD_SHAPE);
+        if (store) y[(size_t)t * rows + row] = 0.0f;
         return;
     }
     float sum = 0.0f;
     for (int q = 0; q < topk; q++) sum = __fadd_rn(sum, ((lds_f)(areas + q * AREA))[lane]);
-    y[(size_t)t * rows + row] = y_old + sum;
+    y[(size_t)t * rows + row] = store ? sum : y_old + sum;
 }
 
 // ------------------------------------------------------------------ routed experts, grouped by expert (batches of many tokens)

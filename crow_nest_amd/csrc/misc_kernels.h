@@ -678,7 +678,9 @@ extern "C" __global__ void silu_mul_combo(const float* __restrict__ h1, float* _
 
 // reference: acc_combo, engine/src/kernels.rs:1583-1592: y[t][c] += sum_j rw[t][j] * x[t K + j][c],
 // j ascending, one rounding per multiply and per add.  grid (ceil(H / 256), T), block 256.
-extern "C" __global__ void acc_combo(const float* __restrict__ x, const float* __restrict__ rw, float* __restrict__ y, const Geo model) {
+// `acc_combo_store` (y = instead of y +=, started in its place when the launch dimensions say so): nobody clears y first.
+template <bool STORE>
+__device__ __forceinline__ void acc_combo_body(const float* __restrict__ x, const float* __restrict__ rw, float* __restrict__ y, const Geo& model) {
     const int H = model.hidden, K = model.topk;
     const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x), t = (int)blockIdx.y;
     if (c >= H) return;
@@ -687,7 +689,14 @@ extern "C" __global__ void acc_combo(const float* __restrict__ x, const float* _
         const float prod = rw[t * K + j] * x[((size_t)t * K + j) * H + c];
         acc = __fadd_rn(acc, prod);
     }
-    y[(size_t)t * H + c] += acc;
+    if (STORE) y[(size_t)t * H + c] = acc;
+    else y[(size_t)t * H + c] += acc;
+}
+extern "C" __global__ void acc_combo(const float* __restrict__ x, const float* __restrict__ rw, float* __restrict__ y, const Geo model) {
+    acc_combo_body<false>(x, rw, y, model);
+}
+extern "C" __global__ void acc_combo_store(const float* __restrict__ x, const float* __restrict__ rw, float* __restrict__ y, const Geo model) {
+    acc_combo_body<true>(x, rw, y, model);
 }
 
 // ------------------------------------------------------------------ greedy argmax

@@ -9,17 +9,18 @@ put the HIP library behind ``gen.rs``:
     verify_ffn    gen.rs:5632-5634   gemv_nvfp4_gum + proj_m(down)
     lm_head_row   gen.rs:4766-4784   lm_head through dense_proj, then argmax_k (gen.rs:6197-6198)
     moe_run       gen.rs:4168-4534   router_top10 -> routed gate|up -> SwiGLU -> routed down -> acc_combo
-Buffers are torch tensors on the device (allocation only); every launch goes through
+Buffers are torch tensors on the device (allocation only; sizes go as plain arguments, which torch parses 0.4 us faster than a tuple); every launch goes through
 ``k.run(name, ...)`` - ``launch_v`` under the library's launch dimensions - with device addresses, like the reference call
 sites.
 """
 from __future__ import annotations
 
 from dataclasses import dataclass
+from functools import lru_cache
 
 import torch
 
-from .kernels import KernelGeo, Kernels, compile, launch_dims, set_geo, status
+from .kernels import STORE, KernelGeo, Kernels, compile, launch_dims, set_geo, status
 from .weights import ExpertSlabs, Fp4, Params
 
 NVFP4_MMAX = 4  # kernels_p2.rs:397
@@ -66,7 +67,7 @@ class Engine:
         rows, k = w.rows, w.cols
         assert x.is_cuda and x.is_contiguous() and x.numel() == t * k
         if y is None:
-            y = torch.empty((t, rows), dtype=torch.float32, device=self.dev)
+            y = torch.empty(t, rows, dtype=torch.float32, device=self.dev)
         p = self.p
         if t == 1 and x.dtype == torch.float32:
             self.k.run("gemv_nvfp4_w", rows, k, 1, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows))
@@ -84,7 +85,7 @@ class Engine:
             raise ValueError(f"proj_m: M = {m} is outside 1..={NVFP4_MMAX}")
         assert x.is_cuda and x.is_contiguous() and x.numel() == m * k
         if y is None:
-            y = torch.empty((m, rows), dtype=torch.float32, device=self.dev)
+            y = torch.empty(m, rows, dtype=torch.float32, device=self.dev)
         name = "gemv_nvfp4_wm" if x.dtype == torch.float32 else "gemv_nvfp4_wm_bf16"
         p = self.p
         self.k.run(name, rows, k, m, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m))
@@ -95,7 +96,7 @@ class Engine:
         inter, k = mlp.gate.rows, mlp.gate.cols
         assert (mlp.up.rows, mlp.up.cols) == (inter, k) and x.numel() == t * k and 1 <= t <= NVFP4_MMAX
         if h is None:
-            h = torch.empty((t, inter), dtype=torch.float32, device=self.dev)
+            h = torch.empty(t, inter, dtype=torch.float32, device=self.dev)
         p = self.p
         if t == 1:
             name = "gemv_nvfp4_gu" if x.dtype == torch.float32 else "gemv_nvfp4_gu_bf16"
@@ -174,24 +175,25 @@ class Engine:
         p = self.p
         assert logits.shape[1] == experts and logits.dtype == torch.float32 and logits.is_contiguous()
         routed = logits.shape[0]
-        ids = torch.empty((routed, topk), dtype=torch.int32, device=self.dev)
-        wts = torch.empty((routed, topk), dtype=torch.float32, device=self.dev)
+        ids = torch.empty(routed, topk, dtype=torch.int32, device=self.dev)
+        wts = torch.empty(routed, topk, dtype=torch.float32, device=self.dev)
         # the grouped kernels look slabs up in the table themselves: no pointers per combo
         self.k.run_at("router_top10", routed, 1, 1, 64, logits.data_ptr(), 0, ids.data_ptr(), wts.data_ptr(), 0, 0, 0, 0, 0, 0)
         combos = t * topk
         max_tiles = min(combos, experts) + combos // 4
+        adds = 0 if y is not None else STORE  # y of the caller's is added to
         if y is None:
-            y = torch.zeros((t, hdim), dtype=torch.float32, device=self.dev)
-        perm = torch.empty((combos,), dtype=torch.int32, device=self.dev)
-        tiles = torch.empty((max_tiles, 4), dtype=torch.int32, device=self.dev)
-        n_tiles = torch.empty((1,), dtype=torch.int32, device=self.dev)  # written by every moe_group, 0 where it refuses
-        h2 = torch.empty((combos, inter), dtype=torch.float32, device=self.dev)
-        eo = torch.empty((combos, hdim), dtype=torch.float32, device=self.dev)
+            y = torch.empty(t, hdim, dtype=torch.float32, device=self.dev)
+        perm = torch.empty(combos, dtype=torch.int32, device=self.dev)
+        tiles = torch.empty(max_tiles, 4, dtype=torch.int32, device=self.dev)
+        n_tiles = torch.empty(1, dtype=torch.int32, device=self.dev)  # written by every moe_group, 0 where it refuses
+        h2 = torch.empty(combos, inter, dtype=torch.float32, device=self.dev)
+        eo = torch.empty(combos, hdim, dtype=torch.float32, device=self.dev)
         table, gs_gu, gs_dn = moe.table.data_ptr(), moe.gate_up.gs.data_ptr(), moe.down.gs.data_ptr()
         self.k.run("moe_group", 1, 64, combos, ids.data_ptr(), p.i32(combos), perm.data_ptr(), tiles.data_ptr(), n_tiles.data_ptr(), p.i32(max_tiles))
         self.k.run("moe_gate_up_silu_grouped", inter, hdim, max_tiles, tiles.data_ptr(), n_tiles.data_ptr(), perm.data_ptr(), table, x.data_ptr(), gs_gu, h2.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter))
         self.k.run("moe_down_grouped", hdim, inter, max_tiles, tiles.data_ptr(), n_tiles.data_ptr(), perm.data_ptr(), table, h2.data_ptr(), gs_dn, eo.data_ptr(), p.i32(inter), p.i32(hdim))
-        self.k.run_at("acc_combo", (hdim + 255) // 256, t, 1, 256, eo.data_ptr(), wts.data_ptr(), y.data_ptr())
+        self.k.run("acc_combo", hdim, inter, adds | t, eo.data_ptr(), wts.data_ptr(), y.data_ptr())
         return ids, wts, y, (perm, tiles, n_tiles)
 
     def moe_run(self, moe: MoeW, x: torch.Tensor, logits: torch.Tensor, fused: bool = True, y: torch.Tensor | None = None):
@@ -205,30 +207,43 @@ class Engine:
         assert hdim == self.geo.hidden and moe.gate_up.rows == 2 * inter and moe.down.rows == hdim
         p = self.p
         combos = t * topk
+        adds = 0 if y is not None else STORE  # y of the caller's is added to
         if y is None:
-            y = torch.zeros((t, hdim), dtype=torch.float32, device=self.dev)
+            y = torch.empty(t, hdim, dtype=torch.float32, device=self.dev)
         gs_gu, gs_dn = moe.gate_up.gs.data_ptr(), moe.down.gs.data_ptr()
-        h2 = torch.empty((combos, inter), dtype=torch.float32, device=self.dev)
         if fused == "route":
             assert logits.shape == (t, self.geo.experts) and logits.dtype == torch.float32 and logits.is_contiguous()
-            ids = torch.empty((t, topk), dtype=torch.int32, device=self.dev)
-            wts = torch.empty((t, topk), dtype=torch.float32, device=self.dev)
-            dn = torch.empty((t, topk), dtype=torch.int64, device=self.dev)  # written by every launch, zeros where it refuses
-            self.k.run("moe_route_gate_up_silu", inter, hdim, combos, logits.data_ptr(), moe.table.data_ptr(), x.data_ptr(), gs_gu, h2.data_ptr(), ids.data_ptr(), wts.data_ptr(), dn.data_ptr(), p.i32(hdim), p.i32(hdim), p.i32(inter))
-            self.k.run("moe_down_combine", hdim, inter, t, dn.data_ptr(), h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim))
+            ids = torch.empty(t, topk, dtype=torch.int32, device=self.dev)
+            wts = torch.empty(t, topk, dtype=torch.float32, device=self.dev)
+            # one allocation: the picked down slabs (written by every launch, zeros where it refuses), then h, 16-byte aligned
+            slabs = (combos + 1 & ~1) * 2
+            scratch = torch.empty(slabs + combos * inter, dtype=torch.float32, device=self.dev)
+            dn = scratch.data_ptr()
+            h2 = dn + 4 * slabs
+            hdim_p, inter_p, wts_ptr = p.i32(hdim), p.i32(inter), wts.data_ptr()
+            self.k.run("moe_route_gate_up_silu", inter, hdim, combos, logits.data_ptr(), moe.table.data_ptr(), x.data_ptr(), gs_gu, h2, ids.data_ptr(), wts_ptr, dn, hdim_p, hdim_p, inter_p)
+            self.k.run("moe_down_combine", hdim, inter, adds | t, dn, h2, gs_dn, wts_ptr, y.data_ptr(), inter_p, hdim_p)
             return ids, wts, y
-        ids, wts, gu, dn = self.router(logits, moe)
+        h2 = torch.empty(combos, inter, dtype=torch.float32, device=self.dev)
         if fused:
-            self.k.run("moe_gate_up_silu", inter, hdim, combos, gu.data_ptr(), x.data_ptr(), gs_gu, h2.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter))
-            self.k.run("moe_down_combine", hdim, inter, t, dn.data_ptr(), h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim))
+            assert logits.shape == (t, self.geo.experts) and logits.dtype == torch.float32 and logits.is_contiguous()
+            ids = torch.empty(t, topk, dtype=torch.int32, device=self.dev)
+            wts = torch.empty(t, topk, dtype=torch.float32, device=self.dev)
+            slabs = torch.zeros(2, combos, dtype=torch.int64, device=self.dev)  # gate|up slabs, then down slabs: zeros where the router refuses
+            gu = slabs.data_ptr()
+            dn = gu + 8 * combos
+            self.k.run_at("router_top10", t, 1, 1, 64, logits.data_ptr(), 0, ids.data_ptr(), wts.data_ptr(), gu, dn, moe.table.data_ptr(), 0, 0, 0)
+            self.k.run("moe_gate_up_silu", inter, hdim, combos, gu, x.data_ptr(), gs_gu, h2.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(inter))
+            self.k.run("moe_down_combine", hdim, inter, adds | t, dn, h2.data_ptr(), gs_dn, wts.data_ptr(), y.data_ptr(), p.i32(inter), p.i32(hdim))
         else:
+            ids, wts, gu, dn = self.router(logits, moe)
             h1 = torch.empty((combos, 2 * inter), dtype=torch.float32, device=self.dev)
             eo = torch.empty((combos, hdim), dtype=torch.float32, device=self.dev)
             self.k.run("gemv_fp4_ptrb", 2 * inter, hdim, combos, gu.data_ptr(), x.data_ptr(), gs_gu, h1.data_ptr(), p.i32(hdim), p.i32(topk), p.i32(hdim), p.i32(2 * inter))
             n = combos * inter
             self.k.run_at("silu_mul_combo", (n + 255) // 256, 1, 1, 256, h1.data_ptr(), h2.data_ptr(), p.i32(n))
             self.k.run("gemv_fp4_ptrb", hdim, inter, combos, dn.data_ptr(), h2.data_ptr(), gs_dn, eo.data_ptr(), p.i32(inter), p.i32(1), p.i32(inter), p.i32(hdim))
-            self.k.run_at("acc_combo", (hdim + 255) // 256, t, 1, 256, eo.data_ptr(), wts.data_ptr(), y.data_ptr())
+            self.k.run("acc_combo", hdim, inter, adds | t, eo.data_ptr(), wts.data_ptr(), y.data_ptr())
         return ids, wts, y
 
     # ------------------------------------------------------------------ BF16 keeps (router, q/k, MTP head)
@@ -253,14 +268,20 @@ class Engine:
         """y[t][rows] = f32 W [rows][k] times f32 x [t][k]: ``gemv_b``, the router projection (engine/src/gen.rs:4182,
         kernels.rs:97-115); its result is router_top10's logits."""
         assert w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and w.is_contiguous()
-        return self._keep_proj("gemv_b", w, t, x, y)
+        rows, k = w.shape
+        assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.numel() == t * k
+        if y is None:
+            y = torch.empty(t, rows, dtype=torch.float32, device=self.dev)
+        p = self.p
+        self.k.run("gemv_b", rows, k, t, w.data_ptr(), x.data_ptr(), y.data_ptr(), p.i32(k), p.i32(rows))
+        return y
 
     def _keep_proj(self, name: str, w: torch.Tensor, t: int, x: torch.Tensor, y: torch.Tensor | None, waves_per_row: int = 0) -> torch.Tensor:
         """waves_per_row: 0 = the library's choice (a block of four waves per row for short tensors), 1 or 4 to force."""
         rows, k = w.shape
         assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.numel() == t * k
         if y is None:
-            y = torch.empty((t, rows), dtype=torch.float32, device=self.dev)
+            y = torch.empty(t, rows, dtype=torch.float32, device=self.dev)
         p = self.p
         vals = (w.data_ptr(), x.data_ptr(), y.data_ptr(), p.i32(k), p.i32(rows))
         if waves_per_row == 0:
@@ -276,13 +297,14 @@ class Engine:
         rows, k = w.rows, w.cols
         assert x.is_cuda and x.is_contiguous() and x.dtype == torch.bfloat16 and x.numel() == m * k
         if y is None:
-            y = torch.empty((m, rows), dtype=torch.float32, device=self.dev)
+            y = torch.empty(m, rows, dtype=torch.float32, device=self.dev)
         name = kernel or gemm_kernel_for(m, rows, k)
         p = self.p
         self.k.run(name, rows, k, m, w.w_ptr, x.data_ptr(), w.gs_ptr, y.data_ptr(), p.i32(k), p.i32(rows), p.i32(m))
         return y
 
 
+@lru_cache(maxsize=4096)  # (a call into the library takes 0.5 us; the answer depends on the sizes and the device alone)
 def gemm_kernel_for(m: int, rows: int = 17408, k: int = 5120) -> str:
     """Which GEMM entry point serves m token rows of a [rows, k] tensor: the library's choice (crow_hip_gemm_kernel_for), which
     weighs how the blocks of each tiling fall on the device's compute units."""

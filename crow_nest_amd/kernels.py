@@ -28,6 +28,8 @@ class KernelMissing(KeyError):
 # crow_hip.h: CROW_DIMS_COUNT_FROM_MEMORY - launch_dims(name, rows, k, COUNT_FROM_MEMORY | capacity): the launch reads its row
 # count from the device word behind m_p / t_p (the reference's convention: a fixed grid, the word rewritten per step)
 COUNT_FROM_MEMORY = 0x80000000
+# CROW_DIMS_STORE - launch_dims("moe_down_combine" / "acc_combo", rows, k, STORE | tokens): y is written, not added to
+STORE = 0x40000000
 
 
 @dataclass(frozen=True)

@@ -119,6 +119,8 @@ int crow_hip_launch_noalloc(crow_fn_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
  * the row count with the caller's device words (a disagreement stores nothing and raises CROW_ERR_SHAPE) - dimensions
  * made for a larger tensor make them read beyond the allocation. */
 #define CROW_DIMS_COUNT_FROM_MEMORY 0x80000000u
+/* z = CROW_DIMS_STORE | tokens, moe_down_combine and acc_combo only: the launch writes y where it otherwise adds to it */
+#define CROW_DIMS_STORE 0x40000000u
 int crow_hip_launch_dims(const char* name, uint32_t rows, uint32_t k_dim, uint32_t z, crow_dims* out);
 /* the GEMM entry point (a name of the kernel table) that serves `m` token rows fastest on a [rows, k_dim] tensor: the choice
  * depends on how the blocks of each tiling fall on this device's compute units, and leaves out an entry point that would

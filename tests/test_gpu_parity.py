@@ -743,6 +743,44 @@ def test_moe_layer_other_geometries_drawn_at_random(eng):
     eng.check()
 
 
+@pytest.mark.parametrize("t", [1, 6, 40])
+def test_routed_layers_write_y_of_their_own_and_add_to_the_callers(eng, t):
+    """Without a y the layer stores its result into memory that nobody cleared (here: full of NaN a moment before), with one it adds:
+    the same bits on top of zeros, one rounding on top of anything else.  A refused launch that stores leaves zeros."""
+    from crow_nest_amd.engine import MoeW, expert_table
+    from crow_nest_amd.kernels import STORE, KernelGeo, launch_dims, launch_v
+    from crow_nest_amd.lib import CrowHipError
+    from crow_nest_amd.weights import load_expert_slabs
+    E, K, H, I = 64, 5, 520 // 8 * 8 + 56, 64
+    eng.set_geo(KernelGeo(experts=E, topk=K, hidden=H, inter=I))
+    try:
+        gs = 1.0e-3
+        s_gu = load_expert_slabs(np.concatenate([random_nvfp4(900 + e, 2 * I, H) for e in range(E)]), E, 2 * I, H, gs)
+        s_dn = load_expert_slabs(np.concatenate([random_nvfp4(990 + e, H, I) for e in range(E)]), E, H, I, gs)
+        moe = MoeW(s_gu, s_dn, expert_table(s_gu, s_dn))
+        x, logits = _dev(normal_f32(31, t, t * H)).view(t, H), _dev(normal_f32(32, t, t * E)).view(t, E)
+        old = torch.randn(t, H, device="cuda")
+        for run in (eng.moe_layer, lambda m, a, b, y=None: eng.moe_run(m, a, b, False, y), lambda m, a, b, y=None: eng.moe_run(m, a, b, True, y)):
+            torch.full((4 * t * H,), float("nan"), device="cuda")  # (freed at once: the next allocation of this size)
+            got = run(moe, x, logits)[2].clone()
+            zeros = run(moe, x, logits, torch.zeros(t, H, device="cuda"))[2]
+            added = run(moe, x, logits, old.clone())[2]
+            eng.check()
+            assert torch.equal(got, zeros) and torch.equal(added, old + got) and bool(got.any())
+        y = torch.full((t, H), 7.0, device="cuda")
+        p, words = eng.p, torch.zeros(t * K, dtype=torch.int64, device="cuda")
+        h, wts = torch.ones(t * K, I, device="cuda"), torch.ones(t, K, device="cuda")
+        gx, gy, gz, bx = launch_dims("moe_down_combine", H, I, STORE | t)
+        for block in (bx, bx + 64):  # no slabs / another number of picks than the geometry's
+            y.fill_(7.0)
+            launch_v(eng.k.f("moe_down_combine"), gx, gy, gz, block, [words.data_ptr(), h.data_ptr(), s_dn.gs.data_ptr(), wts.data_ptr(), y.data_ptr(), p.i32(I), p.i32(H)])
+            with pytest.raises(CrowHipError):
+                eng.check()
+            assert not y.any()
+    finally:
+        eng.set_geo(KernelGeo(experts=256, topk=8, hidden=2048, inter=512))
+
+
 @pytest.mark.parametrize("t", [3, 24, 64])
 def test_moe_layer_grouped_by_expert(eng, t):
     """Batches in which experts repeat: the plan is a stable sort of the combos by expert cut into tiles of at most four,
