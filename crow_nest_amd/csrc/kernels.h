@@ -140,8 +140,10 @@ __device__ __forceinline__ int rows_of(GemvArgs& a, int geo, const int* m_p) {
     return hint;
 }
 // x [M][k_dim] and y [M][rows] in place: the strides are K (by value) and the row count (needed before the first store only)
+// (three waves per SIMD: the widest body took 171 registers, which leaves two; at 168 [17408, 5120] takes 12.7 / 15.4 / 18.8 / 20.4 us at one to
+// four rows, 14.3 / 16.8 / 20.4 / 22.1 before; 128, four waves, spills and is slower from three rows on, and so is the two-tensor kernel at 168)
 // reference: gemv_nvfp4_wm, engine/src/kernels_p2.rs:472-497
-extern "C" __global__ void __launch_bounds__(512) gemv_nvfp4_wm(const unsigned char* __restrict__ w, const float* __restrict__ x,
+extern "C" __global__ void __launch_bounds__(512, 3) gemv_nvfp4_wm(const unsigned char* __restrict__ w, const float* __restrict__ x,
                                                                  const float* __restrict__ gs_ptr, float* __restrict__ y,
                                                                  const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
                                                                  const int* __restrict__ m_p, int geo, const Workspace ws) {
@@ -228,14 +230,14 @@ __device__ __forceinline__ void gemv_tokens(const unsigned char* w, const float*
     }
     gemv_m_dispatch<1, false, EPI_SCALE, CROW_MULTI_STRIPS, RUNS>(a, m, blockIdx.z, LDS, ws);
 }
-extern "C" __global__ void __launch_bounds__(512) gemv_fp4_b(const unsigned char* __restrict__ w, const float* __restrict__ x,
+extern "C" __global__ void __launch_bounds__(512, 3) gemv_fp4_b(const unsigned char* __restrict__ w, const float* __restrict__ x,
                                                               const float* __restrict__ gs_ptr, float* __restrict__ y,
                                                               const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
                                                               const int* __restrict__ t_p, int geo, const Workspace ws) {
     ENTER(w, x, gs_ptr, y, k_dim_p, rows_p, t_p, geo);
     gemv_tokens(w, x, gs_ptr, y, geo, k_dim_p, rows_p, t_p, 0, ws);
 }
-extern "C" __global__ void __launch_bounds__(512) gemv_fp4_b1k(const unsigned char* __restrict__ w, const float* __restrict__ x,
+extern "C" __global__ void __launch_bounds__(512, 3) gemv_fp4_b1k(const unsigned char* __restrict__ w, const float* __restrict__ x,
                                                                 const float* __restrict__ gs_ptr, float* __restrict__ y,
                                                                 const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
                                                                 const int* __restrict__ t_p, int geo, const Workspace ws) {
@@ -256,14 +258,14 @@ extern "C" __global__ void __launch_bounds__(512) gemv_fp4_bs(const unsigned cha
 }
 // The three kernels above with two runs of columns per wave, which the launcher starts in their place when the launch dimensions
 // say so (crow_hip_launch_dims: many token groups of a tensor of few strips).  Same bits: the runs are the same.
-extern "C" __global__ void __launch_bounds__(512) gemv_fp4_b_two(const unsigned char* __restrict__ w, const float* __restrict__ x,
+extern "C" __global__ void __launch_bounds__(512, 3) gemv_fp4_b_two(const unsigned char* __restrict__ w, const float* __restrict__ x,
                                                                   const float* __restrict__ gs_ptr, float* __restrict__ y,
                                                                   const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,
                                                                   const int* __restrict__ t_p, int geo, const Workspace ws) {
     ENTER(w, x, gs_ptr, y, k_dim_p, rows_p, t_p, geo);
     gemv_tokens<2>(w, x, gs_ptr, y, geo, k_dim_p, rows_p, t_p, 0, ws);
 }
-extern "C" __global__ void __launch_bounds__(512) gemv_fp4_bs_two(const unsigned char* __restrict__ w, const float* __restrict__ x,
+extern "C" __global__ void __launch_bounds__(512, 3) gemv_fp4_bs_two(const unsigned char* __restrict__ w, const float* __restrict__ x,
                                                                    const float* __restrict__ gs_ptr, float* __restrict__ y,
                                                                    const int* __restrict__ k_dim_p, const int* __restrict__ y_stride_p,
                                                                    const int* __restrict__ rows_p, const int* __restrict__ t_p, int geo, const Workspace ws) {
