@@ -311,82 +311,6 @@ __device__ __forceinline__ void gemm_pipe_body(const unsigned char* __restrict__
     gemm_store<TBK>(acc, gs_ptr[0], y, rt, m0, rows, m_total, lane);
 }
 
-// Wide shared-X body: a block is EIGHT waves - two per SIMD, so that one wave's operand reads, decode and barrier waits run
-// under the other's matrix instructions (with one wave per SIMD all of them are serial: a 256 x 128 x 256 unit takes 5.6 us
-// against 3.3 us of issue time) - wave w owns row tile 8 * blockIdx.x + w and all of the block's MT = 16 * TBK token rows,
-// staged once in LDS for the eight row tiles.  There is ONE weight register set per wave: the next panel's weights are
-// requested when the current panel's last instruction has read them, and the SIMD's other wave hides the latency; the next
-// X tile travels through registers into the other LDS buffer as in the body above.  One barrier per panel.
-template <int TBK>
-__device__ __forceinline__ void gemm_wide_body(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x,
-                                               const float* __restrict__ gs_ptr, float* __restrict__ y, int k_dim, int rows, int m_total,
-                                               __bf16* xs2) {
-    constexpr int NW = 8;
-    constexpr int MT = 16 * TBK;
-    constexpr int NT = 64 * NW;
-    constexpr int XCH = MT * 32 / NT;  // 16-byte chunks of an X tile per thread
-    static_assert(MT * 32 % NT == 0, "whole chunks per thread");
-    constexpr int XBUF = MT * CROW_GEMM_XS_STRIDE;
-    const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int row_tiles = (rows + CROW_TILE_ROWS - 1) / CROW_TILE_ROWS;
-    const int rt = (int)blockIdx.x * NW + wave;
-    const bool has_rows = rt < row_tiles;  // wave-uniform; idle waves still stage X and join the barriers
-    const int m0 = (int)blockIdx.y * MT;
-    const int panels = (k_dim + CROW_PANEL_COLS - 1) / CROW_PANEL_COLS;
-    f32x4 acc[TBK][4];
-#pragma unroll
-    for (int tb = 0; tb < TBK; tb++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
-    // chunk c = i * 512 + thread: token row c / 32, 8 columns from 8 (c % 32); rows beyond M read row M - 1 (never stored)
-    const int xq = ((int)threadIdx.x & 31) * 8;
-    unsigned xoff[XCH];
-#pragma unroll
-    for (int i = 0; i < XCH; i++) {
-        const int m = m0 + ((i * NT + (int)threadIdx.x) >> 5);
-        xoff[i] = (unsigned)(m < m_total ? m : m_total - 1) * (unsigned)k_dim + (unsigned)xq;
-    }
-    auto load_x = [&](int p, uint4 (&xv)[XCH]) {
-        const int k0 = p * CROW_PANEL_COLS;
-        const bool full = k0 + CROW_PANEL_COLS <= k_dim;  // uniform
-#pragma unroll
-        for (int i = 0; i < XCH; i++) {
-            xv[i] = make_uint4(0, 0, 0, 0);  // (the last, partial panel: columns beyond K are zeros)
-            if (full || k0 + xq < k_dim) xv[i] = *(const uint4*)(x + (size_t)(xoff[i] + (unsigned)k0));
-        }
-    };
-    auto store_x = [&](__bf16* xs, const uint4 (&xv)[XCH]) {
-#pragma unroll
-        for (int i = 0; i < XCH; i++) {
-            const int c = i * NT + (int)threadIdx.x, r = c >> 5, q = c & 31;
-            *(uint4*)(xs + r * CROW_GEMM_XS_STRIDE + q * 8) = xv[i];
-        }
-    };
-    const int lane_off = (lane & 15) * CROW_GEMM_XS_STRIDE + (lane >> 4) * 8;
-    PanelRegs pr;
-    uint4 xv[XCH];
-    load_x(0, xv);
-    load_panel(w, has_rows ? rt : 0, strips, panels, 0, lane, pr);
-    store_x(xs2, xv);
-    __syncthreads();
-    int h = 0;
-    for (int p = 0; p < panels; p++) {
-        const bool more = p + 1 < panels;
-        if (more) load_x(p + 1, xv);
-        gemm_panel<TBK>(pr, xs2 + h * XBUF + lane_off, acc);
-        if (more) {
-            load_panel(w, has_rows ? rt : 0, strips, panels, p + 1, lane, pr);
-            store_x(xs2 + (h ^ 1) * XBUF, xv);
-        }
-        __syncthreads();  // the other buffer is written, and this one read, by every wave
-        h ^= 1;
-    }
-    if (!has_rows) return;
-    gemm_store<TBK>(acc, gs_ptr[0], y, rt, m0, rows, m_total, lane);
-}
-
 // Tall-tile body: a block is FOUR waves, one per SIMD, wave w owning NJ adjacent strips (16 NJ weight rows) and all of the
 // block's MT = 16 TBK token rows, so that one decoded operand feeds TBK matrix instructions and the decode (17 vector
 // instructions a unit) fits under them.  With one wave per SIMD nothing else hides a latency, so the wave's own stream does.
@@ -591,6 +515,182 @@ struct TallTile {
     }
 };
 
+
+// Eight-wave body: the tall tile's stream of units with TWO waves per SIMD (256 registers each): wave w owns NJ = 4 adjacent strips (a 64-row
+// tile; 512 rows a block) and all of the block's MT = 16 TBK token rows.  A lone wave issues a vector instruction every 8 cycles,
+// two waves one every 4, so that a matrix instruction with two of them behind it takes 17 cycles, where the tall tile's takes 22; the price
+// is a decode that serves fewer tokens and half the registers, and a block twice as large.  What differs from the tall tile:
+//   * one set of activation operands: behind the last unit of a segment each one's register takes the next segment's as soon as it is
+//     free (eight matrix instructions of two waves cover an LDS read);
+//   * so the panel's barrier stands before its last unit.
+// Measured (us, the compiler's own order of the same instructions before): w96 [8192, 5120] x 1536 122 -> 112, w80 [17408, 5120] x 512 107 -> 95,
+// w64 [17408, 5120] x 512 180 -> 157, w48 [4096, 4096] x 1000 62 -> 56; with NJ = 3 and 128 tokens 98 / 300 where the tall tile takes 97 / 309
+// ([17408, 5120] x 512 / [5120, 17408] x 1999): not kept.
+template <int TBK>
+struct EightWaveTile {
+    static constexpr int NW = 8, NJ = 4;
+    static constexpr int MT = 16 * TBK;
+    static constexpr int XCH = MT * 32 / (64 * NW);  // 16-byte chunks of an X tile per thread, XROWS token rows apart
+    static constexpr int XROWS = 2 * NW;
+    static constexpr int XBUF = MT * CROW_GEMM_XS_STRIDE;
+    static constexpr int UNITS = 8 * NJ, STORE0 = UNITS - 1 - XCH;  // the first unit that writes a chunk of the next X tile
+    static_assert(MT * 32 % (64 * NW) == 0 && STORE0 > 2 * XCH, "whole chunks per thread, requested well before they are written");
+    unsigned sc[NJ], even[NJ], odd[NJ];
+    uint4 cd[2][NJ];
+    uint4 xv[XCH];
+    bf16x8 A[TBK];
+    u32x4 B[2];
+    f32x4 acc[TBK][NJ];
+    const unsigned char* wp[NJ];
+    unsigned xrow, xlast, kd;  // as in TallTile
+    const unsigned short* x;
+    const __bf16 *cur, *nxt;
+    __bf16* put;
+    f32x2 pair;
+    float scale, low;
+    const unsigned short* from;
+    unsigned at_k, inside;
+    int lane;
+
+    __device__ __forceinline__ void load_scale(int J, int p) { sc[J] = *((const unsigned*)(wp[J] + (size_t)p * CROW_GROUP_BYTES) + lane); }
+    __device__ __forceinline__ void load_codes(int H, int J, int p) {
+        cd[H][J] = *((const uint4*)(wp[J] + (size_t)p * CROW_GROUP_BYTES + CROW_GROUP_SCALE_BYTES + 1024 * H) + lane);
+    }
+    __device__ __forceinline__ void set_scales() {
+#pragma unroll
+        for (int J = 0; J < NJ; J++) {
+            const u32x2 sw = __builtin_amdgcn_permlane16_swap(sc[J], sc[J], false, false);
+            even[J] = sw.x;
+            odd[J] = sw.y;
+        }
+    }
+    __device__ __forceinline__ void load_x(int i) {
+        const unsigned row = xrow + (unsigned)(XROWS * i) * kd;  // rows beyond M read row M - 1 (never stored)
+        const u32x4 v = *(const __attribute__((address_space(1))) u32x4*)(from + (size_t)(((row < xlast ? row : xlast) & inside) + at_k));
+        xv[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    __device__ __forceinline__ void store_x(int i) { *(uint4*)(put + i * XROWS * CROW_GEMM_XS_STRIDE) = xv[i]; }
+    template <int U, int D, int D1>
+    __device__ __forceinline__ void decode() {  // steps D .. D1 - 1 of unit U's eight (TallTile::decode)
+        if constexpr (D < D1) {
+            constexpr int S = U / NJ, J = U % NJ, Q = D / 2;
+            const unsigned codes = u4_get(cd[S >> 2][J], S & 3);
+            if constexpr (D == 0) scale = e4m3_to_f32<(S >> 1)>((S & 1) ? odd[J] : even[J]);
+            if constexpr (D % 2 == 0) {
+                pair = fp4x2_to_f32<Q>(codes);
+                low = pair.x * scale;
+            } else {
+                B[U & 1][Q] = __builtin_amdgcn_perm(__float_as_uint(pair.y * scale), __float_as_uint(low), 0x07060302u);
+            }
+            decode<U, D + 1, D1>();
+        }
+    }
+    template <int U, int T>
+    __device__ __forceinline__ void unit_steps() {
+        if constexpr (T < TBK) {
+            constexpr int J = U % NJ, S = U / NJ;
+            acc[T][J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, B[U & 1]), A[T], acc[T][J], 0, 0, 0);
+            decode<(U + 1) % UNITS, T * 8 / TBK, (T + 1) * 8 / TBK>();
+            if constexpr (J == NJ - 1) A[T] = *(const bf16x8*)((S == 7 ? nxt : cur) + T * 16 * CROW_GEMM_XS_STRIDE + ((S + 1) & 7) * 32);
+            __builtin_amdgcn_sched_barrier(0);
+            unit_steps<U, T + 1>();
+        }
+    }
+    template <int U>
+    __device__ __forceinline__ void units(int pn) {
+        if constexpr (U < UNITS) {
+            constexpr int S = U / NJ, J = U % NJ;
+            if constexpr (U == UNITS - 1) __syncthreads();  // the next X tile is written by every wave; nobody reads this one's any more
+            if constexpr (U < XCH) load_x(U);
+            if constexpr (U >= STORE0 && U < UNITS - 1) store_x(U - STORE0);
+            if constexpr (S == 4) load_scale(J, pn);
+            if constexpr (S == 4) load_codes(0, J, pn);
+            if constexpr (U == UNITS - 1) set_scales();
+            __builtin_amdgcn_sched_barrier(0);
+            unit_steps<U, 0>();
+            units<U + 1>(pn);
+        }
+    }
+
+    // grid (ceil(row tiles / 8), ceil(M / MT))
+    __device__ __forceinline__ void run(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x_, const float* __restrict__ gs_ptr,
+                                        float* __restrict__ y, int k_dim, int rows, int m_total, __bf16* xs2) {
+        lane = lane_id();
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        const int strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
+        const int panels = (k_dim + CROW_PANEL_COLS - 1) / CROW_PANEL_COLS;
+        const int strip0 = ((int)blockIdx.x * NW + wave) * NJ, m0 = (int)blockIdx.y * MT;
+        if ((int)blockIdx.x * NW * NJ >= strips || m0 >= m_total) return;  // a grid larger than the problem: the whole block leaves
+#pragma unroll
+        for (int J = 0; J < NJ; J++)  // strips beyond the tensor re-read the last one (their rows are never stored)
+            wp[J] = w + (size_t)(strip0 + J < strips ? strip0 + J : strips - 1) * panels * CROW_GROUP_BYTES;
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // chunk c = i * 512 + thread: token row c / 32, 8 columns from 8 (c % 32)
+        const int xq = ((int)threadIdx.x & 31) * 8;
+        kd = (unsigned)k_dim;
+        x = x_ + (size_t)m0 * k_dim;
+        xlast = (unsigned)(m_total - m0 < MT ? m_total - m0 - 1 : MT - 1) * kd;
+        xrow = (threadIdx.x >> 5) * kd;
+        auto next_panel = [&](int p, int buf) {  // the X tile that load_x and store_x move
+            const int k = p * CROW_PANEL_COLS + xq;
+            from = k < k_dim ? x : (const unsigned short*)gemm_zeros.words;
+            inside = k < k_dim ? ~0u : 0u;
+            at_k = k < k_dim ? (unsigned)k : 0u;
+            put = xs2 + buf * XBUF + ((int)threadIdx.x >> 5) * CROW_GEMM_XS_STRIDE + xq;
+        };
+        const int lane_off = (lane & 15) * CROW_GEMM_XS_STRIDE + (lane >> 4) * 8;
+        next_panel(0, 0);
+#pragma unroll
+        for (int i = 0; i < XCH; i++) load_x(i);
+#pragma unroll
+        for (int J = 0; J < NJ; J++) {
+            load_scale(J, 0);
+            load_codes(0, J, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < XCH; i++) store_x(i);
+        __syncthreads();
+#pragma unroll
+        for (int tb = 0; tb < TBK; tb++) A[tb] = *(const bf16x8*)(xs2 + lane_off + tb * 16 * CROW_GEMM_XS_STRIDE);
+        set_scales();
+        decode<0, 0, 8>();
+        int h = 0;
+        for (int p = 0; p < panels; p++) {
+            const int pn = p + 1 < panels ? p + 1 : p;  // behind the last panel: requested once more, never used
+            cur = xs2 + h * XBUF + lane_off;
+            h ^= 1;
+            nxt = xs2 + h * XBUF + lane_off;
+            next_panel(pn, h);
+#pragma unroll
+            for (int J = 0; J < NJ; J++) load_codes(1, J, p);
+            units<0>(pn);
+        }
+        // acc[tb][j][r] of lane (g, n): weight row 16 (strip0 + j) + 4 g + r, token m0 + 16 tb + n (as in TallTile)
+        const float gs = gs_ptr[0];
+        const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int col = (strip0 + j) * CROW_STRIP_ROWS + 4 * g;
+#pragma unroll
+            for (int tb = 0; tb < TBK; tb++) {
+                const int m = m0 + 16 * tb + n;
+                const f32x4 v = acc[tb][j] * gs;
+                if (m >= m_total) continue;
+                float* to = y + (size_t)m * rows + col;
+                if (col + 3 < rows) {
+                    *(f32x4_dword*)to = v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < rows) to[r] = v[r];
+                }
+            }
+        }
+    }
+};
 
 // K-split body: up to 64 token rows, and as many as there are where a tensor of few strips leaves the larger tiles' blocks fewer than compute units.  A block is NJ adjacent strips and ONE token block
 // of MT = 16 TBK rows; its W waves divide the 256-column panels among themselves (and, if a tensor has too few strips for the
@@ -846,9 +946,9 @@ CROW_GEMM_PIPE_ENTRY(gemm_nvfp4_bf16_m48, 3, 2)
 CROW_GEMM_PIPE_ENTRY(gemm_nvfp4_bf16_m64, 4, 2)
 CROW_GEMM_PIPE_ENTRY(gemm_nvfp4_bf16_m96, 6, 1)
 CROW_GEMM_PIPE_ENTRY(gemm_nvfp4_bf16, 8, 1)
-// the wide shared-X body: grid (ceil(row_tiles / 8), ceil(M / MT)), block 512, MT = 16 TBK tokens; dynamic LDS = two X tiles
+// the eight-wave body: grid (ceil(row_tiles / 8), ceil(M / MT)), block 512, MT = 16 TBK tokens; dynamic LDS = two X tiles
 #define CROW_GEMM_WIDE_ENTRY(NAME, TBK)                                                                                        \
-    extern "C" __global__ void __launch_bounds__(512, 1) NAME(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x, \
+    extern "C" __global__ void __launch_bounds__(512, 2) NAME(const unsigned char* __restrict__ w, const unsigned short* __restrict__ x, \
                                                          const float* __restrict__ gs_ptr, float* __restrict__ y,              \
                                                          const int* __restrict__ k_dim_p, const int* __restrict__ rows_p,      \
                                                          const int* __restrict__ m_p) {                                        \
@@ -857,7 +957,8 @@ CROW_GEMM_PIPE_ENTRY(gemm_nvfp4_bf16, 8, 1)
             if (threadIdx.x == 0) atomicOr(crow::g_ws.status, crow::STATUS_BAD_SHAPE);                                         \
             return;                                                                                                            \
         }                                                                                                                      \
-        crow::gemm_wide_body<TBK>(w, x, gs_ptr, y, *k_dim_p, *rows_p, *m_p, (__bf16*)crow_dyn_lds);                            \
+        crow::EightWaveTile<TBK> t;                                                                                            \
+        t.run(w, x, gs_ptr, y, *k_dim_p, *rows_p, *m_p, (__bf16*)crow_dyn_lds);                                                \
     }
 CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w48, 3)
 CROW_GEMM_WIDE_ENTRY(gemm_nvfp4_bf16_w64, 4)
