@@ -562,9 +562,11 @@ static KSplitPlan ksplit_plan(uint32_t strips, uint32_t panels, uint32_t m, uint
 // decoded weights serve the most tokens (t64 .. t128, 320 rows each), unless the last round is nearly empty with them and full with
 // others ([8192, 5120] x 1536: w96 has 256 blocks, one round, 114 us; t96 416, two, 140).
 //   us = rounds (a + b K / 1024) + blocks / compute units (c + d K / 1024) + (alone + alone_k K / 1024, one block on a unit)
-// was fitted to every entry point's time on MI355X at 1,122 sizes (rows 512 .. 17408, K 256 .. 17408, 17 .. 1999 tokens) and
-// names one within 3 % of the fastest at all but 9 of them (0.1 % on average); 96- and 128-token blocks of the shared-X body
-// (m96, the general name) are never ahead by more than that and are left to callers by name.
+// was fitted to every entry point's time on MI355X at 1,122 sizes (rows 512 .. 17408, K 256 .. 17408, 17 .. 1999 tokens), the eight-wave ones' again
+// at 770 after their body changed; what it names is 0.6 % behind the fastest of them on average, up to 10 % at K = 256 and 512.  m32's line is that of
+// the body it had alone then; the K-split kernels that its dimensions start now are 1.2 to 1.4 times as fast where it is named, and would win at
+// more sizes (by up to 1.27 times around 128 tokens, [17408, 5120] x 128 50 us against m48's 55), which stay with the kernels that add in one order.
+// 96- and 128-token blocks of the shared-X body (m96, the general name) are never ahead and are left to callers by name.
 // An entry point that would refuse the product is left out: those that address X with 32-bit element offsets from its start (m K up
 // to 2^32 - 1) and count token blocks in the grid's second dimension; the tall tiles count from a block's first token row (K < 2^25).
 // If none takes it, m32 is named, whose refusal the status reports.
@@ -573,9 +575,9 @@ static const char* gemm_choice(uint32_t rows, uint32_t m, uint32_t k_dim, bool k
     if (m <= 64) return "gemm_nvfp4_bf16_m32";
     static const struct { const char* name; uint32_t mt, strips; double a, b, c, d, alone, alone_k; } cand[] = {
         {"gemm_nvfp4_bf16_m32", 32, 4, 2.31, 1.46, 0.0, 0.44, 2.43, 0.48},    {"gemm_nvfp4_bf16_m48", 48, 16, 2.03, 6.56, 0.84, 1.81, 1.58, 2.46},
-        {"gemm_nvfp4_bf16_m64", 64, 16, 3.03, 5.5, 0.84, 4.96, 1.01, 4.51},   {"gemm_nvfp4_bf16_w48", 48, 32, 3.94, 12.93, 2.54, 1.31, 0.0, 0.0},
-        {"gemm_nvfp4_bf16_w64", 64, 32, 3.96, 15.51, 4.16, 1.61, 0.0, 0.0},   {"gemm_nvfp4_bf16_w80", 80, 32, 4.92, 16.17, 3.8, 2.45, 0.0, 0.0},
-        {"gemm_nvfp4_bf16_w96", 96, 32, 6.1, 17.18, 6.18, 3.24, 0.0, 0.0},    {"gemm_nvfp4_bf16_t64", 64, 20, 5.53, 10.69, 1.98, 0.0, 0.0, 0.0},
+        {"gemm_nvfp4_bf16_m64", 64, 16, 3.03, 5.5, 0.84, 4.96, 1.01, 4.51},   {"gemm_nvfp4_bf16_w48", 48, 32, 5.6, 11.58, 1.12, 1.3, 0.0, 0.0},
+        {"gemm_nvfp4_bf16_w64", 64, 32, 6.56, 13.13, 2.63, 1.64, 0.0, 0.0},   {"gemm_nvfp4_bf16_w80", 80, 32, 7.48, 13.91, 3.55, 2.14, 0.0, 0.0},
+        {"gemm_nvfp4_bf16_w96", 96, 32, 8.4, 14.89, 4.77, 2.49, 0.0, 0.0},    {"gemm_nvfp4_bf16_t64", 64, 20, 5.53, 10.69, 1.98, 0.0, 0.0, 0.0},
         {"gemm_nvfp4_bf16_t96", 96, 20, 4.69, 12.31, 5.31, 0.0, 0.0, 0.0},    {"gemm_nvfp4_bf16_t128", 128, 20, 9.56, 12.71, 1.44, 1.72, 0.0, 0.0}};
     const unsigned long long strips = (rows + CROW_STRIP_ROWS - 1) / CROW_STRIP_ROWS;
     const unsigned long long cus = g.cus > 0 ? (unsigned long long)g.cus : 256ull;
