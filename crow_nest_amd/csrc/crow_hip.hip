@@ -34,12 +34,14 @@ struct FnEntry {
     const void* two_stub = nullptr;  // ... and one with two runs of columns per wave, when S = CROW_TWO_RUNS
     const void* twin_stub = nullptr;  // a twin started when the launch's gz = CROW_TWIN: unquantised GEMVs, weights alone requested ahead; acc_combo, y stored
     bool ksplit = false;  // GEMM for few token rows: one of g_ksplit starts in its place when the launch's gz says which (CROW_KSPLIT)
+    const void* rows_stub = nullptr;  // gemv_b: a twin with 4 x 4 rows per wave, when the launch's gz = CROW_ROWS | activation rows
 };
 // values of S in a launch's `gy` word (GEMV family, K up to 16384; a strip of at most 64 groups never has that many slices): one
 // slice, and one strip per block where the kernel otherwise takes `ns` of them / two runs of columns per wave of the block
 #define CROW_ONE_STRIP 0x81u
 #define CROW_TWO_RUNS 0x82u
 #define CROW_TWIN 2u  // (the grid of those kernels has no third dimension)
+#define CROW_ROWS 0x80000000u
 #define CROW_STORE 0x83u  // moe_down_combine: y is stored, not added to
 // A K-split GEMM in gz: this bit, bits 0..7 the column slices, 8..11 the strips per block, 12..15 the 16-token blocks per block, 16..23
 // the waves per block
@@ -63,6 +65,9 @@ constexpr int checked_nargs(F) {
     return NARGS;
 }
 #define CROW_FN(name, nargs) {#name, (const void*)&name, checked_nargs<nargs, 0>(&name), 0u, 0, 16, 0, 1, false, nullptr, false}
+// ... with a twin for several rows of both operands per wave, which is handed the activation row count
+#define CROW_FN_KEEP_ROWS(name, nargs, twin, rows) \
+    {#name, (const void*)&name, checked_nargs<nargs, 0>(&name) + 0 * checked_nargs<nargs, 0>(&twin) + 0 * checked_nargs<nargs, 1>(&rows), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, (const void*)&twin, false, (const void*)&rows}
 #define CROW_FN_KEEP(name, nargs, twin) \
     {#name, (const void*)&name, checked_nargs<nargs, 0>(&name) + 0 * checked_nargs<nargs, 0>(&twin), 0u, 0, 16, 0, 1, false, nullptr, false, nullptr, nullptr, (const void*)&twin}
 #define CROW_FN_KSPLIT(name, nargs) \
@@ -109,7 +114,7 @@ const FnEntry g_table[] = {
     {"gemm_nvfp4_bf16_t96", (const void*)&gemm_nvfp4_bf16_t96, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t96), 2u * 96u * 528u, 0, 4, 0, 1, false},
     {"gemm_nvfp4_bf16_t128", (const void*)&gemm_nvfp4_bf16_t128, checked_nargs<7, 0>(&gemm_nvfp4_bf16_t128), 2u * 128u * 528u, 0, 4, 0, 1, false},
     CROW_FN_KSPLIT(gemm_nvfp4_bf16_m32, 7), CROW_FN_KSPLIT(gemm_nvfp4_bf16_m16, 7), CROW_FN_KEEP(gemv_bf16_w, 5, gemv_bf16_ahead),
-    CROW_FN_KEEP(gemv_bf16, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_bf16_b, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_b, 5, gemv_b_ahead),
+    CROW_FN_KEEP(gemv_bf16, 5, gemv_bf16_ahead), CROW_FN_KEEP(gemv_bf16_b, 5, gemv_bf16_ahead), CROW_FN_KEEP_ROWS(gemv_b, 5, gemv_b_ahead, gemv_b_rows),
     CROW_FN_KEEP(gemv_bf16_ws, 5, gemv_bf16_ws_ahead), CROW_FN_KEEP(gemv_bf16_bs, 6, gemv_bf16_bs_ahead),
     CROW_FN(gemv_nvfp4_w_valu1, 6), CROW_FN(gemv_nvfp4_w_valu2, 6), CROW_FN(gemv_nvfp4_w_valu4, 6),  // measurement only
 };
@@ -271,6 +276,13 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
     if (e->twin_stub != nullptr && grid.z == CROW_TWIN) {
         stub = e->twin_stub;
         grid.z = 1;
+    }
+    if (e->rows_stub != nullptr && (grid.z & CROW_ROWS) != 0) {
+        geo = (int)(grid.z & ~CROW_ROWS);
+        if (geo < 1) return CROW_ERR_BAD_ARGUMENT;
+        stub = e->rows_stub;
+        grid.z = 1;
+        args[na++] = (void*)&geo;
     }
     if (with_ws) args[na++] = (void*)&ws_arg;
     crow::Geo model_arg = g.model;
@@ -639,6 +651,12 @@ int crow_hip_launch_dims_split(const char* name, uint32_t rows, uint32_t k_dim, 
         // up to 256 MB together is ahead by up to 1.4 times: bf16 [10240, 8192] x 16 356 / 290)
         const bool ahead = (z > 1 && (unsigned long long)rows * k_dim * (f32 ? 4 : 2) > (256ull << 20)) ||
                            (!f32 && block_per_row && k_dim >= 4096 && (unsigned long long)rows * z > 768);
+        // 4 x 4 rows per wave pay from about 8192 outputs on (us, a row each / 4 x 4: [256, 2048] x 24 5.0 / 5.7, x 32 5.9 / 5.7, x 64 9.6 / 6.0; [128, 2048] x 64
+        // 5.9 / 5.7; [500, 2048] x 12 5.4 / 5.7, x 17 6.9 / 5.7; [256, 4096] x 64 16.7 / 8.2; [5000, 2048] x 3 18.7 / 9.0, x 500 2804 / 692)
+        if (e->rows_stub != nullptr && force_w == 0 && !ahead && z >= 3 && z <= 0x7FFFFFFFu && (unsigned long long)rows * z >= 8192) {
+            *out = crow_dims{(rows + 15) / 16, (z + 3) / 4, CROW_ROWS | z, 256};
+            return CROW_OK;
+        }
         *out = crow_dims{block_per_row ? rows : (rows + 3) / 4, z, ahead ? CROW_TWIN : 1u, 256};
         return CROW_OK;
     }

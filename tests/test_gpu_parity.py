@@ -1593,6 +1593,22 @@ def test_f32_keep_gemv_router_projection(eng, rows, cols, t):
 
 
 # beyond what the memory-side cache holds from one row to the next, and long bf16 rows a block each: the kernels that request weights alone ahead
+@pytest.mark.parametrize("rows,cols,t", [(2731, 4, 3), (257, 772, 33), (300, 1028, 40), (258, 2048, 64), (2049, 1284, 5)])
+def test_f32_keep_gemv_with_four_rows_of_both_operands_per_wave_keeps_the_bits(eng, rows, cols, t):
+    """The shape chosen from 8192 outputs on: the same bits as one wave per (row, token), at partial blocks of weight and activation
+    rows, at K of one lane and of a partial trip; nothing written outside y."""
+    from crow_nest_amd.kernels import launch_dims
+    dims = launch_dims("gemv_b", rows, cols, t)
+    assert dims == (-(-rows // 16), -(-t // 4), 0x80000000 | t, 256)
+    wd = torch.from_numpy(normal_f32(81, rows, rows * cols).reshape(rows, cols)).cuda()
+    x = _dev(normal_f32(82, t, t * cols)).view(t, cols)
+    y = torch.full((t * rows + 2,), float("nan"), device="cuda")
+    eng.f32_proj(wd, t, x, y[1:-1].view(t, rows))
+    want = eng._keep_proj("gemv_b", wd, t, x, None, 1)
+    eng.check()
+    assert torch.equal(y[1:-1].view(t, rows), want) and torch.isnan(y[0]) and torch.isnan(y[-1])
+
+
 @pytest.mark.parametrize("name,rows,cols,t", [("gemv_b", 13108, 5124, 2), ("gemv_bf16_w", 16385, 8200, 3), ("gemv_bf16", 801, 4104, 1),
                                               ("gemv_bf16_b", 401, 8192, 2), ("gemv_bf16_ws", 1000, 6152, 2), ("gemv_bf16_bs", 999, 4104, 2)])
 def test_unquantised_gemvs_with_weights_ahead_keep_the_bits(eng, name, rows, cols, t):
