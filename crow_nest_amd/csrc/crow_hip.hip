@@ -35,6 +35,7 @@ struct FnEntry {
     const void* twin_stub = nullptr;  // a twin started when the launch's gz = CROW_TWIN: unquantised GEMVs, weights alone requested ahead; acc_combo, y stored
     bool ksplit = false;  // GEMM for few token rows: one of g_ksplit starts in its place when the launch's gz says which (CROW_KSPLIT)
     const void* rows_stub = nullptr;  // gemv_b: a twin with 4 x 4 rows per wave, when the launch's gz = CROW_ROWS | activation rows
+    const void* whole_stub = nullptr;  // a twin for blocks of two waves and strips of up to CROW_WHOLE_GROUPS groups, one slice
 };
 // values of S in a launch's `gy` word (GEMV family, K up to 16384; a strip of at most 64 groups never has that many slices): one
 // slice, and one strip per block where the kernel otherwise takes `ns` of them / two runs of columns per wave of the block
@@ -94,7 +95,8 @@ const FnEntry g_table[] = {
     CROW_GEMV(gemv_nvfp4_wm_bf16, 7, 1, 4, true),  CROW_GEMV(gemv_nvfp4_gum_bf16, 9, 2, 4, true), CROW_GEMV(gemv_fp4, 6, 1, 1, false),
     CROW_GEMV_TWO(gemv_fp4_b, 7, gemv_fp4_b_two),  CROW_GEMV_TWO(gemv_fp4_b1k, 7, gemv_fp4_b_two), CROW_GEMV_TWO(gemv_fp4_bs, 8, gemv_fp4_bs_two),
     CROW_GEMV(gemv_fp4_ptrb, 8, 1, 1, false),      CROW_GEMV(moe_gate_up_silu, 8, 2, 1, false),  CROW_GEMV_GEO(moe_down_combine, 7, 1, 1, false),
-    CROW_GEMV_GEO(moe_route_gate_up_silu, 11, 2, 1, false),
+    {"moe_route_gate_up_silu", (const void*)&moe_route_gate_up_silu, checked_nargs<11, 3>(&moe_route_gate_up_silu) + 0 * checked_nargs<11, 3>(&moe_route_gate_up_silu_whole), 0u, 2, 16,
+     crow::crow_gemv_lds_per_wave(1, false), 1, true, nullptr, true, nullptr, nullptr, nullptr, false, nullptr, (const void*)&moe_route_gate_up_silu_whole},
     {"moe_gate_up_silu_grouped", (const void*)&moe_gate_up_silu_grouped, checked_nargs<11, 2>(&moe_gate_up_silu_grouped) + 0 * checked_nargs<11, 2>(&moe_gate_up_silu_grouped_tile), 0u, 2, 8, crow::crow_gemv_lds_per_wave(4, false), CROW_MULTI_STRIPS, true, (const void*)&moe_gate_up_silu_grouped_tile, false},
     {"moe_down_grouped", (const void*)&moe_down_grouped, checked_nargs<9, 2>(&moe_down_grouped) + 0 * checked_nargs<9, 2>(&moe_down_grouped_tile), 0u, 1, 8, crow::crow_gemv_lds_per_wave(4, false), CROW_MULTI_STRIPS, true, (const void*)&moe_down_grouped_tile, false},
     CROW_FN_GEO(moe_group, 6),
@@ -249,6 +251,11 @@ int launch_entry(const FnEntry* e, dim3 grid, dim3 block, const uint64_t* vals, 
                 return CROW_ERR_WORKSPACE;
             geo = (int)(word & 0xFFFFFFu);
             if (store) geo = pairs | CROW_GEO_STORE;
+            const int groups = (pairs + CROW_GROUP_PAIRS - 1) / CROW_GROUP_PAIRS;
+            if (e->whole_stub != nullptr && waves == 2 && slices == 1 && groups <= CROW_WHOLE_GROUPS) {
+                stub = e->whole_stub;
+                lds = (size_t)crow::crow_gemv_lds_whole(groups);
+            }
             grid.y = (unsigned)slices;
         }
         if (lds > g.lds_cap) return CROW_ERR_SHAPE;

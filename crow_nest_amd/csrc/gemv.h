@@ -738,6 +738,105 @@ struct MultiWalk {
     }
 };
 
+// A strip of up to CROW_WHOLE_GROUPS groups that one wave walks alone, on f32 activations that the block has staged for all its waves
+// (whole_stage): the walk has no staging left.  Four groups in flight as in StripWalk (five, six and eight are slower by up to 10 %: the
+// waves of a launch all wait for the same first data).  Per group the operation sequence is StripWalk's.
+#define CROW_WHOLE_GROUPS 10
+struct WholeWalk {
+    static constexpr int SLOT = Staging<1, false>::SLOT;
+    unsigned sc[CROW_GEMV_RING][1];
+    u32x4 cd[CROW_GEMV_RING][1][2];
+    lds_p a1, a2;
+    int step1, step2;  // to the next group's slot (none in the zero area)
+    const unsigned char* wl;
+    int lane;
+    float acc[1][1];
+
+    __device__ __forceinline__ void init(const unsigned char* strip, lds_p staged, lds_p zero) {
+        lane = lane_id();
+        wl = strip;
+        acc[0][0] = 0.0f;
+        const int g = lane >> 4, i = lane & 15, r4 = i & 3;
+        const bool live = (g >> 1) == (i >> 3) && r4 < 3, second = ((i >> 2) & 1) != 0;  // as StripWalk::init
+        lds_p data = staged + r4 * CROW_GEMV_XROW_BYTES + 16 * g;
+        a1 = live && !second ? data : zero + 16 * g;
+        a2 = live && second ? data + 64 : zero + 16 * g;
+        step1 = live && !second ? SLOT : 0;
+        step2 = live && second ? SLOT : 0;
+    }
+    __device__ __forceinline__ void request(int j, int slot) {  // (both known when compiled)
+        const unsigned char* p = wl + (size_t)j * CROW_GROUP_BYTES;
+        sc[slot][0] = stream_load_u32((const unsigned*)p + lane);
+        cd[slot][0][0] = stream_load_v((const uint4*)(p + CROW_GROUP_SCALE_BYTES) + lane);
+        cd[slot][0][1] = stream_load_v((const uint4*)(p + CROW_GROUP_SCALE_BYTES + 1024) + lane);
+    }
+    template <int N>
+    __device__ __forceinline__ void walk() {
+        constexpr int D = N < CROW_GEMV_RING ? N : CROW_GEMV_RING;
+#pragma unroll
+        for (int j = 0; j < D; j++) request(j, j);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const lds_p x1[1] = {a1 + j * step1}, x2[1] = {a2 + j * step2};
+            group_multiply<1, false, 1>(sc[j % D], cd[j % D], x1, x2, acc);
+            if (j + D < N) request(j + D, j % D);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __device__ __forceinline__ void go(int count) {
+        switch (count) {
+            case 1: walk<1>(); break;
+            case 2: walk<2>(); break;
+            case 3: walk<3>(); break;
+            case 4: walk<4>(); break;
+            case 5: walk<5>(); break;
+            case 6: walk<6>(); break;
+            case 7: walk<7>(); break;
+            case 8: walk<8>(); break;
+            case 9: walk<9>(); break;
+            case 10: walk<10>(); break;
+            default: break;
+        }
+    }
+    __device__ __forceinline__ float finish() const {
+        const unsigned a = __float_as_uint(acc[0][0]);
+        const u32x2 sw = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+        const unsigned b = __float_as_uint(__fadd_rn(__uint_as_float(sw.x), __uint_as_float(sw.y)));
+        const u32x2 sq = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        return __fadd_rn(__uint_as_float(sq.x), __uint_as_float(sq.y));
+    }
+};
+// One wave: the three bf16 terms of a row of f32 activations, all groups of it (up to CROW_WHOLE_GROUPS), and the zero area.
+__device__ __forceinline__ void whole_stage(const float* x, int k_dim, int groups, lds_p staged, lds_p zero) {
+    const int lane = lane_id();
+    if (lane < CROW_GEMV_ZERO_BYTES / 16) lds_store16(zero + 16 * lane, 0, 0, 0, 0);
+    static_assert(CROW_GEMV_ZERO_BYTES <= 1024, "one store per lane");
+    constexpr int AT_ONCE = CROW_WHOLE_GROUPS / 2;
+    for (int g0 = 0; g0 < groups; g0 += AT_ONCE) {
+        f32x4 v[AT_ONCE];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; i++) {
+            const int col = (g0 + i) * CROW_GROUP_COLS + 4 * lane;
+            v[i] = *(const __attribute__((address_space(1))) f32x4*)((const unsigned char*)x + 4 * (size_t)(col < k_dim ? col : k_dim - 4));
+        }
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; i++) {
+            if (g0 + i >= groups) break;  // uniform
+            const bool in = (g0 + i) * CROW_GROUP_COLS + 4 * lane < k_dim;
+            unsigned h[4], m[4], l[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) split3(in ? v[i][c] : 0.f, h[c], m[c], l[c]);
+            lds_p row = staged + (g0 + i) * WholeWalk::SLOT + 8 * lane;
+            lds_store8(row, __builtin_amdgcn_perm(h[1], h[0], 0x07060302u), __builtin_amdgcn_perm(h[3], h[2], 0x07060302u));
+            lds_store8(row + CROW_GEMV_XROW_BYTES, __builtin_amdgcn_perm(m[1], m[0], 0x07060302u), __builtin_amdgcn_perm(m[3], m[2], 0x07060302u));
+            lds_store8(row + 2 * CROW_GEMV_XROW_BYTES, __builtin_amdgcn_perm(l[1], l[0], 0x07060302u), __builtin_amdgcn_perm(l[3], l[2], 0x07060302u));
+        }
+    }
+}
+// the dynamic LDS of such a block: the zero area, the row's terms, a wave's sixteen sums
+CROW_HD static constexpr int crow_gemv_lds_whole(int groups) { return CROW_GEMV_ZERO_BYTES + groups * (3 * CROW_GEMV_XROW_BYTES) + 64; }
+
 // The walk of a wave over MANY strips of FEW groups (short K: the routed experts' slabs, K = 2048 / 512 -> eight / two groups
 // per strip).  Walking such strips one block each means tens of thousands of blocks that each stage the same activation rows,
 // fill a pipeline of a few groups and drain it again.  Here the block stages the tile's activation rows ONCE (all groups of all

@@ -379,7 +379,7 @@ __device__ __forceinline__ void router_body(const float* __restrict__ logits, co
                                             float* __restrict__ wts, unsigned long long* __restrict__ gu_ptrs,
                                             unsigned long long* __restrict__ dn_ptrs, const unsigned long long* __restrict__ table,
                                             unsigned int* __restrict__ cold_mask, unsigned long long* __restrict__ counters,
-                                            unsigned long long* __restrict__ sel_counts, int K, int t, bool write, int& picked) {
+                                            unsigned long long* __restrict__ sel_counts, int K, int t, bool write, int need, int& picked) {
     constexpr int E = SLOTS * 64;
     const int lane = lane_id();
     float l[SLOTS], red[SLOTS];
@@ -404,37 +404,24 @@ __device__ __forceinline__ void router_body(const float* __restrict__ logits, co
     for (int j = 0; j < SLOTS; j++) key[j] = __float_as_uint(l[j] / den) + 1u;
     float sum = 0.0f, my_w = 0.0f;
     int my_id = 0;
-    for (int k = 0; k < K; k++) {
+    // (a pick is a round of instructions on one wave, 0.15 us of a launch's chain and more where blocks share a SIMD: a block that needs only
+    // its own pick stops there, and what can be is on the scalar side)
+    for (int k = 0; k < need; k++) {
         unsigned best = key[0];
-        int best_id = lane;  // the lane's best: lowest slot (= lowest id in this lane) on ties
 #pragma unroll
-        for (int j = 1; j < SLOTS; j++)
-            if (key[j] > best) {
-                best = key[j];
-                best_id = j * 64 + lane;
-            }
+        for (int j = 1; j < SLOTS; j++) best = max(best, key[j]);
         const unsigned top = wave_umax(best);
-        const unsigned long long tied = __ballot(best == top);
-        int pick;
-        if (__popcll(tied) == 1) {
-            pick = __builtin_amdgcn_readlane(best_id, (int)__builtin_ctzll(tied));
-        } else {  // equal probabilities in several lanes: the lowest expert id
-            const unsigned inv = best == top ? ~(unsigned)best_id : 0u;
-            pick = (int)~wave_umax(inv);
-        }
+        unsigned pick = ~0u;  // the lowest expert id among equals: per slot the first lane that has it (none: all ones)
+#pragma unroll
+        for (int j = 0; j < SLOTS; j++) pick = min(pick, (unsigned)(__builtin_ffsll((long long)__ballot(key[j] == top)) - 1) | (64u * j));
         const float pw = __uint_as_float(top - 1u);
         sum += pw;
-        if (lane == k) {
-            my_w = pw;
-            my_id = pick;
-        }
-        if ((pick & 63) == lane) {
+        my_w = lane == k ? pw : my_w;
+        my_id = lane == k ? (int)pick : my_id;
 #pragma unroll
-            for (int j = 0; j < SLOTS; j++)
-                if (j == (pick >> 6)) key[j] = 0u;
-        }
+        for (int j = 0; j < SLOTS; j++) key[j] = (unsigned)lane + 64u * j == pick ? 0u : key[j];
     }
-    picked = my_id;  // lane k: the k-th pick
+    picked = my_id;  // lane k < need: the k-th pick
     if (!write) return;
     unsigned cold = 0;
     if (lane < K) {
@@ -463,13 +450,13 @@ __device__ __forceinline__ void router_dispatch(int E, const float* __restrict__
                                                 float* __restrict__ wts, unsigned long long* __restrict__ gu_ptrs, unsigned long long* __restrict__ dn_ptrs,
                                                 const unsigned long long* __restrict__ table, unsigned int* __restrict__ cold_mask,
                                                 unsigned long long* __restrict__ counters, unsigned long long* __restrict__ sel_counts, int K, int t,
-                                                bool write, int& picked) {
+                                                bool write, int need, int& picked) {
     switch (E >> 6) {
-        case 1: router_body<1>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, picked); break;
-        case 2: router_body<2>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, picked); break;
-        case 4: router_body<4>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, picked); break;
-        case 8: router_body<8>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, picked); break;
-        default: router_body<16>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, picked); break;
+        case 1: router_body<1>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, need, picked); break;
+        case 2: router_body<2>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, need, picked); break;
+        case 4: router_body<4>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, need, picked); break;
+        case 8: router_body<8>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, need, picked); break;
+        default: router_body<16>(logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, t, write, need, picked); break;
     }
 }
 
@@ -490,21 +477,20 @@ extern "C" __global__ void __launch_bounds__(64) router_top10(const float* __res
         return;
     }
     int picked;
-    router_dispatch(E, logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, (int)blockIdx.x, true, picked);
+    router_dispatch(E, logits, bitmap, ids, wts, gu_ptrs, dn_ptrs, table, cold_mask, counters, sel_counts, K, (int)blockIdx.x, true, K, picked);
 }
 
 // Router and routed gate|up + SwiGLU in ONE launch: every block works out its token's routing itself (wave 0; the
 // logits row is 1 KB) instead of reading pointers a router launch left behind, which takes a launch (4 us back to back) off
 // the layer.  grid (inter / 16, 1, T K), block as moe_gate_up_silu.  Block (strip 0, pick 0) of each token writes
 // ids, wts and dn_ptrs for moe_down_combine.  table[2 e] / table[2 e + 1] = gate|up / down slab of expert e.
-extern "C" __global__ void __launch_bounds__(1024) moe_route_gate_up_silu(const float* __restrict__ logits, const unsigned long long* __restrict__ table,
-                                                                          const float* __restrict__ x, const float* __restrict__ gs_ptr,
-                                                                          float* __restrict__ h, int* __restrict__ ids, float* __restrict__ wts,
-                                                                          unsigned long long* __restrict__ dn_ptrs, const int* __restrict__ k_dim_p,
-                                                                          const int* __restrict__ x_stride_p, const int* __restrict__ inter_p, int geo, const Workspace ws,
-                                                                          const Geo model) {
-    ENTER(logits, table, x, gs_ptr, h, ids, wts, dn_ptrs, k_dim_p, x_stride_p, inter_p, geo);
+template <bool WHOLE>
+__device__ __forceinline__ void moe_route_body(const float* __restrict__ logits, const unsigned long long* __restrict__ table, const float* __restrict__ x,
+                                               const float* __restrict__ gs_ptr, float* __restrict__ h, int* __restrict__ ids, float* __restrict__ wts,
+                                               unsigned long long* __restrict__ dn_ptrs, const int* __restrict__ k_dim_p, const int* __restrict__ x_stride_p,
+                                               const int* __restrict__ inter_p, int geo, const Workspace& ws, const Geo& model) {
     const int pairs = geo & 0xFFFFF;
+    const int groups = (pairs + CROW_GROUP_PAIRS - 1) / CROW_GROUP_PAIRS;
     __shared__ unsigned long long s_slab;
     const int E = model.experts, K = model.topk;
     if (E < 64 || E > 1024 || (E & (E - 1)) != 0 || K < 1 || K > 16 || K > E || table == nullptr) {
@@ -529,7 +515,8 @@ extern "C" __global__ void __launch_bounds__(1024) moe_route_gate_up_silu(const 
             }
         }
         int picked;
-        router_dispatch(E, logits, nullptr, ids, wts, nullptr, dn_ptrs, table, nullptr, nullptr, nullptr, K, t, blockIdx.x == 0 && j == 0, picked);
+        const bool write = blockIdx.x == 0 && j == 0;
+        router_dispatch(E, logits, nullptr, ids, wts, nullptr, dn_ptrs, table, nullptr, nullptr, nullptr, K, t, write, write ? K : j + 1, picked);
         const int e = __builtin_amdgcn_readlane(picked, j);
         if (E <= 256) {
             const int q = e >> 6;  // uniform
@@ -539,18 +526,62 @@ extern "C" __global__ void __launch_bounds__(1024) moe_route_gate_up_silu(const 
         } else if (threadIdx.x == 0) {
             s_slab = table[2 * e];
         }
+    } else if constexpr (WHOLE) {  // wave 1, meanwhile
+        whole_stage(x + (size_t)t * *x_stride_p, pairs * CROW_PAIR_COLS, groups, LDS + CROW_GEMV_ZERO_BYTES, LDS);
     }
     __syncthreads();
-    const int inter = *inter_p;
+    const int inter = *inter_p, k_word = WHOLE ? *k_dim_p : 0;
+    const float gs = WHOLE ? *gs_ptr : 0.0f;
     const unsigned char* w = (const unsigned char*)s_slab;
     CROW_REFUSE_NULL_SLAB(w);  // a table with an empty entry: uniform over the block, after the only barrier before the body
     if (inter % CROW_STRIP_ROWS != 0) {
         if (threadIdx.x == 0) atomicOr(ws.status, STATUS_BAD_SHAPE);
         return;
     }
+    if constexpr (WHOLE) {  // gate by wave 0, up by wave 1
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
+        WholeWalk walk;
+        walk.init((wave == 0 ? w : w + up_offset(inter, pairs)) + (size_t)blockIdx.x * groups * CROW_GROUP_BYTES, LDS + CROW_GEMV_ZERO_BYTES, LDS);
+        walk.go(groups);
+        const float v = walk.finish();
+        lds_f up = (lds_f)(LDS + CROW_GEMV_ZERO_BYTES + groups * WholeWalk::SLOT);
+        if (wave == 1 && lane < CROW_STRIP_ROWS) up[lane] = v;
+        __syncthreads();
+        if (wave == 1) return;
+        if (k_word != pairs * CROW_PAIR_COLS) {  // the launch geometry was made for another problem: nothing is stored
+            if (lane == 0) atomicOr(ws.status, STATUS_BAD_SHAPE);
+            return;
+        }
+        const int row = (int)blockIdx.x * CROW_STRIP_ROWS + lane;
+        if (lane < CROW_STRIP_ROWS && row < inter) h[(size_t)combo * inter + row] = silu_mul(v * gs, up[lane] * gs);
+        return;
+    }
     GemvArgs a = gemv_args(w, w + up_offset(inter, pairs), gs_ptr, gs_ptr, x + (size_t)t * *x_stride_p, 0, h, 0, pairs, k_dim_p, inter_p);
     a.y_row0 = combo;
     gemv_body<2, 1, false, EPI_SILU_GU>(a, blockIdx.z, LDS, ws);
+}
+extern "C" __global__ void __launch_bounds__(1024) moe_route_gate_up_silu(const float* __restrict__ logits, const unsigned long long* __restrict__ table,
+                                                                          const float* __restrict__ x, const float* __restrict__ gs_ptr,
+                                                                          float* __restrict__ h, int* __restrict__ ids, float* __restrict__ wts,
+                                                                          unsigned long long* __restrict__ dn_ptrs, const int* __restrict__ k_dim_p,
+                                                                          const int* __restrict__ x_stride_p, const int* __restrict__ inter_p, int geo, const Workspace ws,
+                                                                          const Geo model) {
+    ENTER(logits, table, x, gs_ptr, h, ids, wts, dn_ptrs, k_dim_p, x_stride_p, inter_p, geo);
+    moe_route_body<false>(logits, table, x, gs_ptr, h, ids, wts, dn_ptrs, k_dim_p, x_stride_p, inter_p, geo, ws, model);
+}
+// The one above for blocks of two waves and strips of up to CROW_WHOLE_GROUPS groups, which the launcher starts in its place there (the
+// launch dimensions have one wave per tensor exactly up to ten groups).  Bound by a chain: logits, routing, first weights, the walk.  While
+// wave 0 routes, wave 1 stages the token's row for both, so that the walk behind the barrier only multiplies.  Same bits.  With the shorter
+// picks of router_body (us, before / now, 1, 2, 4 and 8 tokens): 256 experts, top-8, [2 x 512, 2048] 8.1 9.5 11.8 17.4 / 7.0 8.8 10.8 16.3;
+// 128, top-8, [2 x 768, 2560] 10.0 11.2 17.0 28.4 / 9.0 10.7 16.2 27.9; 512, top-10, [2 x 512, 2048] 10.2 11.3 15.2 24.9 / 9.1 10.2 12.5 19.7.
+extern "C" __global__ void __launch_bounds__(128) moe_route_gate_up_silu_whole(const float* __restrict__ logits, const unsigned long long* __restrict__ table,
+                                                                          const float* __restrict__ x, const float* __restrict__ gs_ptr,
+                                                                          float* __restrict__ h, int* __restrict__ ids, float* __restrict__ wts,
+                                                                          unsigned long long* __restrict__ dn_ptrs, const int* __restrict__ k_dim_p,
+                                                                          const int* __restrict__ x_stride_p, const int* __restrict__ inter_p, int geo, const Workspace ws,
+                                                                          const Geo model) {
+    ENTER(logits, table, x, gs_ptr, h, ids, wts, dn_ptrs, k_dim_p, x_stride_p, inter_p, geo);
+    moe_route_body<true>(logits, table, x, gs_ptr, h, ids, wts, dn_ptrs, k_dim_p, x_stride_p, inter_p, geo, ws, model);
 }
 
 // Sort the n routed combos of a batch by expert and cut them into tiles of at most four combos of one expert: the work of

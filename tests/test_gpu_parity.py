@@ -781,6 +781,32 @@ def test_routed_layers_write_y_of_their_own_and_add_to_the_callers(eng, t):
         eng.set_geo(KernelGeo(experts=256, topk=8, hidden=2048, inter=512))
 
 
+@pytest.mark.parametrize("hidden,experts,topk", [(64, 64, 4), (256, 1024, 16), (1216, 128, 8), (2048, 512, 10), (2112, 64, 5), (2560, 256, 8), (2624, 64, 3)])
+def test_routing_inside_the_gate_up_launch_keeps_the_bits(eng, hidden, experts, topk):
+    """Strips of one group, four and one more, eight, nine and ten, whole and ragged, take the twin in which one wave stages the row while
+    the other routes (2624 columns, eleven groups, do not): picks, weights and h are those of the router and the gate | up launch by
+    themselves.  Logits in few steps: most picks are ties, which go to the lowest expert id."""
+    from crow_nest_amd.engine import MoeW, expert_table
+    from crow_nest_amd.kernels import KernelGeo
+    from crow_nest_amd.weights import load_expert_slabs
+    eng.set_geo(KernelGeo(experts=experts, topk=topk, hidden=hidden, inter=64))
+    try:
+        gs = 1.0e-3
+        s_gu = load_expert_slabs(np.concatenate([random_nvfp4(900 + e, 128, hidden) for e in range(experts)]), experts, 128, hidden, gs)
+        s_dn = load_expert_slabs(np.concatenate([random_nvfp4(990 + e, hidden, 64) for e in range(experts)]), experts, hidden, 64, gs)
+        moe = MoeW(s_gu, s_dn, expert_table(s_gu, s_dn))
+        for t in (1, 5):
+            x, logits = _dev(normal_f32(31, t, t * hidden)).view(t, hidden), _dev(normal_f32(32, t, t * experts)).view(t, experts).mul(2).round()
+            ids, wts, y = eng.moe_run(moe, x, logits, "route")
+            r_ids, r_wts, r_y = eng.moe_run(moe, x, logits, True)
+            eng.check()
+            assert torch.equal(ids, r_ids) and torch.equal(wts, r_wts) and torch.equal(y, r_y) and bool(y.any())
+            order = torch.sort(torch.softmax(logits.double(), 1), dim=1, descending=True, stable=True).indices[:, :topk]
+            assert torch.equal(ids.long(), order)
+    finally:
+        eng.set_geo(KernelGeo(experts=256, topk=8, hidden=2048, inter=512))
+
+
 @pytest.mark.parametrize("t", [3, 24, 64])
 def test_moe_layer_grouped_by_expert(eng, t):
     """Batches in which experts repeat: the plan is a stable sort of the combos by expert cut into tiles of at most four,
