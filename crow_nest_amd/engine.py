@@ -155,14 +155,16 @@ class Engine:
         return ids, wts, gu, dn
 
     def moe_layer(self, moe: MoeW, x: torch.Tensor, logits: torch.Tensor, y: torch.Tensor | None = None):
-        """The routed part of one MoE layer with the launch sequence that is faster for this batch, as measured on MI355X at
-        256 experts, top-8: up to 4 tokens the router rides inside the gate|up launch (two launches: 1 token 12.5 us against
-        14.1 us for three, 4 tokens 17.8 / 19.8; at 8 tokens every block repeating its token's routing no longer pays); 5 to
-        27 tokens per combo in three launches; from 28 grouped by expert (five launches, every expert slab read once per four
-        combos: 16 tokens 50 / 57 us per combo / grouped, 24 tokens 69 / 72, 32 tokens 86 / 78, 64 tokens 158 / 101)."""
+        """The routed part of one MoE layer with the launch sequence that is faster for this batch, as measured on MI355X (captured and
+        replayed, us a layer; 256 experts, top-8, hidden 2048, inter 512 unless said).  Up to 8 tokens the router rides inside the
+        gate|up launch (two launches / three: 1 token 12.5 / 14.9, 4 tokens 17.7 / 20.4, 8 tokens 27.3 / 29.8; 512 experts, top-10,
+        8 tokens 35.9 / 40.1).  Beyond, every block repeating its token's routing soon costs what the launch did (16 tokens 48.0 /
+        49.9, hidden 5120 144.8 / 142.2, 1024 experts, top-16, 45.2 / 42.0): 9 to 27 tokens per combo in three launches.  From 28
+        grouped by expert (five launches, every expert slab read once per four combos; per combo / grouped: 20 tokens 60 / 62,
+        24 tokens 68 / 73, 28 tokens 78 / 76, 32 tokens 86 / 79, 64 tokens 161 / 103)."""
         if x.shape[0] >= 28:
             return self.moe_run_grouped(moe, x, logits, y)[:3]
-        return self.moe_run(moe, x, logits, "route" if x.shape[0] <= 4 else True, y)
+        return self.moe_run(moe, x, logits, "route" if x.shape[0] <= 8 else True, y)
 
     def moe_run_grouped(self, moe: MoeW, x: torch.Tensor, logits: torch.Tensor, y: torch.Tensor | None = None):
         """The routed part of one MoE layer for a batch in which experts repeat: router_top10, moe_group (combos sorted by

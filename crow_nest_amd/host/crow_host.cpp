@@ -270,7 +270,7 @@ void Engine::moe_run(const MoeW& moe, int t, uint64_t x, uint64_t logits, uint64
     if (moe.gate_up.rows != 2 * inter || moe.gate_up.cols != hdim || moe.down.rows != hdim || moe.down.cols != inter || moe.gate_up.experts != geo.experts)
         throw Panic("moe_run: the expert tensors do not match the geometry");
     const uint32_t combos = (uint32_t)(t * topk);
-    if (t <= 4) {  // the router inside the gate|up launch
+    if (t <= 8) {  // the router inside the gate|up launch (engine.py: moe_layer has the figures)
         launch_v(k.f("moe_route_gate_up_silu"), launch_dims("moe_route_gate_up_silu", (uint32_t)inter, (uint32_t)hdim, combos),
                  {logits, moe.table.ptr(), x, moe.gate_up.gs.ptr(), h2, ids, wts, dn_ptrs, p.i32(hdim), p.i32(hdim), p.i32(inter)});
     } else {

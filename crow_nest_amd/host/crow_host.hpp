@@ -185,7 +185,7 @@ class Engine {
     // gen.rs:4766-4784 + 6197-6198: logits[V] and the greedy token (tie rule of argmax_k); synchronises to return it
     int lm_head_row(const Fp4& w, uint64_t x, uint64_t logits);
     // gen.rs:4168-4534, routed part: ids [t][K] i32, wts [t][K] f32, y[t][H] += sum_j w_j down_e(silu(gate_e x) * up_e x);
-    // h2 is scratch [t K][I], dn_ptrs scratch u64 [t][K].  Up to 4 tokens the router runs inside the gate|up launch.
+    // h2 is scratch [t K][I], dn_ptrs scratch u64 [t][K].  Up to 8 tokens the router runs inside the gate|up launch.
     void moe_run(const MoeW& moe, int t, uint64_t x, uint64_t logits, uint64_t ids, uint64_t wts, uint64_t y, uint64_t h2, uint64_t gu_ptrs,
                  uint64_t dn_ptrs);
     // the same for a batch in which experts repeat (the prefill path's idea, kernels.rs:3322-3384): router_top10, moe_group
