@@ -7,7 +7,8 @@
 // is the CDNA4 form of the latter: weights decode to EXACT bf16 (e2m1 * ue4m3 has at most 6
 // significant bits), X is bf16, products are exact in f32, v_mfma_f32_16x16x32_bf16 accumulates.
 //
-// Data flow.  A wave owns a 64-row weight tile - four 16-row strips of the layout - per 256-column panel and MT = 16 * TBK token
+// Data flow (of the shared-X bodies; the K-split, tall and eight-wave ones, which the launcher mostly starts, say below what they do otherwise).
+// A wave owns a 64-row weight tile - four 16-row strips of the layout - per 256-column panel and MT = 16 * TBK token
 // rows.  Per panel:
 //   * the wave loads the panel's group of each of its four strips (4 x 2304 bytes) straight into registers; every code
 //     dword is the B operand of one "unit" (16 weight rows x 32 columns, layout.h) as it stands;

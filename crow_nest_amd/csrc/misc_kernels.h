@@ -804,7 +804,7 @@ extern "C" __global__ void __launch_bounds__(1024) argmax_finish(int* __restrict
 // Order: a lane adds its products in column order with one FMA each, four steps of loads in flight at a time, then the
 // 64 lane sums are added by halving (lane l += lane l + 32, + 16, ... + 1), then (second shape) the wave sums in wave order.
 // Bound by latency (a row is 8 KB): weights and activations of four steps are requested together; [256, 2048] f32: one token 3.3 us
-// (3.6 with the activations requested behind the weights), 64 tokens 10.7 us (12.6).
+// (3.6 with the activations requested behind the weights), 64 tokens 9.6 to 10.7 us (12.6; gemv_b_rows below: 6.0).
 //   gemv_bf16_w   engine/src/kernels.rs:1130-1157 (warp per row; k_dim % 8 == 0)
 //   gemv_bf16     engine/src/kernels.rs:1061-1077 (block per row, one token; + rows_p: the reference's grid.x is the row count)
 //   gemv_bf16_b   engine/src/kernels.rs:1080-1098 (block per row, grid.y tokens; + rows_p)
